@@ -221,7 +221,8 @@ __device__ __forceinline__ P partial_sum(const P *base, int64_t stride,
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (each with its own
-// L2). Renumber them so that consecutive logical tile ids share an XCD, then
+// L2). Renumber them so that consecutive logical tile ids share an XCD (XCD x
+// takes one run of num_wg / 8 tiles, the first num_wg % 8 XCDs one more), then
 // walk tiles in GROUP_M-row bands so an XCD's tiles reuse the same A row
 // panels and B column panels from its L2.
 __device__ __forceinline__ void xcd_tile_order(int wg, int num_wg,
@@ -229,8 +230,10 @@ __device__ __forceinline__ void xcd_tile_order(int wg, int num_wg,
                                                int group_m, int *tm, int *tn) {
   constexpr int kXcds = 8;
   int logical = wg;
-  if (num_wg % kXcds == 0)
-    logical = (wg % kXcds) * (num_wg / kXcds) + wg / kXcds;
+  if (num_wg > 1) {  // 1: wg is a logical tile id already (stream-K)
+    const int xcd = wg % kXcds, rest = num_wg % kXcds;
+    logical = xcd * (num_wg / kXcds) + (xcd < rest ? xcd : rest) + wg / kXcds;
+  }
   int per_group = group_m * tiles_n;
   int group = logical / per_group;
   int first_m = group * group_m;
