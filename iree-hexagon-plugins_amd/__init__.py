@@ -675,14 +675,17 @@ def _torch_stream(stream, dev):
     return stream
 
 
-def stream_workspace(need: int, device=None, stream=None, layout=None):
+def stream_workspace(need: int, device=None, stream=None, layout=None,
+                     partial=False):
     """(pointer, bytes) of the wrapper's workspace for `stream` (None: the
     current one; an int: a raw hipStream_t) on `device`, holding at least
     `need` bytes; (None, 0) when `need` is 0. `layout` keeps apart buffers
     whose arrival counters sit at different offsets (a command buffer's lane
     slices): None for flat calls, whose counters open the buffer. Under graph
     capture a buffer that is too small is not grown:
-    MI355XError(WORKSPACE_TOO_SMALL)."""
+    MI355XError(WORKSPACE_TOO_SMALL), or with `partial` what there is of it
+    (a general matmul then splits K less, or not at all; a call that cannot
+    run with it is refused by the library, with the same status)."""
     import torch
     if need <= 0:
         return None, 0
@@ -696,6 +699,8 @@ def stream_workspace(need: int, device=None, stream=None, layout=None):
     if have >= need:
         return bufs[-1].data_ptr(), have
     if torch.cuda.is_current_stream_capturing():
+        if partial:
+            return (bufs[-1].data_ptr(), have) if bufs else (None, 0)
         raise MI355XError(
             WORKSPACE_TOO_SMALL,
             f"the stream is capturing and its workspace holds {have} < "
@@ -814,7 +819,7 @@ def matmul(a, b, c=None, *, b_transposed=False, accumulate=False,
     if a.dtype != torch.int8 and out_dtype == torch.float32:
         flags |= OUT_F32
     ws, wsb = stream_workspace(_matmul_workspace_need(m, n, k, flags),
-                               a.device, s)
+                               a.device, s, partial=True)
     if a.dtype == torch.int8:
         _check(lib.iree_mi355x_matmul_i8(a.data_ptr(), b.data_ptr(),
                                          c.data_ptr(), m, n, k, a.stride(0),
@@ -915,7 +920,7 @@ def batch_matmul(a, b, c=None, *, b_transposed=False, accumulate=False,
              (A_TRANSPOSED if a_transposed else 0))
     st = _stream_ptr(stream)
     ws, wsb = stream_workspace(_batch_workspace_need(batch, m, n, k, flags),
-                               a.device, st)
+                               a.device, st, partial=True)
     _check(lib.iree_mi355x_batch_matmul_f16(
         a3.data_ptr(), b3.data_ptr(), c3.data_ptr(), batch, m, n, k,
         a3.stride(1), b3.stride(1), c3.stride(1), sa, sb, sc, flags,
@@ -956,7 +961,7 @@ def quantized_matmul(x, w, scale, y=None, *, w_transposed=False, stream=None):
     flags = B_TRANSPOSED if w_transposed else 0
     st = _stream_ptr(stream)
     ws, wsb = stream_workspace(_matmul_workspace_need(m, n, k, flags),
-                               x.device, st)
+                               x.device, st, partial=True)
     _check(lib.iree_mi355x_w8a16_matmul(
         x.data_ptr(), w.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k,
         x.stride(0), w.stride(0), y.stride(0), flags, ws, wsb, st))
@@ -1229,10 +1234,12 @@ class CommandBuffer:
         arr, n = binding_table(list(table))
         s = _stream_ptr(stream)
         if workspace is None:
-            need = self._lib.iree_mi355x_command_buffer_workspace_bytes(
-                self._h, arr, n, max_concurrent)
-            slice_ = self._lib.iree_mi355x_command_buffer_workspace_bytes(
-                self._h, arr, n, 1) if need else 0
+            need = slice_ = \
+                self._lib.iree_mi355x_command_buffer_workspace_bytes(
+                    self._h, arr, n, max_concurrent)
+            if need and max_concurrent > 1:
+                slice_ //= 1 + max(
+                    op[1] for op in self.lane_schedule(max_concurrent))
             ws, wsb = stream_workspace(need, None, s, ("lanes", slice_))
         else:
             ws, wsb = _ptr_len(workspace)

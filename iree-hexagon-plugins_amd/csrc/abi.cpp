@@ -140,6 +140,31 @@ static int launch_mfma(MatmulArgs &args, const iree_mi355x_matmul_plan_t &plan,
                        cfgs[plan.config_index].name);
 }
 
+// plan_general for a described matmul (planner.cpp).
+bool plan_general_desc(const iree_mi355x_matmul_desc_t &d, bool wide,
+                       size_t workspace_limit, GeneralPlan *plan);
+
+// The general matmul of `desc`, its K split within the workspace the call
+// has (a validate-only call: within workspace_bytes, whether or not a buffer
+// is given yet).
+static int run_general(const char *who, MatmulArgs &args,
+                       const iree_mi355x_matmul_desc_t &desc, void *workspace,
+                       size_t workspace_bytes) {
+  GeneralPlan plan;
+  const bool wide =
+      args.lda * (desc.a_elem == IREE_MI355X_ELEM_I8 ? 1 : 2) >=
+          kMaxFastPitchBytes ||
+      args.ldb * (desc.b_elem == IREE_MI355X_ELEM_I8 ? 1 : 2) >=
+          kMaxFastPitchBytes;
+  if (!plan_general_desc(desc, wide, workspace || g_dry_run ? workspace_bytes : 0,
+                         &plan))
+    return fail(IREE_MI355X_UNSUPPORTED, "%s: no plan", who);
+  if (dry_run(plan.workspace))
+    return ok();
+  args.workspace = plan.workspace > 0 ? workspace : nullptr;
+  return launch_status(launch_general(args, plan), who);
+}
+
 // Shared shape / stride checks for the three matmul entry points.
 static int check_matmul(const char *who, const void *a, const void *b,
                         void *c, int64_t m, int64_t n, int64_t k, int64_t lda,
@@ -201,9 +226,10 @@ size_t iree_mi355x_matmul_workspace_bytes(int64_t m, int64_t n, int64_t k,
   if (m <= 0 || n <= 0 || k <= 0)
     return 0;
   // The largest workspace any f16, int8 or W8A16 plan of this shape uses (plans
-  // assume 16-byte aligned operands, the case that can pick split-K), over
-  // both layouts a call may take: one row of a transposed A with unit pitch
-  // runs as the untransposed row (see m1_row_layout).
+  // assume 16-byte aligned operands; others take the general kernel, which
+  // runs with any workspace), over both layouts a call may take: one row of a
+  // transposed A with unit pitch runs as the untransposed row (see
+  // m1_row_layout).
   size_t most = 0;
   const int32_t forms[4][3] = {
       {IREE_MI355X_ELEM_F16, IREE_MI355X_ELEM_F16, IREE_MI355X_ELEM_F16},
@@ -258,6 +284,8 @@ static int matmul_f16_run(const char *who, MatmulArgs &args, uint32_t flags,
   iree_mi355x_matmul_plan_t plan;
   if (iree_mi355x_plan_matmul(&desc, &plan) != IREE_MI355X_OK)
     return fail(IREE_MI355X_UNSUPPORTED, "%s: no plan", who);
+  if (plan.family == IREE_MI355X_FAMILY_GENERAL)
+    return run_general(who, args, desc, workspace, workspace_bytes);
   if (dry_run(plan.workspace_bytes))
     return ok();
   int st;
@@ -269,13 +297,8 @@ static int matmul_f16_run(const char *who, MatmulArgs &args, uint32_t flags,
         return st;
       return launch_status(launch_gemv(args, 2, nullptr, out_f32, workspace),
                            "gemv_f16");
-    case IREE_MI355X_FAMILY_MFMA:
-      return launch_mfma(args, plan, workspace, workspace_bytes, who);
     default:
-      return launch_status(
-          launch_general(args, out_f32 ? kGeneralF16F32 : kGeneralF16F16,
-                         nullptr),
-          "gemm_general_f16");
+      return launch_mfma(args, plan, workspace, workspace_bytes, who);
   }
 }
 
@@ -432,12 +455,11 @@ int iree_mi355x_matmul_i8(const int8_t *a, const int8_t *b, int32_t *c,
   iree_mi355x_matmul_plan_t plan;
   if (iree_mi355x_plan_matmul(&desc, &plan) != IREE_MI355X_OK)
     return fail(IREE_MI355X_UNSUPPORTED, "matmul_i8: no plan");
+  if (plan.family == IREE_MI355X_FAMILY_GENERAL)
+    return run_general("matmul_i8", args, desc, workspace, workspace_bytes);
   if (dry_run(plan.workspace_bytes))
     return ok();
-  if (plan.family == IREE_MI355X_FAMILY_MFMA)
-    return launch_mfma(args, plan, workspace, workspace_bytes, "matmul_i8");
-  return launch_status(launch_general(args, kGeneralI8I32, nullptr),
-                       "gemm_general_i8");
+  return launch_mfma(args, plan, workspace, workspace_bytes, "matmul_i8");
 }
 
 int iree_mi355x_w8a16_matmul(const void *x, const int8_t *w, const void *scale,
@@ -465,6 +487,9 @@ int iree_mi355x_w8a16_matmul(const void *x, const int8_t *w, const void *scale,
   iree_mi355x_matmul_plan_t plan;
   if (iree_mi355x_plan_matmul(&desc, &plan) != IREE_MI355X_OK)
     return fail(IREE_MI355X_UNSUPPORTED, "w8a16_matmul: no plan");
+  if (plan.family == IREE_MI355X_FAMILY_GENERAL)
+    return run_general("w8a16_matmul", args, desc, workspace,
+                       workspace_bytes);
   if (dry_run(plan.workspace_bytes))
     return ok();
   if (plan.family == IREE_MI355X_FAMILY_GEMV) {
@@ -474,10 +499,7 @@ int iree_mi355x_w8a16_matmul(const void *x, const int8_t *w, const void *scale,
     return launch_status(launch_gemv(args, 1, scale, 0, workspace),
                          "gemv_w8a16");
   }
-  if (plan.family == IREE_MI355X_FAMILY_MFMA)
-    return launch_mfma(args, plan, workspace, workspace_bytes, "w8a16_matmul");
-  return launch_status(launch_general(args, kGeneralW8A16, scale),
-                       "gemm_general_w8a16");
+  return launch_mfma(args, plan, workspace, workspace_bytes, "w8a16_matmul");
 }
 
 int iree_mi355x_attention_f16_strided(

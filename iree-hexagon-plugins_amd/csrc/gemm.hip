@@ -989,118 +989,6 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
 }
 
 // ----------------------------------------------------------------------------
-// General path: any extents, strides, A and B layout; bounds-checked element
-// loads staged through registers into LDS (B converted to the MFMA input type
-// on the way, which is where W8A16 dequantizes), 64x64 tiles, 4 waves of
-// 32x32 fragments, optional per-column scale in the epilogue.
-// ----------------------------------------------------------------------------
-
-template <typename TA, typename TB, typename OutT, bool kScale>
-__global__ __launch_bounds__(256) void gemm_general_kernel(
-    const TA *__restrict__ A, const TB *__restrict__ B, OutT *__restrict__ C,
-    const f16 *__restrict__ scale, int M, int N, int K, int64_t lda,
-    int64_t ldb, int64_t ldc, int b_transposed, int accumulate, int64_t sa,
-    int64_t sb, int64_t sc, Epi epi, int64_t s_mul, int a_transposed) {
-  {
-    const int64_t z = blockIdx.z;
-    A += z * sa;
-    B += z * sb;
-    C += z * sc;
-    epi.mul += z * s_mul;  // s_mul is 0 without a multiplier
-  }
-  // MFMA input type: f16 unless both operands are int8.
-  typedef typename MfmaInput<TA, TB>::type TM;
-  typedef Mfma32<TM> MF;
-  constexpr int KE = 64 / (int)sizeof(TM);  // K elements per 64-byte slab
-  constexpr int ROWB = 64 + 16;             // padded staged row (bytes)
-  __shared__ __attribute__((aligned(16))) char As[64 * ROWB];
-  __shared__ __attribute__((aligned(16))) char Bs[64 * ROWB];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t m0 = (int64_t)blockIdx.y * 64, n0 = (int64_t)blockIdx.x * 64;
-  typename MF::Acc acc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r)
-    acc[r] = 0;
-
-  constexpr int EPT = 16 / (int)sizeof(TM);  // elements per thread per slab
-  const int ld_r = tid / 4, ld_c = (tid % 4) * EPT;
-
-  for (int k0 = 0; k0 < K; k0 += KE) {
-    if (!a_transposed) {  // A rows are M
-      TM *dst = (TM *)(As + ld_r * ROWB) + ld_c;
-      const int64_t m = m0 + ld_r;
-#pragma unroll
-      for (int e = 0; e < EPT; ++e) {
-        const int k = k0 + ld_c + e;
-        dst[e] = (m < M && k < K) ? (TM)A[m * lda + k] : (TM)0;
-      }
-    } else {  // A [K,M]: m fastest across threads, staged transposed
-      const int mm = tid & 63, kq = tid >> 6;
-      constexpr int KPT = KE / 4;
-      TM *dst = (TM *)(As + mm * ROWB) + kq * KPT;
-      const int64_t m = m0 + mm;
-#pragma unroll
-      for (int e = 0; e < KPT; ++e) {
-        const int k = k0 + kq * KPT + e;
-        dst[e] = (m < M && k < K) ? (TM)A[(int64_t)k * lda + m] : (TM)0;
-      }
-    }
-    if (b_transposed) {  // B rows are N
-      TM *dst = (TM *)(Bs + ld_r * ROWB) + ld_c;
-      const int64_t n = n0 + ld_r;
-#pragma unroll
-      for (int e = 0; e < EPT; ++e) {
-        const int k = k0 + ld_c + e;
-        dst[e] = (n < N && k < K) ? (TM)B[n * ldb + k] : (TM)0;
-      }
-    } else {  // B [K,N]: n fastest across threads, staged transposed
-      const int nn = tid & 63, kq = tid >> 6;
-      constexpr int KPT = KE / 4;
-      TM *dst = (TM *)(Bs + nn * ROWB) + kq * KPT;
-      const int64_t n = n0 + nn;
-#pragma unroll
-      for (int e = 0; e < KPT; ++e) {
-        const int k = k0 + kq * KPT + e;
-        dst[e] = (n < N && k < K) ? (TM)B[(int64_t)k * ldb + n] : (TM)0;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const int ch = 2 * ks + (lane >> 5);
-      i32x4 af = *(const i32x4 *)(As + (wm * 32 + (lane & 31)) * ROWB + ch * 16);
-      i32x4 bf = *(const i32x4 *)(Bs + (wn * 32 + (lane & 31)) * ROWB + ch * 16);
-      acc = MF::mma(af, bf, acc);
-    }
-    __syncthreads();
-  }
-
-  const int64_t col = n0 + wn * 32 + (lane & 31);
-  if (col >= N)
-    return;
-  float s = 1.0f;
-  if (kScale)
-    s = (float)scale[col];
-  const int mode = accumulate ? kStoreAccumulate : kStorePlain;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int64_t row = m0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-    if (row < M) {
-      if constexpr (std::is_same<OutT, int32_t>::value) {
-        store_out(C + row * ldc + col, acc[r], mode);
-      } else {
-        float v = (float)acc[r];
-        if (kScale)
-          v *= s;
-        store_out(C + row * ldc + col, epi_apply(v, row, col, epi), mode);
-      }
-    }
-  }
-}
-
-// ----------------------------------------------------------------------------
 // Host launchers.
 // ----------------------------------------------------------------------------
 
@@ -1359,8 +1247,7 @@ const FastConfig *fast_configs(int *count) {
   return kFastConfigs;
 }
 
-// Every GEMM kernel: the macro-tile configurations, then the general kernel's
-// four instances.
+// Every GEMM kernel: the macro-tile configurations, then the general kernel's.
 const KernelEntry *gemm_kernels(int *count) {
   static const std::vector<KernelEntry> all = [] {
     std::vector<KernelEntry> v;
@@ -1373,43 +1260,19 @@ const KernelEntry *gemm_kernels(int *count) {
                               : kExportMatmulF16 | kExportBatchMatmulF16;
       v.push_back({c.name, c.kernel, c.threads, ex});
     }
-    const uint32_t f16x = kExportMatmulF16 | kExportBatchMatmulF16;
-    v.push_back({"general_f16", (const void *)&gemm_general_kernel<f16, f16, f16, false>, 256, f16x});
-    v.push_back({"general_f16f32", (const void *)&gemm_general_kernel<f16, f16, float, false>, 256, f16x});
-    v.push_back({"general_i8", (const void *)&gemm_general_kernel<int8_t, int8_t, int32_t, false>, 256, kExportMatmulI8});
-    v.push_back({"general_w8a16", (const void *)&gemm_general_kernel<f16, int8_t, f16, true>, 256, kExportW8A16});
+    int n = 0;
+    const GeneralConfig *g = general_configs(&n);
+    for (int i = 0; i < n; ++i) {
+      const uint32_t ex = g[i].kind == kGeneralI8I32   ? kExportMatmulI8
+                          : g[i].kind == kGeneralW8A16 ? kExportW8A16
+                                                       : kExportMatmulF16 |
+                                                             kExportBatchMatmulF16;
+      v.push_back({g[i].name, g[i].kernel, g[i].threads, ex});
+    }
     return v;
   }();
   *count = (int)all.size();
   return all.data();
-}
-
-template <typename TA, typename TB, typename OutT, bool kScale>
-static hipError_t launch_general_t(const MatmulArgs &a, const void *scale) {
-  dim3 grid((unsigned)((a.n + 63) / 64), (unsigned)((a.m + 63) / 64),
-            (unsigned)a.batch);
-  hipLaunchKernelGGL((gemm_general_kernel<TA, TB, OutT, kScale>), grid,
-                     dim3(256), 0, (hipStream_t)a.stream, (const TA *)a.a,
-                     (const TB *)a.b, (OutT *)a.c, (const f16 *)scale,
-                     (int)a.m, (int)a.n, (int)a.k, a.lda, a.ldb, a.ldc,
-                     a.b_transposed, a.accumulate, a.sa, a.sb, a.sc,
-                     make_epi(a), epi_batch_stride(a), a.a_transposed);
-  return hipGetLastError();
-}
-
-hipError_t launch_general(const MatmulArgs &a, GeneralKind kind,
-                          const void *scale) {
-  switch (kind) {
-    case kGeneralF16F16:
-      return launch_general_t<f16, f16, f16, false>(a, nullptr);
-    case kGeneralF16F32:
-      return launch_general_t<f16, f16, float, false>(a, nullptr);
-    case kGeneralI8I32:
-      return launch_general_t<int8_t, int8_t, int32_t, false>(a, nullptr);
-    case kGeneralW8A16:
-      return launch_general_t<f16, int8_t, f16, true>(a, scale);
-  }
-  return hipErrorInvalidValue;
 }
 
 }  // namespace ihp

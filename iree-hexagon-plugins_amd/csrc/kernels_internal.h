@@ -180,8 +180,37 @@ enum GeneralKind {
   kGeneralI8I32 = 2,
   kGeneralW8A16 = 3,
 };
-hipError_t launch_general(const MatmulArgs &a, GeneralKind kind,
-                          const void *scale);
+// A compiled configuration of the general matmul kernel (gemm_ragged.hip):
+// any extents, strides and alignment of one kind and layout.
+struct GeneralConfig {
+  const char *name;
+  GeneralKind kind;
+  int a_trans, b_trans;
+  int bm, bn;
+  int wgs;        // workgroups a CU holds
+  int any;        // any pitch and row length (general_any)
+  int threads;
+  int lds_bytes;
+  const void *kernel;
+  hipError_t (*launch)(const MatmulArgs &, int splits, int k_split);
+};
+const GeneralConfig *general_configs(int *count);
+
+// A general matmul's configuration and K split. A split needs a workspace;
+// plan_general never asks for more than the caller has, so a general matmul
+// runs with any workspace or none.
+struct GeneralPlan {
+  int index;
+  int splits, k_split;
+  int64_t tiles;      // per batch
+  int64_t workspace;  // bytes (0: one split)
+};
+// wide: a row pitch of kMaxFastPitchBytes or more.
+bool plan_general(GeneralKind kind, int64_t m, int64_t n, int64_t k,
+                  int64_t batch, bool a_trans, bool b_trans, bool wide,
+                  int64_t lds_budget, size_t workspace_limit,
+                  GeneralPlan *plan);
+hipError_t launch_general(const MatmulArgs &a, const GeneralPlan &plan);
 
 // Skinny (M <= kGemvMaxRows) matmul with B [K,N] row-major: split-K streaming
 // kernel with an in-kernel last-arriver reduction over `splits` partials.
@@ -305,19 +334,24 @@ __device__ __forceinline__ float sigmoid_fast(float a) {
   return __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-__device__ __forceinline__ float epi_apply(float v, int64_t row, int64_t col,
-                                           const Epi &e) {
-  if (e.bias)
-    v += (float)e.bias[col];
-  if (e.act == kActRelu) {
+__device__ __forceinline__ float epi_act(float v, int act) {
+  if (act == kActRelu) {
     v = v > 0.0f ? v : 0.0f;
-  } else if (e.act != kActNone) {
+  } else if (act != kActNone) {
     const float a =
-        e.act == kActGeluTanh
+        act == kActGeluTanh
             ? 1.5957691216057308f * (v + 0.044715f * v * v * v)
             : v;
     v *= sigmoid_fast(a);
   }
+  return v;
+}
+
+__device__ __forceinline__ float epi_apply(float v, int64_t row, int64_t col,
+                                           const Epi &e) {
+  if (e.bias)
+    v += (float)e.bias[col];
+  v = epi_act(v, e.act);
   if (e.mul)
     v *= (float)e.mul[row * e.ld_mul + col];
   return v;

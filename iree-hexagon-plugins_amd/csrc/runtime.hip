@@ -180,10 +180,12 @@ struct Ready {
 };
 
 // Resolve and validate every command; the largest workspace any dispatch
-// asks for goes to *max_workspace. Enqueues nothing.
+// asks for, of the `workspace_limit` bytes it may have, goes to
+// *max_workspace. Enqueues nothing.
 int prepare(const iree_mi355x_command_buffer_t *cb,
             const iree_mi355x_binding_t *table, uint32_t count,
-            std::vector<Ready> *out, size_t *max_workspace) {
+            size_t workspace_limit, std::vector<Ready> *out,
+            size_t *max_workspace) {
   *max_workspace = 0;
   out->assign(cb->commands.size(), Ready());
   const iree_mi355x_executable_export_table_t &ex = cb->library->exports;
@@ -211,6 +213,7 @@ int prepare(const iree_mi355x_command_buffer_t *cb,
         s.binding_count = (uint32_t)r.ptrs.size();
         s.binding_ptrs = r.ptrs.data();
         s.binding_lengths = r.lengths.data();
+        s.workspace_bytes = workspace_limit;
         s.workspace_query = &need;
         if ((st = ex.ptrs[c.ordinal](nullptr, &s))) {
           const std::string why = iree_mi355x_last_error();
@@ -573,13 +576,15 @@ size_t iree_mi355x_command_buffer_workspace_bytes(
     uint32_t max_concurrent) {
   if (!cb || max_concurrent > IREE_MI355X_MAX_CONCURRENCY)
     return 0;
-  std::vector<Ready> ready;
-  size_t need = 0;
-  if (prepare(cb, binding_table, binding_count, &ready, &need) !=
-      IREE_MI355X_OK)
-    return 0;
   const uint32_t lanes = lanes_for(
       cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
+  // In order, one buffer serves every dispatch: ask for all that their plans
+  // can use. Lanes take slices, sized by what the plans require only.
+  std::vector<Ready> ready;
+  size_t need = 0;
+  if (prepare(cb, binding_table, binding_count, lanes == 1 ? SIZE_MAX : 0,
+              &ready, &need) != IREE_MI355X_OK)
+    return 0;
   return need ? slice_bytes(need) * lanes : 0;
 }
 
@@ -597,15 +602,17 @@ int iree_mi355x_command_buffer_submit(
     return fail(IREE_MI355X_INVALID_ARGUMENT,
                 "submit: concurrency %u > %u", max_concurrent,
                 IREE_MI355X_MAX_CONCURRENCY);
+  const uint32_t lanes = lanes_for(
+      cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
   std::vector<Ready> ready;
   size_t need = 0;
-  int st = prepare(cb, binding_table, binding_count, &ready, &need);
+  int st = prepare(cb, binding_table, binding_count,
+                   lanes == 1 && workspace ? workspace_bytes : 0, &ready,
+                   &need);
   if (st)
     return st;
   if (cb->commands.empty())
     return IREE_MI355X_OK;
-  const uint32_t lanes = lanes_for(
-      cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
   const size_t slice = need ? slice_bytes(need) : 0;
   // The caller provides the lane slices: the runtime allocates no device
   // memory.
@@ -627,9 +634,11 @@ int iree_mi355x_command_buffer_submit(
   const uint32_t n = (uint32_t)cb->commands.size();
 
   if (lanes == 1) {
-    // In order on the caller's stream: barriers hold by stream order.
+    // In order on the caller's stream: barriers hold by stream order, and
+    // every dispatch may use the whole workspace.
     for (uint32_t i = 0; i < n && !st; ++i)
-      st = enqueue(cb, i, ready[i], caller, slice ? ws : nullptr, slice);
+      st = enqueue(cb, i, ready[i], caller, slice ? ws : nullptr,
+                   slice ? workspace_bytes : 0);
     roctxRangePop();
     return st;
   }

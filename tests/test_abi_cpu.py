@@ -868,3 +868,25 @@ def test_workspace_query_matches_dispatch_dry_run(pkg):
             assert need > 0  # runs as the GEMV, which needs a workspace
         qb = lib.iree_mi355x_batch_matmul_workspace_bytes(1, m, n, k, flags)
         assert need <= qb
+
+
+def test_general_split_fits_the_workspace_it_gets(pkg):
+    """A general matmul needs no workspace; what a caller offers bounds its K
+    split (the query reports the part it would use)."""
+    m, n, k = 65, 200, 4100
+    consts = pkg.matmul_constants(m, n, k, k, n, n, 0)
+    sizes = [m * k * 2, k * n * 2, m * n * 2]
+    needs = []
+    for limit in (0, 256 * 1024, 1 << 20, 1 << 40):
+        st, need = pkg.call_export("matmul_f16", consts, [FAKE] * 3, sizes,
+                                   workspace_bytes=limit, query=True)
+        assert st == pkg.OK and need <= limit
+        needs.append(need)
+    assert needs[0] == needs[1] == 0 < needs[2] <= needs[3]
+    assert needs[3] == pkg.plan(pkg.make_desc(F16, F16, F16, m, n, k,
+                                              0)).workspace_bytes
+    # whole rows of fewer elements than one load, and rows 8 MiB apart, take
+    # the any-stride form
+    for shape in ((65, 200, 7), (65, 7, 4100)):
+        p = pkg.plan(pkg.make_desc(F16, F16, F16, *shape, 0))
+        assert p.config_name == b"general_f16_any"

@@ -1,0 +1,221 @@
+"""The general matmul (csrc/gemm_ragged.hip): any extents, strides, alignment
+and layout, f16 with f16 / f32 results, int8 and W8A16, with and without a K
+split.
+
+Bars: int8 results are exact; f16 and W8A16 ones max|y - y_cpu| / max|y_cpu|
+<= 2e-3 (the fp16 parity bound) against the oracle, f32 ones 1e-5 (f32 sums of
+at most 777 products). Operands are views into NaN-filled (int8: random)
+buffers, outputs views into filled ones: nothing outside a view is used or
+written.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BOUND = {"f16": 2e-3, "f32": 1e-5, "w8a16": 2e-3}
+
+# edges of the 64 / 128 tiles, of a 16-byte load and of a K stage (64 f16,
+# 128 int8), and the smallest of everything
+SHAPES = [(1, 1, 1), (2, 3, 5), (7, 17, 9), (16, 8, 15), (63, 65, 64),
+          (64, 64, 128), (65, 63, 129), (127, 129, 63), (128, 128, 200),
+          (129, 127, 257), (5, 1030, 777), (300, 72, 130)]
+
+
+def view_in(rows, cols, t, fill, pad, lead):
+    """`t` as a [rows, cols] view whose rows are `pad` elements further apart
+    than their length and which starts `lead` elements into its buffer."""
+    buf = torch.full((lead + rows * (cols + pad),), fill, dtype=t.dtype)
+    if t.dtype == torch.int8:
+        buf = torch.randint(-128, 128, buf.shape, dtype=torch.int8)
+    v = torch.as_strided(buf, (rows, cols), (cols + pad, 1), lead)
+    v.copy_(t)
+    d = buf.cuda()
+    return torch.as_strided(d, (rows, cols), (cols + pad, 1), lead)
+
+
+def operands(kind, at, bt, m, n, k, pad, lead):
+    g = torch.Generator().manual_seed(m * 7919 + n * 31 + k)
+
+    def f16(r, c):
+        return torch.randn(r, c, generator=g).half()
+
+    def i8(r, c):
+        return torch.randint(-128, 128, (r, c), generator=g).to(torch.int8)
+
+    a = (i8 if kind == "i8" else f16)(*((k, m) if at else (m, k)))
+    b = (i8 if kind in ("i8", "w8a16") else f16)(*((n, k) if bt else (k, n)))
+    nan = float("nan")
+    da = view_in(*a.shape, a, 0 if kind == "i8" else nan, pad, lead)
+    db = view_in(*b.shape, b, 0 if b.dtype == torch.int8 else nan, pad, lead)
+    return a, b, da, db
+
+
+def run(pkg, kind, at, bt, da, db, scale, m, n, c):
+    if kind == "w8a16":
+        pkg.quantized_matmul(da, db, scale, c, w_transposed=bt)
+    else:
+        pkg.matmul(da, db, c, a_transposed=at, b_transposed=bt,
+                   out_dtype=c.dtype)
+
+
+def output(kind, m, n):
+    dt = {"i8": torch.int32, "f32": torch.float32}.get(kind, torch.float16)
+    buf = torch.full((m + 2, n + 5), 77, dtype=dt, device="cuda")
+    return buf, buf[1:m + 1, :n]
+
+
+def check(oracle, kind, at, bt, a, b, scale, buf, m, n):
+    full = buf.cpu()
+    c = full[1:m + 1, :n].numpy().copy()
+    full[1:m + 1, :n] = 77
+    assert bool((full == 77).all()), "write outside the output view"
+    an, bn = a.numpy(), b.numpy()
+    if kind == "i8":
+        assert np.array_equal(c, oracle.matmul_i8(an, bn, b_transposed=bt))
+        return
+    if kind == "w8a16":
+        ref = oracle.w8a16(an, np.ascontiguousarray(bn.T) if bt else bn,
+                           scale.numpy())
+    else:
+        ref = oracle.matmul_f16(np.ascontiguousarray(an.T) if at else an, bn,
+                                b_transposed=bt, out_f32=kind == "f32")
+    assert np.isfinite(c).all()
+    assert oracle.fp16_parity(c, ref) <= BOUND[kind]
+
+
+FORMS = [(kind, at, bt) for kind in ("f16", "f32", "i8", "w8a16")
+         for at in (False, True) for bt in (False, True)
+         if not (at and kind in ("i8", "w8a16"))]
+
+
+@pytest.mark.parametrize("kind,at,bt", FORMS)
+def test_general_edges(pkg, oracle, dev, kind, at, bt):
+    for i, (m, n, k) in enumerate(SHAPES):
+        pad, lead = ((0, 0), (1, 1), (5, 3), (8, 8))[i % 4]
+        print(f"{kind} at={at} bt={bt} {m}x{n}x{k} pad={pad}", flush=True)
+        a, b, da, db = operands(kind, at, bt, m, n, k, pad, lead)
+        scale = (torch.rand(n) * 0.019 + 0.001).half()
+        buf, c = output(kind, m, n)
+        run(pkg, kind, at, bt, da, db, scale.cuda(), m, n, c)
+        check(oracle, kind, at, bt, a, b, scale, buf, m, n)
+
+
+@pytest.mark.parametrize("kind,at,bt", FORMS)
+def test_general_wide_pitch(pkg, oracle, dev, kind, at, bt):
+    """Rows 8 MiB apart: the lane offsets of a tile pass 32 bits."""
+    m, n, k = 5, 20, 24
+    a, b, _, _ = operands(kind, at, bt, m, n, k, 0, 0)
+    pitch = 8 << 20
+
+    def wide(t):
+        buf = torch.zeros((t.shape[0] - 1) * pitch + t.shape[1],
+                          dtype=t.dtype, device="cuda")
+        v = torch.as_strided(buf, tuple(t.shape), (pitch, 1))
+        v.copy_(t)
+        return v
+
+    scale = (torch.rand(n) * 0.019 + 0.001).half()
+    buf, c = output(kind, m, n)
+    run(pkg, kind, at, bt, wide(a), wide(b), scale.cuda(), m, n, c)
+    check(oracle, kind, at, bt, a, b, scale, buf, m, n)
+
+
+@pytest.mark.parametrize("kind,bt", [("f16", False), ("f32", True),
+                                     ("i8", True), ("w8a16", True)])
+def test_general_split_and_no_workspace(pkg, oracle, dev, kind, bt):
+    """A shape whose plan splits K, twice on one workspace (the counters are
+    re-armed), and without a workspace, where it runs unsplit."""
+    m, n, k = 65, 200, 4100
+    a, b, da, db = operands(kind, False, bt, m, n, k, 1, 1)
+    scale = (torch.rand(n) * 0.019 + 0.001).half()
+    ds = scale.cuda()
+    types = {"f16": (0, 0, 0), "f32": (0, 0, 3), "i8": (1, 1, 2),
+             "w8a16": (0, 1, 0)}[kind]
+    p = pkg.plan(pkg.make_desc(*types, m, n, k, 1 if bt else 0,
+                               has_scale=kind == "w8a16", aligned=False))
+    assert p.family == pkg.FAMILY_GENERAL and p.splits > 1
+    for _ in range(2):
+        buf, c = output(kind, m, n)
+        run(pkg, kind, False, bt, da, db, ds, m, n, c)
+        if kind == "f32":  # 4100 products: 2e-5
+            ref = oracle.matmul_f16(a.numpy(), b.numpy(), b_transposed=bt,
+                                    out_f32=True)
+            assert oracle.fp16_parity(c.cpu().numpy(), ref) <= 2e-5
+        else:
+            check(oracle, kind, False, bt, a, b, scale, buf, m, n)
+    split = c.clone()
+    c.fill_(77)
+    lib, st = pkg.library(), torch.cuda.current_stream().cuda_stream
+    flags = (1 if bt else 0) | (pkg.OUT_F32 if kind == "f32" else 0)
+    if kind == "w8a16":
+        rc = lib.iree_mi355x_w8a16_matmul(
+            da.data_ptr(), db.data_ptr(), ds.data_ptr(), c.data_ptr(), m, n,
+            k, da.stride(0), db.stride(0), c.stride(0), flags, None, 0, st)
+    else:
+        fn = (lib.iree_mi355x_matmul_i8 if kind == "i8"
+              else lib.iree_mi355x_matmul_f16)
+        rc = fn(da.data_ptr(), db.data_ptr(), c.data_ptr(), m, n, k,
+                da.stride(0), db.stride(0), c.stride(0), flags, None, 0, st)
+    assert rc == pkg.OK, pkg.last_error()
+    if kind == "i8":
+        assert torch.equal(c, split)
+    else:
+        err = (c.double() - split.double()).abs().max() / split.abs().max()
+        assert float(err) <= (2e-5 if kind == "f32" else 2e-3)
+
+
+@pytest.mark.parametrize("act", ["none", "relu", "gelu_tanh", "silu"])
+@pytest.mark.parametrize("shape", [(3, 65, 67, 70), (2, 130, 129, 1030)])
+def test_general_batched_epilogue(pkg, oracle, dev, act, shape):
+    z, m, n, k = shape
+    g = torch.Generator().manual_seed(m + n)
+    x = torch.randn(z, m, k, generator=g).half()
+    w = (torch.randn(z, k, n, generator=g) / k ** 0.5).half()
+    bias = torch.randn(n, generator=g).half()
+    mul = torch.randn(z, m, n, generator=g).half()
+    init = torch.randn(z, m, n, generator=g).half()
+    c = init.cuda()
+    pkg.batch_matmul(x.cuda(), w.cuda(), c, bias=bias.cuda(), activation=act,
+                     multiplier=mul.cuda(), accumulate=True)
+    v = torch.matmul(x.double(), w.double()) + bias.double()
+    v = {"none": lambda t: t, "relu": torch.relu,
+         "gelu_tanh": lambda t: torch.nn.functional.gelu(
+             t, approximate="tanh"),
+         "silu": torch.nn.functional.silu}[act](v)
+    ref = init.double() + mul.double() * v
+    err = (c.cpu().double() - ref).abs().max() / ref.abs().max()
+    assert float(err) <= 2e-3
+
+
+def test_general_zero_k(pkg, dev):
+    """K = 0 writes the epilogue of an empty sum, and C_init if it adds."""
+    a = torch.empty(70, 0, dtype=torch.float16, device=dev)
+    b = torch.empty(0, 33, dtype=torch.float16, device=dev)
+    assert bool((pkg.matmul(a, b) == 0).all())
+    c = torch.full((70, 33), 3.0, dtype=torch.float16, device=dev)
+    pkg.matmul(a, b, c, accumulate=True)
+    assert bool((c == 3).all())
+
+
+def test_general_under_capture(pkg, oracle, dev):
+    """A split shape captured on a stream that has no workspace runs unsplit,
+    as it did before it could split; replays agree with the eager result."""
+    m, n, k = 33, 130, 2050
+    a, b, da, db = operands("f16", False, False, m, n, k, 1, 1)
+    eager = pkg.matmul(da, db)
+    s = torch.cuda.Stream()
+    c = torch.zeros(m, n, dtype=torch.float16, device=dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        pkg.matmul(da, db, c)
+    for _ in range(3):
+        c.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = oracle.matmul_f16(a.numpy(), b.numpy())
+        assert oracle.fp16_parity(c.cpu().numpy(), ref) <= 2e-3
+    assert oracle.fp16_parity(eager.cpu().numpy(), ref) <= 2e-3
