@@ -241,6 +241,22 @@ typedef struct iree_mi355x_attention_t {
 } iree_mi355x_attention_t;
 int iree_mi355x_attention(const iree_mi355x_attention_t *args, void *stream);
 
+// iree_mi355x_attention with a workspace (the matmul workspace contract below:
+// zero-filled before its first use, its counter region left zero-filled; may
+// be NULL). Calls of few query rows over many keys deal the keys to several
+// workgroups, whose partial results go through it; a call runs with any
+// workspace or none, with as many parts as fit. No counterpart in the
+// reference, whose online-softmax loop is serial over the keys.
+int iree_mi355x_attention_with_workspace(const iree_mi355x_attention_t *args,
+                                         void *workspace,
+                                         size_t workspace_bytes,
+                                         void *stream);
+
+// The workspace a call of these extents and flags can use (0: none); pointers
+// and strides are not looked at.
+size_t iree_mi355x_attention_workspace_bytes(
+    const iree_mi355x_attention_t *args);
+
 // Workspace a matmul_f16 / matmul_i8 / w8a16_matmul call of this shape
 // needs (split-K
 // partials and arrival counters), 0 if none. Mirrors the scratch query of the

@@ -58,6 +58,8 @@ EXPORTED_SYMBOLS = (
     "iree_mi355x_matmul_f16", "iree_mi355x_matmul_i8",
     "iree_mi355x_w8a16_matmul", "iree_mi355x_attention_f16",
     "iree_mi355x_attention_f16_strided", "iree_mi355x_attention",
+    "iree_mi355x_attention_with_workspace",
+    "iree_mi355x_attention_workspace_bytes",
     "iree_mi355x_matmul_workspace_bytes", "iree_mi355x_last_error",
     "iree_mi355x_version", "iree_mi355x_device_count",
     "iree_mi355x_matmul_desc_init", "iree_mi355x_classify_matmul",
@@ -295,6 +297,9 @@ def library():
     lib.iree_mi355x_attention_f16_strided.argtypes = [
         p, p, p, p, i64, i64, i64, i64, i64, i64, ctypes.c_float, u32, p, p]
     lib.iree_mi355x_attention.argtypes = [p, p]
+    lib.iree_mi355x_attention_with_workspace.argtypes = [p, p, sz, p]
+    lib.iree_mi355x_attention_workspace_bytes.restype = sz
+    lib.iree_mi355x_attention_workspace_bytes.argtypes = [p]
     lib.iree_mi355x_matmul_workspace_bytes.restype = sz
     lib.iree_mi355x_matmul_workspace_bytes.argtypes = [i64, i64, i64, u32]
     lib.iree_mi355x_batch_matmul_f16.argtypes = [
@@ -988,6 +993,23 @@ class AttentionArgs(ctypes.Structure):
                 ("mask_strides", ctypes.c_int64 * 4)]
 
 
+@functools.lru_cache(maxsize=4096)
+def _attention_workspace_need(b, h, hkv, sq, skv, d, dv, flags) -> int:
+    a = AttentionArgs(batch=b, heads=h, kv_heads=hkv, seq_q=sq, seq_kv=skv,
+                      head_dim=d, head_dim_v=dv, flags=flags)
+    return library().iree_mi355x_attention_workspace_bytes(ctypes.byref(a))
+
+
+def _fused_layout(st, pointers, sq, skv) -> bool:
+    """Strides and bases (or-ed) as iree_mi355x_attention_f16_strided demands
+    of a head dim of 64 or 128: it refuses the others, with a workspace too."""
+    every = 0
+    for t in (st.q, st.k, st.v, st.o):
+        every |= t[0] | t[1] | t[2]
+    span = max((sq - 1) * st.q[2], (skv - 1) * max(st.k[2], st.v[2])) * 2
+    return (every & 7) == 0 and (pointers & 15) == 0 and span < (1 << 32) - 256
+
+
 def attention(q, k, v, o=None, *, causal=True, scale=None, mask=None,
               out_dtype=None, stream=None):
     """Fused attention forward: q [B, Hq, Sq, D], k [B, Hkv, Skv, D],
@@ -998,8 +1020,7 @@ def attention(q, k, v, o=None, *, causal=True, scale=None, mask=None,
     -inf is 0. Any operand may be a strided view whose last dimension is
     contiguous (a slice of a longer KV cache, o a permuted view of a
     [B, Sq, Hq, Dv] buffer). Equal head dims of 64 or 128 with no mask and
-    an f16 o run the MFMA kernel; the rest the general one (head dims up to
-    256)."""
+    an f16 o need 16-byte aligned rows; head dims go up to 256."""
     import torch
     for t, nm in ((q, "q"), (k, "k"), (v, "v")):
         if (not isinstance(t, torch.Tensor) or t.dtype != torch.float16
@@ -1041,35 +1062,35 @@ def attention(q, k, v, o=None, *, causal=True, scale=None, mask=None,
         scale = d ** -0.5
     if o is None:
         o = torch.empty(b, h, sq, dv, dtype=out_dtype, device=q.device)
-    flags = CAUSAL if causal else 0
-    fast = (mask is None and out_dtype == torch.float16 and d == dv
-            and d in (64, 128))
-    if fast and hkv == h and all(t.is_contiguous() for t in (q, k, v, o)):
+    flags = ((CAUSAL if causal else 0) |
+             (ATTENTION_OUT_F32 if out_dtype == torch.float32 else 0) |
+             (ATTENTION_MASK if mask is not None else 0))
+    stp = _stream_ptr(stream)
+    need = _attention_workspace_need(b, h, hkv, sq, skv, d, dv, flags)
+    fast = flags in (0, CAUSAL) and d == dv and d in (64, 128)
+    if (fast and not need and hkv == h
+            and all(t.is_contiguous() for t in (q, k, v, o))):
         _check(lib.iree_mi355x_attention_f16(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), b, h, sq,
-            skv, d, float(scale), flags, _stream_ptr(stream)))
+            skv, d, float(scale), flags, stp))
         return o
-    st = AttentionStrides()
-    for field, t in (("q", q), ("k", k), ("v", v), ("o", o)):
-        getattr(st, field)[:] = list(t.stride()[:3])
-    if fast:
+    st = AttentionStrides(q.stride()[:3], k.stride()[:3], v.stride()[:3],
+                          o.stride()[:3])
+    qp, kp, vp, op = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr()
+    if fast and not (need and _fused_layout(st, qp | kp | vp | op, sq, skv)):
         _check(lib.iree_mi355x_attention_f16_strided(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), b, h,
-            hkv, sq, skv, d, float(scale), flags, ctypes.byref(st),
-            _stream_ptr(stream)))
+            qp, kp, vp, op, b, h, hkv, sq, skv, d, float(scale), flags,
+            ctypes.byref(st), stp))
         return o
-    a = AttentionArgs(q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(),
-                      o=o.data_ptr(), batch=b, heads=h, kv_heads=hkv,
+    a = AttentionArgs(q=qp, k=kp, v=vp, o=op, batch=b, heads=h, kv_heads=hkv,
                       seq_q=sq, seq_kv=skv, head_dim=d, head_dim_v=dv,
-                      scale=float(scale), strides=st)
-    if out_dtype == torch.float32:
-        flags |= ATTENTION_OUT_F32
+                      scale=float(scale), flags=flags, strides=st)
     if mask is not None:
-        flags |= ATTENTION_MASK
         a.mask = mask.data_ptr()
-        a.mask_strides[:] = list(mask.stride())
-    a.flags = flags
-    _check(lib.iree_mi355x_attention(ctypes.byref(a), _stream_ptr(stream)))
+        a.mask_strides[:] = mask.stride()
+    ws, wsb = stream_workspace(need, q.device, stp, partial=True)
+    _check(lib.iree_mi355x_attention_with_workspace(ctypes.byref(a), ws, wsb,
+                                                    stp))
     return o
 
 

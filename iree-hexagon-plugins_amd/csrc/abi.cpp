@@ -502,6 +502,141 @@ int iree_mi355x_w8a16_matmul(const void *x, const int8_t *w, const void *scale,
   return launch_mfma(args, plan, workspace, workspace_bytes, "w8a16_matmul");
 }
 
+}  // extern "C"
+
+namespace ihp {
+
+// Modeled times of the attention kernels, in us, for the choice between them
+// (attention_rows.hip takes a call only where it is modeled 1.2 times faster).
+// Fits to both sides of 118 shapes (1 to 2048 queries, 64 to 8192 keys, head
+// dims 40 to 256, causal, masked or neither, 8 to 96 heads): by this rule
+// 1.0 % slower than the better kernel on average. Measured at both ends: one
+// query of 32 heads over 8 KV heads and 3001 keys, batch 4, 13.3 us against
+// 44.0 us for the fused kernel; 2048 x 2048 causal, 32 heads, d 128, 113 us
+// against 44 us.
+static double rows_us(const AttentionRowsPlan &p, int64_t seq_kv, bool causal,
+                      int64_t seq_q, bool mask) {
+  const int i = p.dp == 64 ? 0 : p.dp == 128 ? 1 : 2;
+  static const double kUnit[] = {0.535e-3, 0.68e-3, 2.2e-3};
+  static const double kChain[] = {0.326, 1.16, 0.93};
+  const int64_t blocks = (seq_kv + 31) / 32;
+  const double mean =
+      (double)blocks * (causal && seq_q > 1 ? 0.5 : 1.0) + (causal ? 0.5 : 0);
+  const int64_t wave_blocks = (p.blocks_per_split + 3) / 4;
+  const int64_t held = p.dp < 256 ? 512 : 256;
+  const int64_t rounds = (p.tiles * p.splits + held - 1) / held;
+  return 5.78 +
+         (double)p.tiles * mean * kUnit[i] * (mask ? 1.46 : 1.0) *
+             (p.rf == 1 && p.dp < 256 ? 0.72 : 1.0) +
+         kChain[i] * (double)(wave_blocks * rounds) +
+         (p.splits > 1 ? 3.3 : 0.0);
+}
+
+// The fused kernel: rounds of workgroups of two query blocks, 128 keys a step.
+static double fused_us(const iree_mi355x_attention_t &a, bool causal) {
+  const int64_t n = (a.seq_q + 127) / 128;
+  auto steps = [&](int64_t q) {
+    const int64_t keys =
+        causal && (q + 1) * 128 < a.seq_kv ? (q + 1) * 128 : a.seq_kv;
+    return (double)((keys + 127) / 128);
+  };
+  const double total = steps(n - 1) + (n > 1 ? steps(0) : 0.0);
+  const int64_t rounds = (a.batch * a.heads * ((n + 1) / 2) + 255) / 256;
+  const double step = a.head_dim <= 64 ? (a.mask ? 2.24 : 0.99)
+                                       : (a.mask ? 2.76 : 1.66);
+  return 0.42 + (double)rounds * (step * total + 4.42 * (n > 1 ? 2.0 : 1.0));
+}
+
+// The general kernel: workgroups of 64 query rows (a block and its mirror
+// under the causal mask), 64 keys a step.
+static double general_attention_us(const iree_mi355x_attention_t &a,
+                                   bool causal) {
+  const int64_t d = a.head_dim > a.head_dim_v ? a.head_dim : a.head_dim_v;
+  const int i = d <= 32 ? 0 : d <= 64 ? 1 : d <= 128 ? 2 : 3;
+  static const double kAlone[] = {0.186, 1.83, 2.82, 4.98};
+  static const double kShared[] = {0.192, 0.358, 2.39, 2.72};
+  static const int64_t kHeld[] = {4, 4, 2, 1};
+  const int64_t n = (a.seq_q + 63) / 64;
+  const int64_t wgs = a.batch * a.heads * (causal ? (n + 1) / 2 : n);
+  const int64_t steps = (a.seq_kv + 63) / 64 + (causal ? 1 : 0);
+  const int64_t per_cu = (wgs + 255) / 256;
+  const double alone = (kAlone[i] + (a.mask ? 4.39 : 0.0)) *
+                       (double)((per_cu + kHeld[i] - 1) / kHeld[i]);
+  const double shared =
+      (kShared[i] + (a.mask ? 1.49 : 0.0)) * (double)per_cu;
+  return 4.83 + (double)steps * (alone > shared ? alone : shared);
+}
+
+// Whether the row-packed kernel takes a call, and its plan. It needs head
+// dims that are multiples of 8, and of a mask contiguous keys, at least 4;
+// `fused`: the fused kernel takes the call otherwise.
+static bool rows_plan(const iree_mi355x_attention_t &a, bool fused,
+                      size_t workspace_limit, AttentionRowsPlan *plan) {
+  const int64_t group = a.heads / a.kv_heads;
+  if (a.head_dim % 8 != 0 || a.head_dim_v % 8 != 0 || a.head_dim_v < 8 ||
+      a.seq_kv < 1 || a.seq_q * group >= kMaxExtent / 2 ||
+      (a.mask && (a.mask_strides[3] != 1 || a.seq_kv < 4)))
+    return false;
+  *plan = plan_attention_rows(a.batch, a.kv_heads, group, a.seq_q, a.seq_kv,
+                              a.head_dim, a.head_dim_v, workspace_limit);
+  if (plan->tiles >= kMaxExtent)
+    return false;
+  const bool causal = a.flags & IREE_MI355X_ATTENTION_CAUSAL;
+  const double other =
+      fused ? fused_us(a, causal) : general_attention_us(a, causal);
+  return rows_us(*plan, a.seq_kv, causal, a.seq_q, a.mask != nullptr) * 1.2 <
+         other;
+}
+
+static AttentionGeneralLayout general_layout(const iree_mi355x_attention_t &a) {
+  AttentionGeneralLayout g;
+  const iree_mi355x_attention_strides_t &st = a.strides;
+  for (int i = 0; i < 3; ++i) {
+    g.q[i] = st.q[i];
+    g.k[i] = st.k[i];
+    g.v[i] = st.v[i];
+    g.o[i] = st.o[i];
+  }
+  for (int i = 0; i < 4; ++i)
+    g.mask[i] = a.mask_strides[i];
+  g.heads = (int)a.heads;
+  g.group = (int)(a.heads / a.kv_heads);
+  g.seq_q = (int)a.seq_q;
+  g.seq_kv = (int)a.seq_kv;
+  g.dqk = (int)a.head_dim;
+  g.dv = (int)a.head_dim_v;
+  g.scale = a.scale;
+  g.causal = (a.flags & IREE_MI355X_ATTENTION_CAUSAL) ? 1 : 0;
+  g.vec_k = a.head_dim % 8 == 0 && st.k[0] % 8 == 0 && st.k[1] % 8 == 0 &&
+            st.k[2] % 8 == 0 && aligned(a.k, 16);
+  g.vec_v = a.head_dim_v % 8 == 0 && st.v[0] % 8 == 0 &&
+            st.v[1] % 8 == 0 && st.v[2] % 8 == 0 && aligned(a.v, 16);
+  return g;
+}
+
+// Runs a checked call on the row-packed kernel if that takes it; *ran tells.
+static int try_rows(const iree_mi355x_attention_t &a, bool fused,
+                    void *workspace, size_t workspace_bytes, void *stream,
+                    bool *ran) {
+  AttentionRowsPlan plan;
+  *ran = rows_plan(a, fused, workspace || g_dry_run ? workspace_bytes : 0,
+                   &plan);
+  if (!*ran)
+    return IREE_MI355X_OK;
+  if (dry_run(plan.workspace))
+    return ok();
+  return launch_status(
+      launch_attention_rows(a.q, a.k, a.v, a.o, a.mask, general_layout(a),
+                            plan,
+                            (a.flags & IREE_MI355X_ATTENTION_OUT_F32) ? 1 : 0,
+                            workspace, stream),
+      "attention_rows");
+}
+
+}  // namespace ihp
+
+extern "C" {
+
 int iree_mi355x_attention_f16_strided(
     const void *q, const void *k, const void *v, void *o, int64_t batch,
     int64_t heads, int64_t kv_heads, int64_t seq_q, int64_t seq_kv,
@@ -572,6 +707,24 @@ int iree_mi355x_attention_f16_strided(
       head_span(strides->v, seq_kv) > (int64_t)UINT32_MAX)
     return fail(IREE_MI355X_UNSUPPORTED,
                 "%s: a head's rows span more than 4 GiB", who);
+  iree_mi355x_attention_t a = {};
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.o = o;
+  a.batch = batch;
+  a.heads = heads;
+  a.kv_heads = kv_heads;
+  a.seq_q = seq_q;
+  a.seq_kv = seq_kv;
+  a.head_dim = a.head_dim_v = head_dim;
+  a.scale = scale;
+  a.flags = flags;
+  a.strides = *strides;
+  bool ran = false;
+  const int rows_st = try_rows(a, true, nullptr, 0, stream, &ran);
+  if (ran)
+    return rows_st;
   if (dry_run(0))
     return ok();
   AttentionLayout layout;
@@ -592,7 +745,10 @@ int iree_mi355x_attention_f16_strided(
       "attention_fwd");
 }
 
-int iree_mi355x_attention(const iree_mi355x_attention_t *a, void *stream) {
+int iree_mi355x_attention_with_workspace(const iree_mi355x_attention_t *a,
+                                         void *workspace,
+                                         size_t workspace_bytes,
+                                         void *stream) {
   const char *who = "attention";
   if (!a)
     return fail(IREE_MI355X_INVALID_ARGUMENT, "%s: null arguments", who);
@@ -676,6 +832,11 @@ int iree_mi355x_attention(const iree_mi355x_attention_t *a, void *stream) {
                head_span(st.v, a->seq_kv) > (int64_t)UINT32_MAX ||
                a->batch * a->heads * ((a->seq_q + 127) / 128) >= kMaxExtent))
     fast = false;
+  bool ran = false;
+  const int rows_st =
+      try_rows(*a, fast, workspace, workspace_bytes, stream, &ran);
+  if (ran)
+    return rows_st;
   if (fast && !a->mask && !out_f32 &&
       (a->head_dim == 64 || a->head_dim == 128))
     return iree_mi355x_attention_f16_strided(
@@ -703,33 +864,34 @@ int iree_mi355x_attention(const iree_mi355x_attention_t *a, void *stream) {
                          a->mask, out_f32 ? 1 : 0),
         a->mask ? "attention_fwd_mask" : "attention_fwd");
   }
-  AttentionGeneralLayout g;
-  for (int i = 0; i < 3; ++i) {
-    g.q[i] = st.q[i];
-    g.k[i] = st.k[i];
-    g.v[i] = st.v[i];
-    g.o[i] = st.o[i];
-  }
-  for (int i = 0; i < 4; ++i)
-    g.mask[i] = a->mask_strides[i];
-  g.heads = (int)a->heads;
-  g.group = (int)(a->heads / a->kv_heads);
-  g.seq_q = (int)a->seq_q;
-  g.seq_kv = (int)a->seq_kv;
-  g.dqk = (int)a->head_dim;
-  g.dv = (int)a->head_dim_v;
-  g.scale = a->scale;
-  g.causal = causal ? 1 : 0;
-  g.vec_k = a->head_dim % 8 == 0 && st.k[0] % 8 == 0 && st.k[1] % 8 == 0 &&
-            st.k[2] % 8 == 0 && aligned(a->k, 16);
-  g.vec_v = a->head_dim_v % 8 == 0 && st.v[0] % 8 == 0 &&
-            st.v[1] % 8 == 0 && st.v[2] % 8 == 0 && aligned(a->v, 16);
   return launch_status(
-      launch_attention_general(a->q, a->k, a->v, a->o, a->mask, a->batch, g,
-                               out_f32 ? 1 : 0, stream),
+      launch_attention_general(a->q, a->k, a->v, a->o, a->mask, a->batch,
+                               general_layout(*a), out_f32 ? 1 : 0, stream),
       "attention_general");
 }
 
+int iree_mi355x_attention(const iree_mi355x_attention_t *a, void *stream) {
+  return iree_mi355x_attention_with_workspace(a, nullptr, 0, stream);
+}
+
+size_t iree_mi355x_attention_workspace_bytes(
+    const iree_mi355x_attention_t *a) {
+  if (!a || a->batch < 1 || a->heads < 1 || a->kv_heads < 1 ||
+      a->heads % a->kv_heads != 0 || a->seq_q < 1 || a->seq_kv < 1 ||
+      a->head_dim < 1 || a->head_dim_v < 1 || a->head_dim > 256 ||
+      a->head_dim_v > 256 || a->batch > 65535 || a->heads > 65535 ||
+      a->seq_q >= kMaxExtent / 2 || a->seq_kv >= kMaxExtent / 2)
+    return 0;
+  iree_mi355x_attention_t d = *a;
+  if (a->flags & IREE_MI355X_ATTENTION_MASK) {
+    d.mask = a;  // present; only its strides and extents matter here
+    d.mask_strides[3] = 1;
+  }
+  const bool fused = a->head_dim == a->head_dim_v && a->head_dim % 16 == 0 &&
+                     a->head_dim <= 128 && (!d.mask || a->seq_kv % 4 == 0);
+  AttentionRowsPlan plan;
+  return rows_plan(d, fused, (size_t)-1, &plan) ? (size_t)plan.workspace : 0;
+}
 
 int iree_mi355x_attention_f16(const void *q, const void *k, const void *v,
                               void *o, int64_t batch, int64_t heads,

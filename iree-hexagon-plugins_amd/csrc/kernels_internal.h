@@ -303,6 +303,34 @@ hipError_t launch_attention_general(const void *q, const void *k,
                                     int out_f32, void *stream);
 const KernelEntry *attention_general_kernels(int *count);
 
+// The row-packed attention kernel (attention_rows.hip): the query rows of all
+// heads of a KV head in tiles of 16 rf rows, keys dealt over `splits`
+// workgroups a tile within the workspace the caller has (none: one).
+// One workgroup a CU, at least 256 keys (2 blocks a wave) each, at most 16 a
+// tile: more parts cost more in their merge than they save (32 query heads
+// over 8 KV heads, 3001 keys, d 128: batch 4 14.1 / 13.2 / 14.5 us at 4 / 8 /
+// 16 splits, batch 1 10.6 / 10.0 / 10.1 at 8 / 12 / 16; 8192 keys on 2 tiles
+// 13.0 us at 16, 14.0 at 24).
+constexpr int64_t kRowsTargetWgs = 256;
+constexpr int64_t kRowsSplitBlocks = 8;
+constexpr int64_t kRowsMaxSplits = 16;
+struct AttentionRowsPlan {
+  int dp, rf;  // head-dim bucket, 16-row fragments a tile
+  int64_t row_tiles, tiles, splits, blocks_per_split;
+  int64_t workspace;
+};
+AttentionRowsPlan plan_attention_rows(int64_t batch, int64_t kv_heads,
+                                      int64_t group, int64_t seq_q,
+                                      int64_t seq_kv, int64_t head_dim,
+                                      int64_t head_dim_v,
+                                      size_t workspace_limit);
+hipError_t launch_attention_rows(const void *q, const void *k, const void *v,
+                                 void *o, const void *mask,
+                                 const AttentionGeneralLayout &layout,
+                                 const AttentionRowsPlan &plan, int out_f32,
+                                 void *workspace, void *stream);
+const KernelEntry *attention_rows_kernels(int *count);
+
 #ifdef __HIP_DEVICE_COMPILE__
 #define IHP_HD __device__
 #else

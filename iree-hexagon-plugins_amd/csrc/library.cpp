@@ -244,7 +244,8 @@ int dispatch_attention(const iree_mi355x_executable_environment_t *,
   a.k = s->binding_ptrs[1];
   a.v = s->binding_ptrs[2];
   a.o = s->binding_ptrs[3];
-  return iree_mi355x_attention(&a, s->stream);
+  return iree_mi355x_attention_with_workspace(&a, s->workspace,
+                                              s->workspace_bytes, s->stream);
 }
 
 // "batch_matmul_f16": the matmul_f16 constants, then batch, stride_a,
@@ -339,10 +340,7 @@ const iree_mi355x_executable_dispatch_attrs_t kAttrs[] = {
     {kF16Flags, 163840, 512},
     {kF16Flags, 147456, 512},
     {kF16Flags, 147456, 512},
-    {IREE_MI355X_DISPATCH_FLAG_RESOURCES_VALID |
-         IREE_MI355X_DISPATCH_FLAG_USES_MFMA |
-         IREE_MI355X_DISPATCH_FLAG_USES_LDS_DMA,
-     135168, 512},
+    {kF16Flags, 135168, 512},
     {kF16Flags, 163840, 512},
 };
 
@@ -377,7 +375,8 @@ namespace {
 const ihp::KernelEntry *kernel_at(int index) {
   const ihp::KernelEntry *(*lists[])(int *) = {
       ihp::gemm_kernels, ihp::gemv_kernels, ihp::attention_kernels,
-      ihp::attention_general_kernels, ihp::runtime_kernels};
+      ihp::attention_general_kernels, ihp::attention_rows_kernels,
+      ihp::runtime_kernels};
   for (auto list : lists) {
     int n = 0;
     const ihp::KernelEntry *e = list(&n);
@@ -399,6 +398,8 @@ extern "C" int iree_mi355x_kernel_count(void) {
   ihp::attention_kernels(&n);
   total += n;
   ihp::attention_general_kernels(&n);
+  total += n;
+  ihp::attention_rows_kernels(&n);
   total += n;
   ihp::runtime_kernels(&n);
   return total + n;
