@@ -140,13 +140,35 @@ static int launch_mfma(MatmulArgs &args, const iree_mi355x_matmul_plan_t &plan,
                        cfgs[plan.config_index].name);
 }
 
+// The plan of a call with this much workspace, and the workspace without
+// which the call is refused (planner.cpp).
+int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
+                iree_mi355x_matmul_plan_t *plan, size_t *required);
+
+// Plans a call within the workspace it has (a validate-only call: within
+// workspace_bytes, whether or not a buffer is given yet) and refuses one that
+// has less than it must. *done: nothing is left to run (refused or validated).
+static int plan_call(const char *who, const iree_mi355x_matmul_desc_t &desc,
+                     const void *workspace, size_t workspace_bytes,
+                     iree_mi355x_matmul_plan_t *plan, bool *done) {
+  size_t required = 0;
+  *done = true;
+  if (plan_matmul(&desc, workspace || g_dry_run ? workspace_bytes : 0, plan,
+                  &required) != IREE_MI355X_OK)
+    return fail(IREE_MI355X_UNSUPPORTED, "%s: no plan", who);
+  if (dry_run(plan->workspace_bytes))
+    return ok();
+  const int st = require_workspace(who, required, workspace, workspace_bytes);
+  *done = st != IREE_MI355X_OK;
+  return st;
+}
+
 // plan_general for a described matmul (planner.cpp).
 bool plan_general_desc(const iree_mi355x_matmul_desc_t &d, bool wide,
                        size_t workspace_limit, GeneralPlan *plan);
 
 // The general matmul of `desc`, its K split within the workspace the call
-// has (a validate-only call: within workspace_bytes, whether or not a buffer
-// is given yet).
+// has.
 static int run_general(const char *who, MatmulArgs &args,
                        const iree_mi355x_matmul_desc_t &desc, void *workspace,
                        size_t workspace_bytes) {
@@ -156,11 +178,8 @@ static int run_general(const char *who, MatmulArgs &args,
           kMaxFastPitchBytes ||
       args.ldb * (desc.b_elem == IREE_MI355X_ELEM_I8 ? 1 : 2) >=
           kMaxFastPitchBytes;
-  if (!plan_general_desc(desc, wide, workspace || g_dry_run ? workspace_bytes : 0,
-                         &plan))
+  if (!plan_general_desc(desc, wide, workspace ? workspace_bytes : 0, &plan))
     return fail(IREE_MI355X_UNSUPPORTED, "%s: no plan", who);
-  if (dry_run(plan.workspace))
-    return ok();
   args.workspace = plan.workspace > 0 ? workspace : nullptr;
   return launch_status(launch_general(args, plan), who);
 }
@@ -282,19 +301,15 @@ static int matmul_f16_run(const char *who, MatmulArgs &args, uint32_t flags,
   desc.b_aligned16 = fast_operand(args.b, args.ldb * 2, args.sb * 2);
   desc.batch = args.batch;
   iree_mi355x_matmul_plan_t plan;
-  if (iree_mi355x_plan_matmul(&desc, &plan) != IREE_MI355X_OK)
-    return fail(IREE_MI355X_UNSUPPORTED, "%s: no plan", who);
-  if (plan.family == IREE_MI355X_FAMILY_GENERAL)
-    return run_general(who, args, desc, workspace, workspace_bytes);
-  if (dry_run(plan.workspace_bytes))
-    return ok();
-  int st;
+  bool done = false;
+  const int st =
+      plan_call(who, desc, workspace, workspace_bytes, &plan, &done);
+  if (done)
+    return st;
   switch (plan.family) {
+    case IREE_MI355X_FAMILY_GENERAL:
+      return run_general(who, args, desc, workspace, workspace_bytes);
     case IREE_MI355X_FAMILY_GEMV:
-      if ((st = require_workspace(who, (size_t)plan.workspace_bytes,
-                                  workspace, workspace_bytes)) !=
-          IREE_MI355X_OK)
-        return st;
       return launch_status(launch_gemv(args, 2, nullptr, out_f32, workspace),
                            "gemv_f16");
     default:
@@ -453,12 +468,12 @@ int iree_mi355x_matmul_i8(const int8_t *a, const int8_t *b, int32_t *c,
   desc.a_aligned16 = fast_operand(a, lda);
   desc.b_aligned16 = fast_operand(b, ldb);
   iree_mi355x_matmul_plan_t plan;
-  if (iree_mi355x_plan_matmul(&desc, &plan) != IREE_MI355X_OK)
-    return fail(IREE_MI355X_UNSUPPORTED, "matmul_i8: no plan");
+  bool done = false;
+  st = plan_call("matmul_i8", desc, workspace, workspace_bytes, &plan, &done);
+  if (done)
+    return st;
   if (plan.family == IREE_MI355X_FAMILY_GENERAL)
     return run_general("matmul_i8", args, desc, workspace, workspace_bytes);
-  if (dry_run(plan.workspace_bytes))
-    return ok();
   return launch_mfma(args, plan, workspace, workspace_bytes, "matmul_i8");
 }
 
@@ -485,20 +500,17 @@ int iree_mi355x_w8a16_matmul(const void *x, const int8_t *w, const void *scale,
   desc.b_aligned16 = fast_operand(w, ldw);
   desc.has_scale = 1;
   iree_mi355x_matmul_plan_t plan;
-  if (iree_mi355x_plan_matmul(&desc, &plan) != IREE_MI355X_OK)
-    return fail(IREE_MI355X_UNSUPPORTED, "w8a16_matmul: no plan");
+  bool done = false;
+  st = plan_call("w8a16_matmul", desc, workspace, workspace_bytes, &plan,
+                 &done);
+  if (done)
+    return st;
   if (plan.family == IREE_MI355X_FAMILY_GENERAL)
     return run_general("w8a16_matmul", args, desc, workspace,
                        workspace_bytes);
-  if (dry_run(plan.workspace_bytes))
-    return ok();
-  if (plan.family == IREE_MI355X_FAMILY_GEMV) {
-    if ((st = require_workspace("w8a16_matmul", (size_t)plan.workspace_bytes,
-                                workspace, workspace_bytes)) != IREE_MI355X_OK)
-      return st;
+  if (plan.family == IREE_MI355X_FAMILY_GEMV)
     return launch_status(launch_gemv(args, 1, scale, 0, workspace),
                          "gemv_w8a16");
-  }
   return launch_mfma(args, plan, workspace, workspace_bytes, "w8a16_matmul");
 }
 

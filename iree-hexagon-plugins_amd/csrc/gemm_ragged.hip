@@ -306,6 +306,7 @@ struct RaggedArgs {
   int64_t M, N, K, lda, ldb, ldc, sa, sb, sc, s_mul;
   Epi epi;
   int accumulate;
+  int through;         // store the result past the L2 (kStoreThroughBytes)
   int k_split;         // K elements per split, a multiple of the stage
   float *partials;     // split-K: f32 / i32 partial tiles, else unused
   unsigned *counters;
@@ -438,7 +439,8 @@ __global__ __launch_bounds__(64 * WM *WN, WGS) void gemm_ragged_kernel(
             __builtin_bit_cast(i32x4, acc[i][j]), rs,
             voff + (i * FN + j) * 1024, (int)blockIdx.y * (BM * BN * 4),
             kDeviceScope);
-    unsigned *last = (unsigned *)smem;
+    __shared__ unsigned last_split;
+    unsigned *last = &last_split;
     wait_vmcnt<0>();  // published before it is counted
     __syncthreads();
     if (tid == 0) {
@@ -477,13 +479,26 @@ __global__ __launch_bounds__(64 * WM *WN, WGS) void gemm_ragged_kernel(
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  // out = [C +] mul * act(acc [* scale] + bias), 4 columns a lane.
+  // out = [C +] mul * act(acc [* scale] + bias), 4 columns a lane. i32 and
+  // f32 results are stored from there, 64 bytes of a row an instruction; f16
+  // ones (32 bytes) go through the wave's part of the idle LDS ring, row
+  // chunks swizzled, and leave as whole rows of the wave's tile: short sums
+  // with large results are bound by these stores (int8 weights, 1500 x 4096 x
+  // 256: 17.9 us without the staging).
   constexpr bool kIntOut = std::is_same<OutT, int32_t>::value;
+  constexpr bool kStage = sizeof(OutT) == 2;
+  constexpr int OROW = WTN * (int)sizeof(OutT);  // bytes of a staged row
+  constexpr int OCH = OROW / 16;
+  static_assert(!kStage || (WM * WN * WTM * OROW <= 2 * SLOT &&
+                            (OCH & (OCH - 1)) == 0),
+                "staging");
+  char *const stage = smem + wave * (WTM * OROW);
   OutT *C = (OutT *)p.c + z * p.sc;
   const f16 *mul = p.epi.mul ? p.epi.mul + z * p.s_mul : nullptr;
+  const int64_t row0 = m0 + wm * WTM, col0 = n0 + wn * WTN;
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
-    const int64_t col = n0 + wn * WTN + j * 16 + 4 * (lane >> 4);
+    const int64_t col = col0 + j * 16 + 4 * (lane >> 4);
     const int valid = (int)(p.N - col < 4 ? p.N - col : 4);
     if (valid <= 0)
       continue;
@@ -500,7 +515,7 @@ __global__ __launch_bounds__(64 * WM *WN, WGS) void gemm_ragged_kernel(
     }
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int64_t row = m0 + wm * WTM + i * 16 + (lane & 15);
+      const int64_t row = row0 + i * 16 + (lane & 15);
       if (row >= p.M)
         continue;
       OutT *dst = C + row * p.ldc + col;
@@ -513,7 +528,10 @@ __global__ __launch_bounds__(64 * WM *WN, WGS) void gemm_ragged_kernel(
             for (int r = 0; r < 4; ++r)
               v[r] = (int)((unsigned)old[r] + (unsigned)v[r]);
           }
-          *(i32x4_u4 *)dst = v;
+          if (p.through)
+            store_through16(dst, v);
+          else
+            *(i32x4_u4 *)dst = v;
         } else {
 #pragma unroll
           for (int r = 0; r < 3; ++r)
@@ -530,38 +548,84 @@ __global__ __launch_bounds__(64 * WM *WN, WGS) void gemm_ragged_kernel(
             v[r] *= sc[r];
           v[r] = epi_act(v[r] + bias[r], p.epi.act);
         }
-        if (valid == 4) {
-          if (mul) {
-            const f16x4 g = *(const f16x4_u *)(mul + row * p.epi.ld_mul + col);
+        if (mul) {
+          const f16 *g = mul + row * p.epi.ld_mul + col;
+          f16x4 gv = {0, 0, 0, 0};
+          if (valid == 4)
+            gv = *(const f16x4_u *)g;
+          else
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              v[r] *= (float)g[r];
-          }
-          if constexpr (std::is_same<OutT, float>::value) {
-            f32x4 o = {v[0], v[1], v[2], v[3]};
-            if (p.accumulate)
-              o += *(const f32x4_u *)dst;
-            *(f32x4_u *)dst = o;
-          } else {
-            if (p.accumulate) {
+            for (int r = 0; r < 3; ++r)
+              if (r < valid)
+                gv[r] = g[r];
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            v[r] *= (float)gv[r];
+        }
+        if (p.accumulate) {
+          if (valid == 4) {
+            if constexpr (kStage) {
               const f16x4 old = *(const f16x4_u *)dst;
 #pragma unroll
               for (int r = 0; r < 4; ++r)
                 v[r] += (float)old[r];
+            } else {
+              const f32x4 old = *(const f32x4_u *)dst;
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                v[r] += old[r];
             }
-            *(f16x4_u *)dst =
-                f16x4{(f16)v[0], (f16)v[1], (f16)v[2], (f16)v[3]};
+          } else {
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+              if (r < valid)
+                v[r] += (float)dst[r];
           }
+        }
+        if constexpr (kStage) {
+          const int srow = i * 16 + (lane & 15);
+          const int byte = (j * 16 + 4 * (lane >> 4)) * 2;
+          *(f16x4 *)(stage + srow * OROW +
+                     (((byte >> 4) ^ (srow & (OCH - 1))) << 4) + (byte & 15)) =
+              f16x4{(f16)v[0], (f16)v[1], (f16)v[2], (f16)v[3]};
+        } else if (valid == 4) {
+          const f32x4 o = {v[0], v[1], v[2], v[3]};
+          if (p.through)
+            store_through16(dst, __builtin_bit_cast(i32x4, o));
+          else
+            *(f32x4_u *)dst = o;
         } else {
 #pragma unroll
           for (int r = 0; r < 3; ++r)
-            if (r < valid) {
-              if (mul)
-                v[r] *= (float)mul[row * p.epi.ld_mul + col + r];
-              store_out(dst + r, v[r],
-                        p.accumulate ? kStoreAccumulate : kStorePlain);
-            }
+            if (r < valid)
+              dst[r] = (OutT)v[r];
         }
+      }
+    }
+  }
+  if constexpr (kStage) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < WTM * OCH / 64; ++t) {
+      const int srow = (t * 64 + lane) / OCH, ch = (t * 64 + lane) % OCH;
+      const int64_t row = row0 + srow, col = col0 + ch * 8;
+      if (row >= p.M || col >= p.N)
+        continue;
+      const i32x4 v = *(const i32x4 *)(stage + srow * OROW +
+                                       ((ch ^ (srow & (OCH - 1))) << 4));
+      OutT *dst = C + row * p.ldc + col;
+      if (col + 8 <= p.N) {
+        if (p.through)
+          store_through16(dst, v);
+        else
+          *(i32x4_u *)dst = v;
+      } else {
+        const f16x8 h = __builtin_bit_cast(f16x8, v);
+#pragma unroll
+        for (int r = 0; r < 7; ++r)
+          if (col + r < p.N)
+            dst[r] = h[r];
       }
     }
   }
@@ -594,6 +658,7 @@ static hipError_t launch_ragged(const MatmulArgs &a, int splits, int k_split) {
   p.s_mul = epi_batch_stride(a);
   p.epi = make_epi(a);
   p.accumulate = a.accumulate;
+  p.through = a.m * a.n * a.batch * (int64_t)sizeof(OutT) >= kStoreThroughBytes;
   p.k_split = k_split;
   p.counters = (unsigned *)a.workspace;
   p.partials = (float *)((char *)a.workspace + kWorkspaceCounterBytes);

@@ -479,12 +479,87 @@ double general_us(const GeneralConfig &c, int64_t workgroups, int64_t stages,
   return t;
 }
 
+// Modeled time of a split-K configuration at `splits` splits, in us, as
+// general_us prices the general kernel: a K stage of a lone workgroup, a CU's
+// share of one of two, a round; then the operands' bytes at the rate of a
+// warm cache, and for splits the last arriver's wait, its sum over the
+// partials, and their traffic. Constants fitted to 1500 timings of 203 shapes
+// (m 5..2000, n 256..11008, k 128..11008): the pick is 0.4 % slower than the
+// best split configuration of those on average, 8 % at most, where est_ns
+// was 12 %. 0 for a configuration that was not fitted.
+double split_us(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
+                int64_t tiles, int64_t splits, int64_t k_split, int64_t cus) {
+  struct Rates {
+    const char *name;
+    double alone, shared, round;
+  };
+  static const Rates kRates[] = {
+      {"f16_nn_32x128x64_w1x4_s4_sk", 0.265, 0.240, 0.785},
+      {"f16_nn_64x128x64_w2x2_s4_sk", 0.306, 0.199, 1.88},
+      {"f16_nn_128x128x64_w2x2_s4_sk", 0.452, 0.167, 2.75},
+      {"f16f32_nn_32x128x64_w1x4_s4_sk", 0.251, 0.220, 0.629},
+      {"f16_tn_32x128x64_w1x4_s4_sk", 0.045, 0.240, 0.831},
+      {"f16_tn_128x128x64_w2x2_s4_sk", 0.205, 0.454, 2.72},
+      {"w8a16_nn_32x256x64_w1x4_s4_sk", 0.218, 0.431, 3.44},
+      {"w8a16_nn_128x256x64_w2x4_s4_sk", 0.178, 0.720, 3.29},
+      {"i8_tn_32x128x128_w1x4_s4_sk", 0.246, 0.309, 1.47},
+      {"i8_tn_128x128x128_w2x2_s4_sk", 0.406, 0.242, 3.04},
+      {"i8_nn_32x256x128_w1x4_s4_sk", 0.483, 0.0932, 1.17},
+      {"i8_nn_128x256x128_w2x4_s3_sk", 0.425, 0.638, 2.48}};
+  const Rates *r = nullptr;
+  for (const Rates &x : kRates)
+    if (strcmp(x.name, c.name) == 0)
+      r = &x;
+  if (!r)
+    return 0.0;
+  const int64_t batch = d.batch > 0 ? d.batch : 1;
+  const int64_t held = c.lds_bytes <= 80 * 1024 ? 2 : 1;
+  const int64_t per_cu = (tiles * splits * batch + cus - 1) / cus;
+  const int64_t whole = per_cu / held, rest = per_cu % held;
+  auto stage = [&](int64_t resident) {
+    const double t = r->shared * (double)resident;
+    return resident == 0 ? 0.0 : t > r->alone ? t : r->alone;
+  };
+  double t = (double)(k_split / c.bk) *
+                 ((double)whole * stage(held) + stage(rest)) +
+             (double)(whole + (rest > 0)) * r->round;
+  const double bytes = (double)batch * (double)d.k *
+                       ((double)d.m * elem_bytes(d.a_elem) +
+                        (double)d.n * elem_bytes(d.b_elem));
+  if (t < bytes / 13.4e6)
+    t = bytes / 13.4e6;
+  if (splits > 1) {
+    const double rows = (double)(d.m < c.bm ? d.m : c.bm);
+    t += 3.1 + 0.588 * (double)splits * rows * c.bn / c.threads / 16.0 +
+         0.31e-6 * (double)(tiles * splits * batch) * rows * c.bn * 4.0;
+  }
+  return t;
+}
+
 GeneralKind general_kind(const iree_mi355x_matmul_desc_t &d) {
   if (d.has_scale)
     return kGeneralW8A16;
   if (d.a_elem == IREE_MI355X_ELEM_I8)
     return kGeneralI8I32;
   return d.c_elem == IREE_MI355X_ELEM_F32 ? kGeneralF16F32 : kGeneralF16F16;
+}
+
+double operand_bytes(GeneralKind kind, int64_t m, int64_t n, int64_t k,
+                     int64_t batch) {
+  return (double)batch * (double)k *
+         ((double)m * (kind == kGeneralI8I32 ? 1 : 2) +
+          (double)n * (kind >= kGeneralI8I32 ? 1 : 2));
+}
+
+// general_us of a plan.
+double general_plan_us(const iree_mi355x_matmul_desc_t &d,
+                       const GeneralPlan &g, int64_t cus) {
+  int count = 0;
+  const GeneralConfig &c = general_configs(&count)[g.index];
+  const int64_t batch = d.batch > 0 ? d.batch : 1;
+  const int64_t ke = c.kind == kGeneralI8I32 ? 128 : 64;
+  return general_us(c, g.tiles * batch * g.splits, g.k_split / ke, g.splits,
+                    operand_bytes(c.kind, d.m, d.n, d.k, batch), cus);
 }
 
 }  // namespace
@@ -502,10 +577,7 @@ bool plan_general(GeneralKind kind, int64_t m, int64_t n, int64_t k,
   const int64_t a_row = a_trans ? m : k, b_row = b_trans ? k : n;
   const bool any = wide || a_row < (kind == kGeneralI8I32 ? 16 : 8) ||
                    b_row < (kind >= kGeneralI8I32 ? 16 : 8);
-  const double bytes =
-      (double)batch * (double)k *
-      ((double)m * (kind == kGeneralI8I32 ? 1 : 2) +
-       (double)n * (kind >= kGeneralI8I32 ? 1 : 2));
+  const double bytes = operand_bytes(kind, m, n, k, batch);
   double best = 0;
   bool found = false;
   for (int i = 0; i < count; ++i) {
@@ -598,10 +670,89 @@ int32_t iree_mi355x_classify_matmul(const iree_mi355x_matmul_desc_t *d) {
   return IREE_MI355X_FAMILY_GENERAL;
 }
 
-int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
-                            iree_mi355x_matmul_plan_t *plan) {
-  if (!d || !plan)
-    return IREE_MI355X_INVALID_ARGUMENT;
+}  // extern "C"
+
+namespace {
+
+// The plan fields of a general matmul.
+void describe_general(const iree_mi355x_matmul_desc_t &d,
+                      const GeneralPlan &g, iree_mi355x_matmul_plan_t *plan) {
+  int count = 0;
+  const GeneralConfig &c = general_configs(&count)[g.index];
+  memset(plan, 0, sizeof(*plan));
+  plan->family = IREE_MI355X_FAMILY_GENERAL;
+  plan->config_index = -1;
+  snprintf(plan->config_name, sizeof(plan->config_name), "%s", c.name);
+  plan->tile_m = c.bm;
+  plan->tile_n = c.bn;
+  plan->tile_k = c.kind == kGeneralI8I32 ? 128 : 64;
+  plan->lds_bytes = c.lds_bytes;
+  const int64_t batch = d.batch > 0 ? d.batch : 1;
+  plan->workgroups = g.tiles * g.splits * batch;
+  plan->threads = c.threads;
+  plan->splits = g.splits;
+  plan->k_split = g.k_split;
+  plan->workspace_bytes = g.workspace;
+  const int64_t ab = elem_bytes(d.a_elem), bb = elem_bytes(d.b_elem);
+  plan->traffic_bytes = batch * (ab * d.m * d.k * ((d.n + c.bn - 1) / c.bn) +
+                                 bb * d.n * d.k * ((d.m + c.bm - 1) / c.bm));
+}
+
+// Ranks the split-K configurations again by split_us where est_ns picked one,
+// and beyond 128 rows the general kernel with them, among the plans whose
+// workspace the caller has. Up to 128 rows a shape that est_ns splits stays
+// split, on the macro-tiles (the partial tiles are small there).
+void refine_split(const iree_mi355x_matmul_desc_t &d, int64_t budget,
+                  int64_t cus, size_t workspace_limit, Candidate *best,
+                  GeneralPlan *general, bool *use_general) {
+  int count = 0;
+  const FastConfig *cfgs = fast_configs(&count);
+  double t_best = split_us(d, cfgs[best->index], best->tiles, best->splits,
+                           best->k_split, cus);
+  if (t_best <= 0.0)
+    return;
+  const bool keep_split = d.m <= 128 && best->splits > 1;
+  // The first pick stands unless another is modeled faster by more than the
+  // fit is off (short sums of few rows are off most).
+  t_best = (size_t)best->workspace > workspace_limit
+               ? 1e30
+               : (d.m <= 128 ? 0.85 : 0.92) * t_best;
+  static const int kSplitChoices[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
+  for (int i = 0; i < count; ++i) {
+    if (!cfgs[i].split_k || cfgs[i].table_only || cfgs[i].lds_bytes > budget)
+      continue;
+    for (int forced : kSplitChoices) {
+      Candidate c;
+      if (!evaluate(d, cfgs[i], i, cus, &c, true, forced) ||
+          c.splits != forced || (keep_split && c.splits == 1) ||
+          (c.splits > 1 && c.k_split < kMinStagesPerSplit * cfgs[i].bk) ||
+          (size_t)c.workspace > workspace_limit)
+        continue;
+      const double t =
+          split_us(d, cfgs[i], c.tiles, c.splits, c.k_split, cus);
+      if (t > 0.0 && t < t_best) {
+        *best = c;
+        t_best = t;
+      }
+    }
+  }
+  if (d.m <= 128 || !plan_general_desc(d, false, workspace_limit, general))
+    return;
+  const double t = general_plan_us(d, *general, cus);
+  *use_general = t < 0.92 * t_best;
+}
+
+}  // namespace
+
+namespace ihp {
+
+// The plan of a call with `workspace_limit` bytes of workspace, and the
+// workspace below which the call is refused: what the plan of the first
+// ranking needs, whether or not the refined one needs it (the plan's
+// workspace_bytes is the larger of the two).
+int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
+                iree_mi355x_matmul_plan_t *plan, size_t *required) {
+  *required = 0;
   memset(plan, 0, sizeof(*plan));
   plan->config_index = -1;
   const int32_t family = iree_mi355x_classify_matmul(d);
@@ -652,6 +803,7 @@ int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
     plan->workspace_bytes =
         (int64_t)gemv_workspace_bytes(d->m, d->n, d->k, wb, batch);
     plan->traffic_bytes = batch * (d->n * d->k * wb + d->m * d->k * 2);
+    *required = (size_t)plan->workspace_bytes;
     return IREE_MI355X_OK;
   }
 
@@ -735,6 +887,18 @@ int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
     }
     if (best.index < 0)
       return IREE_MI355X_UNSUPPORTED;
+    *required = best.workspace > 0 ? (size_t)best.workspace : 0;
+    if (!plan->from_tuned_table && cfgs[best.index].split_k) {
+      GeneralPlan g;
+      bool use_general = false;
+      refine_split(*d, budget, cus, workspace_limit, &best, &g, &use_general);
+      if (use_general) {
+        describe_general(*d, g, plan);
+        if ((size_t)plan->workspace_bytes < *required)
+          plan->workspace_bytes = (int64_t)*required;
+        return IREE_MI355X_OK;
+      }
+    }
     const FastConfig &c = cfgs[best.index];
     plan->config_index = best.index;
     snprintf(plan->config_name, sizeof(plan->config_name), "%s", c.name);
@@ -750,33 +914,30 @@ int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
     plan->splits = best.splits;
     plan->k_split = best.k_split;
     plan->stream_k_steps = best.sk_steps;
-    plan->workspace_bytes = best.workspace;
+    plan->workspace_bytes = (size_t)best.workspace > *required
+                                ? best.workspace
+                                : (int64_t)*required;
     plan->traffic_bytes = best.traffic;
     return IREE_MI355X_OK;
   }
 
-  // General kernel, with all the workspace its split wants.
   GeneralPlan g;
-  if (!plan_general_desc(*d, false, (size_t)-1, &g))
+  if (!plan_general_desc(*d, false, workspace_limit, &g))
     return IREE_MI355X_UNSUPPORTED;
-  int count = 0;
-  const GeneralConfig &c = general_configs(&count)[g.index];
-  snprintf(plan->config_name, sizeof(plan->config_name), "%s", c.name);
-  plan->tile_m = c.bm;
-  plan->tile_n = c.bn;
-  plan->tile_k = c.kind == kGeneralI8I32 ? 128 : 64;
-  plan->lds_bytes = c.lds_bytes;
-  const int64_t batch = d->batch > 0 ? d->batch : 1;
-  plan->workgroups = g.tiles * g.splits * batch;
-  plan->threads = c.threads;
-  plan->splits = g.splits;
-  plan->k_split = g.k_split;
-  plan->workspace_bytes = g.workspace;
-  const int64_t ab = elem_bytes(d->a_elem), bb = elem_bytes(d->b_elem);
-  plan->traffic_bytes =
-      batch * (ab * d->m * d->k * ((d->n + c.bn - 1) / c.bn) +
-               bb * d->n * d->k * ((d->m + c.bm - 1) / c.bm));
+  describe_general(*d, g, plan);
   return IREE_MI355X_OK;
+}
+
+}  // namespace ihp
+
+extern "C" {
+
+int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
+                            iree_mi355x_matmul_plan_t *plan) {
+  if (!d || !plan)
+    return IREE_MI355X_INVALID_ARGUMENT;
+  size_t required = 0;
+  return plan_matmul(d, (size_t)-1, plan, &required);
 }
 
 int iree_mi355x_mfma_config_count(void) {
