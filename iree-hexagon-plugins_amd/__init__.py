@@ -667,6 +667,8 @@ def attention_constants(batch, heads, seq_q, seq_kv, head_dim, scale, flags,
 # older buffer, so the ones a larger buffer replaces stay alive too. Two
 # streams never share a buffer (their arrival counters would collide).
 _STREAM_WORKSPACES: dict = {}
+# (pointer, bytes) of the newest flat buffer of a (device index, stream).
+_FLAT_WORKSPACES: dict = {}
 _MIN_WORKSPACE = 64 << 20
 
 
@@ -715,7 +717,21 @@ def stream_workspace(need: int, device=None, stream=None, layout=None,
     with torch.cuda.stream(s):
         buf = torch.zeros(size, dtype=torch.uint8, device=dev)
     bufs.append(buf)
+    if layout is None:
+        _FLAT_WORKSPACES[dev.index, s.cuda_stream] = (buf.data_ptr(), size)
     return buf.data_ptr(), size
+
+
+def _call_workspace(need, index, stream):
+    """stream_workspace of a flat call on device `index` and a raw stream."""
+    if need <= 0:
+        return None, 0
+    have = _FLAT_WORKSPACES.get((index, stream))
+    if have is not None and have[1] >= need:
+        return have
+    import torch
+    return stream_workspace(need, torch.device("cuda", index), stream,
+                            partial=True)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -734,11 +750,21 @@ def _batch_workspace_need(batch, m, n, k, flags) -> int:
 def _stream_ptr(stream=None):
     """hipStream_t of a torch stream (None: the current one); an int is taken
     as the raw handle (0: the null stream)."""
+    if stream is None:
+        return _current_stream_ptr()
     if isinstance(stream, int):
         return stream
+    return stream.cuda_stream
+
+
+def _current_stream_ptr():
+    """torch.cuda.current_stream().cuda_stream without the Stream object
+    (2.6 us a call, of 11 for a small matmul; 0.2 us here)."""
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch.cuda.current_device())
 
 
 def _unit_col(t) -> bool:
@@ -823,8 +849,8 @@ def matmul(a, b, c=None, *, b_transposed=False, accumulate=False,
     s = _stream_ptr(stream)
     if a.dtype != torch.int8 and out_dtype == torch.float32:
         flags |= OUT_F32
-    ws, wsb = stream_workspace(_matmul_workspace_need(m, n, k, flags),
-                               a.device, s, partial=True)
+    ws, wsb = _call_workspace(_matmul_workspace_need(m, n, k, flags),
+                              a.get_device(), s)
     if a.dtype == torch.int8:
         _check(lib.iree_mi355x_matmul_i8(a.data_ptr(), b.data_ptr(),
                                          c.data_ptr(), m, n, k, a.stride(0),
@@ -924,8 +950,8 @@ def batch_matmul(a, b, c=None, *, b_transposed=False, accumulate=False,
              (OUT_F32 if out_dtype == torch.float32 else 0) |
              (A_TRANSPOSED if a_transposed else 0))
     st = _stream_ptr(stream)
-    ws, wsb = stream_workspace(_batch_workspace_need(batch, m, n, k, flags),
-                               a.device, st, partial=True)
+    ws, wsb = _call_workspace(_batch_workspace_need(batch, m, n, k, flags),
+                              a.get_device(), st)
     _check(lib.iree_mi355x_batch_matmul_f16(
         a3.data_ptr(), b3.data_ptr(), c3.data_ptr(), batch, m, n, k,
         a3.stride(1), b3.stride(1), c3.stride(1), sa, sb, sc, flags,
@@ -965,8 +991,8 @@ def quantized_matmul(x, w, scale, y=None, *, w_transposed=False, stream=None):
         y = torch.empty((m, n), dtype=torch.float16, device=x.device)
     flags = B_TRANSPOSED if w_transposed else 0
     st = _stream_ptr(stream)
-    ws, wsb = stream_workspace(_matmul_workspace_need(m, n, k, flags),
-                               x.device, st, partial=True)
+    ws, wsb = _call_workspace(_matmul_workspace_need(m, n, k, flags),
+                              x.get_device(), st)
     _check(lib.iree_mi355x_w8a16_matmul(
         x.data_ptr(), w.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k,
         x.stride(0), w.stride(0), y.stride(0), flags, ws, wsb, st))
@@ -1000,13 +1026,19 @@ def _attention_workspace_need(b, h, hkv, sq, skv, d, dv, flags) -> int:
     return library().iree_mi355x_attention_workspace_bytes(ctypes.byref(a))
 
 
+# iree_mi355x_attention_t and iree_mi355x_attention_strides_t as bytes.
+_ATTENTION_ARGS = struct.Struct("@5P7qfI16q")
+_ATTENTION_STRIDES = struct.Struct("@12q")
+
+
 def _fused_layout(st, pointers, sq, skv) -> bool:
-    """Strides and bases (or-ed) as iree_mi355x_attention_f16_strided demands
-    of a head dim of 64 or 128: it refuses the others, with a workspace too."""
+    """The 12 strides and the bases (or-ed) as
+    iree_mi355x_attention_f16_strided demands of a head dim of 64 or 128: it
+    refuses the others, with a workspace too."""
     every = 0
-    for t in (st.q, st.k, st.v, st.o):
-        every |= t[0] | t[1] | t[2]
-    span = max((sq - 1) * st.q[2], (skv - 1) * max(st.k[2], st.v[2])) * 2
+    for x in st:
+        every |= x
+    span = max((sq - 1) * st[2], (skv - 1) * max(st[5], st[8])) * 2
     return (every & 7) == 0 and (pointers & 15) == 0 and span < (1 << 32) - 256
 
 
@@ -1074,23 +1106,19 @@ def attention(q, k, v, o=None, *, causal=True, scale=None, mask=None,
             q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), b, h, sq,
             skv, d, float(scale), flags, stp))
         return o
-    st = AttentionStrides(q.stride()[:3], k.stride()[:3], v.stride()[:3],
-                          o.stride()[:3])
+    st = (*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *o.stride()[:3])
     qp, kp, vp, op = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr()
     if fast and not (need and _fused_layout(st, qp | kp | vp | op, sq, skv)):
         _check(lib.iree_mi355x_attention_f16_strided(
             qp, kp, vp, op, b, h, hkv, sq, skv, d, float(scale), flags,
-            ctypes.byref(st), stp))
+            _ATTENTION_STRIDES.pack(*st), stp))
         return o
-    a = AttentionArgs(q=qp, k=kp, v=vp, o=op, batch=b, heads=h, kv_heads=hkv,
-                      seq_q=sq, seq_kv=skv, head_dim=d, head_dim_v=dv,
-                      scale=float(scale), flags=flags, strides=st)
-    if mask is not None:
-        a.mask = mask.data_ptr()
-        a.mask_strides[:] = mask.stride()
-    ws, wsb = stream_workspace(need, q.device, stp, partial=True)
-    _check(lib.iree_mi355x_attention_with_workspace(ctypes.byref(a), ws, wsb,
-                                                    stp))
+    mp, ms = (0, (0, 0, 0, 0)) if mask is None else (mask.data_ptr(),
+                                                     mask.stride())
+    args = _ATTENTION_ARGS.pack(qp, kp, vp, op, mp, b, h, hkv, sq, skv, d, dv,
+                                scale, flags, *st, *ms)
+    ws, wsb = _call_workspace(need, q.get_device(), stp)
+    _check(lib.iree_mi355x_attention_with_workspace(args, ws, wsb, stp))
     return o
 
 

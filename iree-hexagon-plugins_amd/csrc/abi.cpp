@@ -145,16 +145,66 @@ static int launch_mfma(MatmulArgs &args, const iree_mi355x_matmul_plan_t &plan,
 int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
                 iree_mi355x_matmul_plan_t *plan, size_t *required);
 
+// plan_general for a described matmul (planner.cpp).
+bool plan_general_desc(const iree_mi355x_matmul_desc_t &d, bool wide,
+                       size_t workspace_limit, GeneralPlan *plan);
+
+// plan_matmul through a small per-thread table: a plan depends on nothing but
+// the description and the workspace, and ranking the split configurations
+// takes 3-6 us of host time, as long as the kernel of a small call.
+static int cached_plan(const iree_mi355x_matmul_desc_t &d,
+                       size_t workspace_limit, iree_mi355x_matmul_plan_t *plan,
+                       GeneralPlan *general, size_t *required) {
+  struct Entry {
+    iree_mi355x_matmul_desc_t desc;
+    size_t limit;
+    iree_mi355x_matmul_plan_t plan;
+    GeneralPlan general;  // of a plan of the general family
+    size_t required;
+    bool used;
+  };
+  static thread_local Entry table[64];
+  uint64_t h = (uint64_t)d.m * 0x9E3779B97F4A7C15ull ^
+               (uint64_t)d.n * 0xC2B2AE3D27D4EB4Full ^
+               (uint64_t)d.k * 0x165667B19E3779F9ull ^
+               ((uint64_t)d.flags << 40) ^ ((uint64_t)d.b_elem << 50) ^
+               (uint64_t)d.batch;
+  h ^= h >> 29;
+  Entry &e = table[(h * 0x9E3779B97F4A7C15ull) >> 58];
+  // desc_init zeroes the padding, so descriptions compare as bytes
+  if (e.used && e.limit == workspace_limit &&
+      memcmp(&e.desc, &d, sizeof(d)) == 0) {
+    *plan = e.plan;
+    *general = e.general;
+    *required = e.required;
+    return IREE_MI355X_OK;
+  }
+  int st = plan_matmul(&d, workspace_limit, plan, required);
+  if (st == IREE_MI355X_OK && plan->family == IREE_MI355X_FAMILY_GENERAL &&
+      !plan_general_desc(d, false, workspace_limit, general))
+    st = IREE_MI355X_UNSUPPORTED;
+  if (st == IREE_MI355X_OK) {
+    memcpy(&e.desc, &d, sizeof(d));
+    e.limit = workspace_limit;
+    e.plan = *plan;
+    e.general = *general;
+    e.required = *required;
+    e.used = true;
+  }
+  return st;
+}
+
 // Plans a call within the workspace it has (a validate-only call: within
 // workspace_bytes, whether or not a buffer is given yet) and refuses one that
 // has less than it must. *done: nothing is left to run (refused or validated).
 static int plan_call(const char *who, const iree_mi355x_matmul_desc_t &desc,
                      const void *workspace, size_t workspace_bytes,
-                     iree_mi355x_matmul_plan_t *plan, bool *done) {
+                     iree_mi355x_matmul_plan_t *plan, GeneralPlan *general,
+                     bool *done) {
   size_t required = 0;
   *done = true;
-  if (plan_matmul(&desc, workspace || g_dry_run ? workspace_bytes : 0, plan,
-                  &required) != IREE_MI355X_OK)
+  if (cached_plan(desc, workspace || g_dry_run ? workspace_bytes : 0, plan,
+                  general, &required) != IREE_MI355X_OK)
     return fail(IREE_MI355X_UNSUPPORTED, "%s: no plan", who);
   if (dry_run(plan->workspace_bytes))
     return ok();
@@ -163,22 +213,18 @@ static int plan_call(const char *who, const iree_mi355x_matmul_desc_t &desc,
   return st;
 }
 
-// plan_general for a described matmul (planner.cpp).
-bool plan_general_desc(const iree_mi355x_matmul_desc_t &d, bool wide,
-                       size_t workspace_limit, GeneralPlan *plan);
-
-// The general matmul of `desc`, its K split within the workspace the call
-// has.
+// The general matmul of `desc` with the plan of plan_call, or for a wide
+// pitch one of its own, its K split within the workspace the call has.
 static int run_general(const char *who, MatmulArgs &args,
-                       const iree_mi355x_matmul_desc_t &desc, void *workspace,
-                       size_t workspace_bytes) {
-  GeneralPlan plan;
+                       const iree_mi355x_matmul_desc_t &desc, GeneralPlan plan,
+                       void *workspace, size_t workspace_bytes) {
   const bool wide =
       args.lda * (desc.a_elem == IREE_MI355X_ELEM_I8 ? 1 : 2) >=
           kMaxFastPitchBytes ||
       args.ldb * (desc.b_elem == IREE_MI355X_ELEM_I8 ? 1 : 2) >=
           kMaxFastPitchBytes;
-  if (!plan_general_desc(desc, wide, workspace ? workspace_bytes : 0, &plan))
+  if (wide && !plan_general_desc(desc, true, workspace ? workspace_bytes : 0,
+                                 &plan))
     return fail(IREE_MI355X_UNSUPPORTED, "%s: no plan", who);
   args.workspace = plan.workspace > 0 ? workspace : nullptr;
   return launch_status(launch_general(args, plan), who);
@@ -301,14 +347,16 @@ static int matmul_f16_run(const char *who, MatmulArgs &args, uint32_t flags,
   desc.b_aligned16 = fast_operand(args.b, args.ldb * 2, args.sb * 2);
   desc.batch = args.batch;
   iree_mi355x_matmul_plan_t plan;
+  GeneralPlan general = {};
   bool done = false;
   const int st =
-      plan_call(who, desc, workspace, workspace_bytes, &plan, &done);
+      plan_call(who, desc, workspace, workspace_bytes, &plan, &general,
+                 &done);
   if (done)
     return st;
   switch (plan.family) {
     case IREE_MI355X_FAMILY_GENERAL:
-      return run_general(who, args, desc, workspace, workspace_bytes);
+      return run_general(who, args, desc, general, workspace, workspace_bytes);
     case IREE_MI355X_FAMILY_GEMV:
       return launch_status(launch_gemv(args, 2, nullptr, out_f32, workspace),
                            "gemv_f16");
@@ -468,12 +516,15 @@ int iree_mi355x_matmul_i8(const int8_t *a, const int8_t *b, int32_t *c,
   desc.a_aligned16 = fast_operand(a, lda);
   desc.b_aligned16 = fast_operand(b, ldb);
   iree_mi355x_matmul_plan_t plan;
+  GeneralPlan general = {};
   bool done = false;
-  st = plan_call("matmul_i8", desc, workspace, workspace_bytes, &plan, &done);
+  st = plan_call("matmul_i8", desc, workspace, workspace_bytes, &plan, &general,
+                 &done);
   if (done)
     return st;
   if (plan.family == IREE_MI355X_FAMILY_GENERAL)
-    return run_general("matmul_i8", args, desc, workspace, workspace_bytes);
+    return run_general("matmul_i8", args, desc, general, workspace,
+                       workspace_bytes);
   return launch_mfma(args, plan, workspace, workspace_bytes, "matmul_i8");
 }
 
@@ -500,13 +551,14 @@ int iree_mi355x_w8a16_matmul(const void *x, const int8_t *w, const void *scale,
   desc.b_aligned16 = fast_operand(w, ldw);
   desc.has_scale = 1;
   iree_mi355x_matmul_plan_t plan;
+  GeneralPlan general = {};
   bool done = false;
   st = plan_call("w8a16_matmul", desc, workspace, workspace_bytes, &plan,
-                 &done);
+                 &general, &done);
   if (done)
     return st;
   if (plan.family == IREE_MI355X_FAMILY_GENERAL)
-    return run_general("w8a16_matmul", args, desc, workspace,
+    return run_general("w8a16_matmul", args, desc, general, workspace,
                        workspace_bytes);
   if (plan.family == IREE_MI355X_FAMILY_GEMV)
     return launch_status(launch_gemv(args, 1, scale, 0, workspace),
