@@ -431,14 +431,17 @@ __global__ __launch_bounds__(64 * WM *WN, WGS) void gemm_ragged_kernel(
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(tile_parts, 0, -1, 0x00027000);
     const int voff = (wave * FM * FN * 64 + lane) * 16;
+    // Fragments of rows past M are neither published nor summed.
+    const int frags = (int)((p.M - m0 - wm * WTM + 15) / 16);
 #pragma unroll
     for (int i = 0; i < FM; ++i)
+      if (i < frags)
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
-        __builtin_amdgcn_raw_buffer_store_b128(
-            __builtin_bit_cast(i32x4, acc[i][j]), rs,
-            voff + (i * FN + j) * 1024, (int)blockIdx.y * (BM * BN * 4),
-            kDeviceScope);
+        for (int j = 0; j < FN; ++j)
+          __builtin_amdgcn_raw_buffer_store_b128(
+              __builtin_bit_cast(i32x4, acc[i][j]), rs,
+              voff + (i * FN + j) * 1024, (int)blockIdx.y * (BM * BN * 4),
+              kDeviceScope);
     __shared__ unsigned last_split;
     unsigned *last = &last_split;
     wait_vmcnt<0>();  // published before it is counted
@@ -459,20 +462,32 @@ __global__ __launch_bounds__(64 * WM *WN, WGS) void gemm_ragged_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           acc[i][j][r] = 0;
-    for (int s = 0; s < splits; ++s) {
-      i32x4 v[FM][FN];
+    // 32 loads a lane in flight (the sum is a chain of memory latencies): U
+    // splits at a time, the last one again where they run out.
+    constexpr int U = 32 / (FM * FN);
+    for (int s0 = 0; s0 < splits; s0 += U) {
+      i32x4 v[U][FM][FN];
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+      for (int u = 0; u < U; ++u) {
+        const int s = s0 + u < splits ? s0 + u : splits - 1;
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-          v[i][j] = __builtin_amdgcn_raw_buffer_load_b128(
-              rs, voff + (i * FN + j) * 1024, s * (BM * BN * 4),
-              kDeviceScope);
+        for (int i = 0; i < FM; ++i)
+          if (i < frags)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+            for (int j = 0; j < FN; ++j)
+              v[u][i][j] = __builtin_amdgcn_raw_buffer_load_b128(
+                  rs, voff + (i * FN + j) * 1024, s * (BM * BN * 4),
+                  kDeviceScope);
+      }
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] += __builtin_bit_cast(Acc, v[i][j]);
+      for (int u = 0; u < U; ++u)
+        if (s0 + u < splits)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+            if (i < frags)
+#pragma unroll
+              for (int j = 0; j < FN; ++j)
+                acc[i][j] += __builtin_bit_cast(Acc, v[u][i][j]);
     }
     if (tid == 0)  // re-arm for the next call on this workspace
       __hip_atomic_store(&p.counters[tile * kCounterStride], 0u,

@@ -445,19 +445,21 @@ bool evaluate(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
 // Modeled time of a general configuration, in us. A CU holds `wgs` workgroups
 // at a time; a K stage takes a lone workgroup `alone` and a CU's share
 // `shared` for each of several; a round of workgroups adds `round`. Splits
-// add the last arriver's wait and its sum over the partial tiles. The
+// add the last arriver's wait, a round trip for every U partial tiles it
+// sums (gemm_ragged.hip) and the partials' traffic (rows below M only). The
 // constants are a fit to 2300 timings of 126 shapes (m 1..2048, n and k
 // 64..11008, every kind and layout, aligned or not, 1 to 16 splits): the pick
-// is 0.7 % slower than the best of those timed on average, 9 % at most.
-double general_us(const GeneralConfig &c, int64_t workgroups, int64_t stages,
-                  int64_t splits, double operand_bytes, int64_t cus) {
+// is 0.7 % slower than the best of those timed on average, 12 % at most.
+double general_us(const GeneralConfig &c, int64_t m, int64_t workgroups,
+                  int64_t stages, int64_t splits, double operand_bytes,
+                  int64_t cus) {
   struct Rates {
     int bm, bn;
     double alone, shared, round;
   };
-  static const Rates kRates[] = {{64, 64, 0.437, 0.270, 0.875},
-                                 {64, 128, 0.618, 0.385, 1.39},
-                                 {128, 128, 0.867, 0.434, 2.05}};
+  static const Rates kRates[] = {{64, 64, 0.403, 0.275, 0.574},
+                                 {64, 128, 0.643, 0.398, 1.16},
+                                 {128, 128, 0.971, 0.541, 1.28}};
   const Rates *r = kRates;
   while (r->bm != c.bm || r->bn != c.bn)
     ++r;
@@ -469,14 +471,15 @@ double general_us(const GeneralConfig &c, int64_t workgroups, int64_t stages,
   };
   double t = (double)stages * ((double)whole * stage(c.wgs) + stage(rest)) +
              (double)(whole + (rest > 0)) * r->round;
-  if (t < operand_bytes / 5.8e6)  // 5.8 TB/s
-    t = operand_bytes / 5.8e6;
+  if (t < operand_bytes / 5.2e6)  // 5.2 TB/s
+    t = operand_bytes / 5.2e6;
   if (splits > 1) {
-    const double tile_bytes = 4.0 * c.bm * c.bn;
-    t += 1.58 + 0.24 * (double)splits * tile_bytes / 16384.0 +
-         0.255e-6 * tile_bytes * (double)workgroups;
+    const int64_t at_once = 8 * 64 * 64 / (c.bm * c.bn);
+    const int64_t rows = m < c.bm ? (m + 15) / 16 * 16 : c.bm;
+    t += 1.26 + 0.787 * (double)((splits + at_once - 1) / at_once) +
+         0.342e-6 * (double)(workgroups * rows * c.bn * 4);
   }
-  return t;
+  return t + 3.46;  // the launch
 }
 
 // Modeled time of a split-K configuration at `splits` splits, in us, as
@@ -533,7 +536,7 @@ double split_us(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
     t += 3.1 + 0.588 * (double)splits * rows * c.bn / c.threads / 16.0 +
          0.31e-6 * (double)(tiles * splits * batch) * rows * c.bn * 4.0;
   }
-  return t;
+  return t + 2.75;  // the launch
 }
 
 GeneralKind general_kind(const iree_mi355x_matmul_desc_t &d) {
@@ -558,8 +561,8 @@ double general_plan_us(const iree_mi355x_matmul_desc_t &d,
   const GeneralConfig &c = general_configs(&count)[g.index];
   const int64_t batch = d.batch > 0 ? d.batch : 1;
   const int64_t ke = c.kind == kGeneralI8I32 ? 128 : 64;
-  return general_us(c, g.tiles * batch * g.splits, g.k_split / ke, g.splits,
-                    operand_bytes(c.kind, d.m, d.n, d.k, batch), cus);
+  return general_us(c, d.m, g.tiles * batch * g.splits, g.k_split / ke,
+                    g.splits, operand_bytes(c.kind, d.m, d.n, d.k, batch), cus);
 }
 
 }  // namespace
@@ -606,7 +609,7 @@ bool plan_general(GeneralKind kind, int64_t m, int64_t n, int64_t k,
       if (ws > 0 && (uint64_t)ws > (uint64_t)workspace_limit)
         break;
       const double t =
-          general_us(c, tiles * batch * splits, per, splits, bytes, cus);
+          general_us(c, m, tiles * batch * splits, per, splits, bytes, cus);
       if (!found || t < best) {
         found = true;
         best = t;
