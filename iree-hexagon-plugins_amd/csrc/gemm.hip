@@ -35,13 +35,18 @@ __device__ __forceinline__ void static_for(F &&f) {
 
 // ----------------------------------------------------------------------------
 // Fast path: A [M,K] K-contiguous, every extent a multiple of the macro-tile,
-// 16-byte aligned rows. Three B forms (BMODE):
+// 16-byte aligned rows. The B forms (BMODE):
 //   kBTN   B [N,K] of the A type (K-contiguous, "column-major B")
 //   kBNN16 B [K,N] f16 (N-contiguous, row-major weights)
 //   kBW8   B [K,N] int8 with a per-column f16 scale (W8A16), dequantized to
 //          f16 in registers after the LDS read, scale applied in the epilogue
 //   kBNN8  B [K,N] int8 with int8 A (row-major int8 weights: the default map
 //          of linalg.matmul and quantized_matmul), int32 accumulation
+//   kBW8T  B [N,K] int8 with a per-column f16 scale (W8A16, weights stored as
+//          [out, in]). A staged row is half as long as A's, so one 16-byte
+//          read holds a lane's weights of two MFMA K steps: step 2 p takes
+//          its first 8 bytes and step 2 p + 1 the others, and A's fragments
+//          are read at the same k (any order of k gives the same sum)
 // ----------------------------------------------------------------------------
 
 template <int CH>
@@ -143,8 +148,10 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
   constexpr int AR = MS == 32 ? 16 : 4;
   constexpr int KSB = MS == 32 ? 32 : 64;
   constexpr int KCH = KSB / 16;
-  constexpr bool kNN = BMODE != kBTN;
-  constexpr int TBB = BMODE == kBW8 ? 1 : (int)sizeof(T);  // B element bytes
+  constexpr bool kNN = BMODE != kBTN && BMODE != kBW8T;
+  constexpr bool kW8T = BMODE == kBW8T;
+  constexpr bool kScaled = b_mode_w8(BMODE);
+  constexpr int TBB = kScaled ? 1 : (int)sizeof(T);  // B element bytes
   constexpr int NT = 64 * WM * WN;
   constexpr int WTM = BM / WM, WTN = BN / WN;
   constexpr int FM = WTM / MS, FN = WTN / MS;
@@ -160,8 +167,8 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
   constexpr int A_RPW = AT ? 64 / ACH : ROWS_PER_WAVE;  // rows per wave copy
   constexpr int A_RPP = AT ? NT / ACH : ROWS_PER_PASS;  // rows per pass
   constexpr int A_PASSES = A_ROWS / A_RPP;
-  // B staging: TN rows are N (BKB bytes each); NN rows are K (BN*TBB bytes).
-  constexpr int BROW = kNN ? BN * TBB : BKB;
+  // B staging: TN rows are N (KE elements each); NN rows are K (BN*TBB bytes).
+  constexpr int BROW = kNN ? BN * TBB : KE * TBB;
   constexpr int BCH = BROW / 16;
   constexpr int B_ROWS = kNN ? KE : BN;
   constexpr int B_RPW = 64 / BCH;    // B rows per wave copy instruction
@@ -176,6 +183,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
   constexpr bool kTwoReadB = BMODE == kBNN16 || BMODE == kBNN8;
   constexpr int B_READS = kTwoReadB ? 2 * FN : FN;
   constexpr int A_READS = AT ? 2 * FM : FM;
+  // (kBW8T reads B at even steps only, for two steps at once.)
   constexpr int RD = A_READS + B_READS;
   static_assert(A_ROWS % A_RPP == 0 && B_ROWS % B_RPP == 0, "tile");
   static_assert(!AT || (sizeof(T) == 2 && !SPLIT && ACH >= 16 &&
@@ -188,6 +196,8 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
   // that period, so a lane's swizzle depends only on its row in the pass.
   static_assert(ROWS_PER_PASS % 16 == 0 && (16 / CH) * CH == 16, "swz");
   static_assert(!kNN || (BCH >= 16 && B_RPP % 8 == 0 && B_RPW <= 8), "nn");
+  static_assert(kNN || (B_RPP % 16 == 0 && (BCH == 4 || BCH == 8)), "tn");
+  static_assert(!kW8T || (CH == 8 && !AT && sizeof(T) == 2), "W8A16 [N,K]");
   // Copy passes start on the row swizzle's period (16 rows for 16x16, 32
   // for the int8 16x16 form).
   static_assert(!kNN || B_RPP % nn_swizzle_period<BMODE, MS>() == 0,
@@ -200,6 +210,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
   // reads return in issue order and lgkmcnt has 4 bits: with more than 15
   // new reads the wait also takes the oldest of them (still correct).
   constexpr int RDW = RD < 16 ? RD : 15;
+  constexpr int RDW_A = A_READS < 16 ? A_READS : 15;
   // Unsplit 256x256 16x16 tiles: the waves of wave row 0 issue the copies
   // of their SIMD partner (wave w + 4) too, and the partner none. Issuing a
   // stage's copies stalls a wave for a while (the address unit drains them
@@ -219,7 +230,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
   // registers; f16 / f32 outputs stage it through LDS as one 8- / 16-byte
   // write instead of four. (W8A16 and transposed-A tiles keep the plain
   // order: not measured.)
-  constexpr bool kSwapAB = MS == 16 && !SPLIT && BMODE != kBW8 && !AT;
+  constexpr bool kSwapAB = MS == 16 && !SPLIT && !kScaled && !AT;
   static_assert(STAGES * STAGE_BYTES <= 160 * 1024, "LDS budget");
 
   __shared__ __attribute__((aligned(1024))) char smem[STAGES * STAGE_BYTES];
@@ -300,9 +311,10 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
     }
     b_base = (const char *)Bv + n0 * TBB + k_begin * ldb_b;
   } else {
-    b_lane = (uint32_t)((wave * ROWS_PER_WAVE + ld_row) * ldb_b +
-                        ld_chunk * 16);
-    b_base = (const char *)Bv + n0 * ldb_b + k_begin * (int64_t)sizeof(T);
+    const int row = wave * B_RPW + lane / BCH;
+    b_lane = (uint32_t)(row * ldb_b +
+                        ((lane % BCH) ^ chunk_swizzle<BCH>(row)) * 16);
+    b_base = (const char *)Bv + n0 * ldb_b + k_begin * (int64_t)TBB;
   }
   IHP_LDS char *lds = (IHP_LDS char *)smem;
 
@@ -334,11 +346,12 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
                           dst + A_BYTES + (wave + DW) * B_RPW * BROW +
                               q * B_RPP * BROW);
       } else {
-        global_to_lds_16s(b_base + ka + (int64_t)q * ROWS_PER_PASS * ldb_b +
-                              (int64_t)DW * ROWS_PER_WAVE * ldb_b,
+        global_to_lds_16s(b_base + (int64_t)kt * BROW +
+                              (int64_t)q * B_RPP * ldb_b +
+                              (int64_t)DW * B_RPW * ldb_b,
                           b_lane,
-                          dst + A_BYTES + (wave + DW) * ROWS_PER_WAVE * BKB +
-                              q * ROWS_PER_PASS * BKB);
+                          dst + A_BYTES + (wave + DW) * B_RPW * BROW +
+                              q * B_RPP * BROW);
       }
     }
   };
@@ -369,11 +382,24 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
   const int rd_row = lane & (MS - 1);
   const int rd_sw = chunk_swizzle<CH>(rd_row) ^ (lane / MS);
   int koff[KSTEPS];
+  // kBW8T: lane group g = lane / MS of GR reads chunk GR p + g of its B row
+  // for the step pair p, and A's chunk 2 (GR p + g) + step % 2.
+  constexpr int GR = 64 / MS;
+  int koff_b[kW8T ? KSTEPS / 2 : 1];
+  if constexpr (kW8T) {
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks)
-    koff[ks] = ((KCH * ks) ^ rd_sw) * 16;
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      const int chunk = GR * (ks / 2) + lane / MS;
+      koff[ks] = ((2 * chunk + (ks & 1)) ^ chunk_swizzle<CH>(rd_row)) * 16;
+      koff_b[ks / 2] = (chunk ^ chunk_swizzle<BCH>(rd_row)) * 16;
+    }
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks)
+      koff[ks] = ((KCH * ks) ^ rd_sw) * 16;
+  }
   const int a_rd = (wm * WTM + rd_row) * BKB;
-  const int b_rd = A_BYTES + (wn * WTN + rd_row) * BKB;
+  const int b_rd = A_BYTES + (wn * WTN + rd_row) * BROW;
   // Read side, transposed A: the row-major B offsets below with M for N.
   int a_nn[FM];
   if constexpr (AT) {
@@ -438,6 +464,9 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
     i32x2 t[kTwoReadB ? 2 * FN : FN];
     i32x2 ta[AT ? 2 * FM : 1];
   };
+  // kBW8T: the raw weights of a step pair (two pairs where a stage has them,
+  // the next pair's read being issued before the last step's conversion).
+  i32x4 raw[kW8T ? 2 : 1][kW8T ? FN : 1];
   auto read_frags = [&](int slot, int ks, Frags &f) {
     const IHP_LDS char *st = lds + slot * STAGE_BYTES;
     if constexpr (AT) {
@@ -458,6 +487,14 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
       static_for<FN>([&](auto j) {
         f.b[j] = lds_read_16_async<decltype(j)::value * MS * BKB>(pb);
       });
+    } else if constexpr (kW8T) {
+      if (ks % 2 == 0) {
+        const IHP_LDS char *pb = st + b_rd + koff_b[ks / 2];
+        static_for<FN>([&](auto j) {
+          raw[ks / 2 % 2][j] =
+              lds_read_16_async<decltype(j)::value * MS * BROW>(pb);
+        });
+      }
     } else {
       const IHP_LDS char *pb = st + ks * KROWS * BROW;
       static_for<FN>([&](auto j) {
@@ -476,7 +513,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
   };
   // Wait until at most N reads are outstanding, pin the fragments, and
   // assemble NN B operands from the transposed reads.
-  auto frags_ready = [&](auto n, Frags &f) {
+  auto frags_ready = [&](auto n, int ks, Frags &f) {
     lgkm_wait<decltype(n)::value>();
     if constexpr (AT) {
 #pragma unroll
@@ -502,6 +539,18 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
         lgkm_tie2(f.t[2 * j + 1]);
         f.b[j] = i32x4{f.t[2 * j][0], f.t[2 * j][1], f.t[2 * j + 1][0],
                        f.t[2 * j + 1][1]};
+      }
+    } else if constexpr (kW8T) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        i32x4 &q = raw[ks / 2 % 2][j];
+        if (ks % 2 == 0)
+          lgkm_tie(q);
+        f.b[j] = ks % 2 == 0 ? i8x8_to_f16x8(i32x2{q[0], q[1]})
+                             : i8x8_to_f16x8(i32x2{q[2], q[3]});
+        // converted before the next read into q is issued
+        if (ks % 2 == 1)
+          lgkm_tie(f.b[j]);
       }
     } else {
 #pragma unroll
@@ -552,7 +601,10 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
       const int cur = ks & 1, nxt = cur ^ 1;
       if (ks + 1 < KSTEPS) {
         read_frags(slot, ks + 1, fr[nxt]);
-        frags_ready(std::integral_constant<int, RDW>(), fr[cur]);
+        if (kW8T && ks % 2 == 0)  // the next step reads A alone
+          frags_ready(std::integral_constant<int, RDW_A>(), ks, fr[cur]);
+        else
+          frags_ready(std::integral_constant<int, RDW>(), ks, fr[cur]);
       } else if constexpr (decltype(handoff)::value) {
         // Stage handoff: this step's fragments are in registers (all LDS
         // reads done), stage kt+1 must have landed for every wave, and every
@@ -560,7 +612,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
         // with stage kt+STAGES. With EXACT this wave has issued every copy
         // up to stage kt+STAGES-1, so stage kt+1 has landed once at most
         // STAGES-2 stages of copies remain in flight; otherwise wait for all.
-        frags_ready(std::integral_constant<int, 0>(), fr[cur]);
+        frags_ready(std::integral_constant<int, 0>(), ks, fr[cur]);
         if constexpr (decltype(exact)::value)
           wait_vmcnt<(STAGES - 2) * LOADS_PER_STAGE * CPM>();
         else
@@ -570,7 +622,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
           load_passes(First(), All(), kt + STAGES, slot);
         read_frags((kt + 1) % STAGES, 0, fr[nxt]);
       } else {
-        frags_ready(std::integral_constant<int, 0>(), fr[cur]);
+        frags_ready(std::integral_constant<int, 0>(), ks, fr[cur]);
       }
       // Issue order. With 16x16 fragments and FN >= 4 the A index runs
       // innermost, boustrophedon, so the B operand changes once per FM
@@ -688,7 +740,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
           if (SPLIT && row >= M)
             continue;
           float v = stage[cc * PITCH + rr];
-          if constexpr (BMODE == kBW8)
+          if constexpr (kScaled)
             v *= (float)scale[col];
           store_out(C + row * ldc + col, epi_apply(v, row, col, epi),
                     store_mode);
@@ -732,7 +784,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
 #pragma unroll
           for (int j = 0; j < FN; ++j) {
             float sc = 1.0f;
-            if constexpr (BMODE == kBW8)
+            if constexpr (kScaled)
               sc = (float)scale[gcol0 + j * MS + col_l];
             if constexpr (kSwapAB && !kIntOut) {
               // four consecutive columns of one row: one 8- or 16-byte write
@@ -763,7 +815,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
                 *(OutT *)(ws + off) = acc[i][j][r];
               } else {
                 float v = (float)acc[i][j][r];
-                if constexpr (BMODE == kBW8)
+                if constexpr (kScaled)
                   v *= sc;
                 *(OutT *)(ws + off) = (OutT)v;
               }
@@ -810,7 +862,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         float sc = 1.0f;
-        if constexpr (BMODE == kBW8)
+        if constexpr (kScaled)
           sc = (float)scale[n0 + wn * WTN + j * MS + col_l];
 #pragma unroll
         for (int r = 0; r < AR; ++r) {
@@ -824,7 +876,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
             store_out(dst, acc[i][j][r], store_mode);
           } else {
             float v = (float)acc[i][j][r];
-            if constexpr (BMODE == kBW8)
+            if constexpr (kScaled)
               v *= sc;
             store_out(dst, v, store_mode);
           }
@@ -919,7 +971,7 @@ __global__ __launch_bounds__(64 * WM *WN, 1) void gemm_lds_kernel(
             store_out(C + row * ldc + col, sum[e], store_mode);
           } else {
             float v = (float)sum[e];
-            if constexpr (BMODE == kBW8)
+            if constexpr (kScaled)
               v *= (float)scale[col];
             if constexpr (decltype(with_epi)::value)
               v = epi_apply(v, row, col, epi);
@@ -1075,6 +1127,10 @@ static hipError_t launch_column_split(const MatmulArgs &a) {
 #define IHP_FAST_CONFIG_S_TABLE(NAME, MODE, T, OUT, BM, BN, BKB, WM, WN, ST)   \
   IHP_FAST_CONFIG_XT(NAME, MODE, T, OUT, BM, BN, BKB, WM, WN, ST, true, false, \
                      32, 1)
+// W8A16 with weights [N,K], weighed against the general kernel by split_us.
+#define IHP_FAST_CONFIG_W8T(NAME, BM, BN, WM, WN, ST, SPLIT)                   \
+  IHP_FAST_CONFIG_XT(NAME, kBW8T, f16, f16, BM, BN, 128, WM, WN, ST, SPLIT,   \
+                     false, 32, 1)
 #define IHP_FAST_CONFIG_XT(NAME, MODE, T, OUT, BM, BN, BKB, WM, WN, ST, SPLIT, \
                            AT, MS, TABLE)                                     \
   {NAME,                                                                      \
@@ -1092,7 +1148,7 @@ static hipError_t launch_column_split(const MatmulArgs &a) {
    ST,                                                                        \
    ST * (BM * BKB + (MODE == kBTN ? BN * BKB                                  \
                                   : (BKB / (int)sizeof(T)) * BN *             \
-                                        (MODE == kBW8 ? 1 : (int)sizeof(T)))),\
+                                        (b_mode_w8(MODE) ? 1 : (int)sizeof(T)))),\
    &launch_fast<T, OUT, BM, BN, BKB, WM, WN, ST, MODE, SPLIT, AT, MS>,      \
    MS,                                                                        \
    TABLE}
@@ -1240,6 +1296,13 @@ static const FastConfig kFastConfigs[] = {
                      kBNN16, f16, float, 128, false, 256, 256, 2, 16, 256, 128, 2, 16),
     IHP_COLUMN_SPLIT("f16f32_tn_", "256x256x64_w2x4_s2_m16", "256x128x64_w2x4_s2_m16",
                      kBTN, f16, float, 128, false, 256, 256, 2, 16, 256, 128, 2, 16),
+    // W8A16 with weights [N,K]: kept last, past the configurations that
+    // iree_mi355x_mfma_config_count lists
+    IHP_FAST_CONFIG_W8T("w8a16_tn_256x256x64_w2x4_s3", 256, 256, 2, 4, 3, false),
+    IHP_FAST_CONFIG_W8T("w8a16_tn_128x256x64_w2x4_s4", 128, 256, 2, 4, 4, false),
+    IHP_FAST_CONFIG_W8T("w8a16_tn_128x256x64_w2x4_s4_sk", 128, 256, 2, 4, 4, true),
+    IHP_FAST_CONFIG_W8T("w8a16_tn_128x128x64_w2x2_s3_sk", 128, 128, 2, 2, 3, true),
+    IHP_FAST_CONFIG_W8T("w8a16_tn_64x128x64_w2x2_s4_sk", 64, 128, 2, 2, 4, true),
 };
 
 const FastConfig *fast_configs(int *count) {
@@ -1255,7 +1318,7 @@ const KernelEntry *gemm_kernels(int *count) {
       if (c.head)
         continue;  // a column split launches two listed kernels
       const uint32_t ex = c.elem == kElemI8 ? kExportMatmulI8
-                          : c.b_mode == kBW8
+                          : b_mode_w8(c.b_mode)
                               ? kExportW8A16
                               : kExportMatmulF16 | kExportBatchMatmulF16;
       v.push_back({c.name, c.kernel, c.threads, ex});

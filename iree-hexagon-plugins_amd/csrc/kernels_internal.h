@@ -17,7 +17,13 @@ enum BMode {
   kBNN16 = 1,  // B [K,N] f16
   kBW8 = 2,    // B [K,N] int8 with per-column f16 scale (W8A16)
   kBNN8 = 3,   // B [K,N] int8, int8 A (row-major int8 weights)
+  kBW8T = 4,   // B [N,K] int8 with per-column f16 scale (W8A16)
 };
+
+// int8 weights of an f16 product (W8A16), in either layout.
+constexpr bool b_mode_w8(int b_mode) {
+  return b_mode == kBW8 || b_mode == kBW8T;
+}
 
 // One matmul launch: C[M,N] = [C +] A[M,K] . B (B [K,N] or [N,K]).
 struct MatmulArgs {
@@ -133,7 +139,7 @@ struct FastConfig {
   int split_k;   // K split over grid.y, M may be ragged (skinny shapes)
   int a_trans;   // A stored [K,M] (f16 only, exact tiling)
   const void *kernel;  // the instantiated kernel (resource queries)
-  int elem;      // ElemKind of A (and of B unless kBW8)
+  int elem;      // ElemKind of A (and of B unless b_mode_w8)
   int out_f32;   // f16 path: f32 output (i8 path: always i32)
   int bm, bn;    // macro-tile
   int bk;        // K elements per LDS stage
@@ -142,7 +148,9 @@ struct FastConfig {
   int lds_bytes; // static LDS per workgroup
   FastLaunchFn launch;
   int mfma;      // MFMA shape: 32 (32x32) or 16 (16x16)
-  int table_only;  // chosen only by a measured planner entry, never ranked
+  // 1: not in the first ranking; chosen by a measured planner entry, or
+  // (kBW8T) against the general kernel by split_us
+  int table_only;
   // Column split (unsplit, batch 1): the configuration named `head` runs
   // over columns [0, n_head) in whole rounds of the chip's CUs, then `tail`
   // over [n_head, N) as a second grid on the same stream

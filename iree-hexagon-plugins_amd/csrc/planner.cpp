@@ -151,11 +151,11 @@ bool gemv_eligible(const iree_mi355x_matmul_desc_t &d) {
 int wanted_b_mode(const iree_mi355x_matmul_desc_t &d) {
   const bool bt = d.flags & IREE_MI355X_MATMUL_B_TRANSPOSED;
   if (d.has_scale)
-    return (!bt && d.a_elem == IREE_MI355X_ELEM_F16 &&
+    return (d.a_elem == IREE_MI355X_ELEM_F16 &&
             d.b_elem == IREE_MI355X_ELEM_I8 &&
             d.c_elem == IREE_MI355X_ELEM_F16 &&
             !(d.flags & IREE_MI355X_MATMUL_ACCUMULATE))
-               ? kBW8
+               ? (bt ? kBW8T : kBW8)
                : -1;
   if (d.a_elem != d.b_elem)
     return -1;
@@ -508,7 +508,15 @@ double split_us(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
       {"i8_tn_32x128x128_w1x4_s4_sk", 0.246, 0.309, 1.47},
       {"i8_tn_128x128x128_w2x2_s4_sk", 0.406, 0.242, 3.04},
       {"i8_nn_32x256x128_w1x4_s4_sk", 0.483, 0.0932, 1.17},
-      {"i8_nn_128x256x128_w2x4_s3_sk", 0.425, 0.638, 2.48}};
+      {"i8_nn_128x256x128_w2x4_s3_sk", 0.425, 0.638, 2.48},
+      // W8A16 [N,K], fitted to 1060 timings of 84 shapes (m 20..2048, n
+      // 512..11008, k 512..11008): the pick is 1.2 % slower than the best
+      // of these tiles on average.
+      {"w8a16_tn_256x256x64_w2x4_s3", 1.17, 1.17, 3.55},
+      {"w8a16_tn_128x256x64_w2x4_s4", 0.666, 0.657, 1.88},
+      {"w8a16_tn_128x256x64_w2x4_s4_sk", 0.703, 0.685, 3.21},
+      {"w8a16_tn_128x128x64_w2x2_s3_sk", 0.478, 0.507, 3.73},
+      {"w8a16_tn_64x128x64_w2x2_s4_sk", 0.317, 0.370, 2.50}};
   const Rates *r = nullptr;
   for (const Rates &x : kRates)
     if (strcmp(x.name, c.name) == 0)
@@ -701,6 +709,29 @@ void describe_general(const iree_mi355x_matmul_desc_t &d,
                                  bb * d.n * d.k * ((d.m + c.bm - 1) / c.bm));
 }
 
+// The plan fields of a macro-tile candidate.
+void describe_fast(const iree_mi355x_matmul_desc_t &d, const Candidate &best,
+                   iree_mi355x_matmul_plan_t *plan) {
+  int count = 0;
+  const FastConfig &c = fast_configs(&count)[best.index];
+  plan->config_index = best.index;
+  snprintf(plan->config_name, sizeof(plan->config_name), "%s", c.name);
+  plan->tile_m = c.bm;
+  plan->tile_n = c.bn;
+  plan->tile_k = c.bk;
+  plan->lds_bytes = c.lds_bytes;
+  plan->workgroups =
+      best.sk_steps > 0
+          ? best.sk_wgs
+          : best.tiles * best.splits * (d.batch > 0 ? d.batch : 1);
+  plan->threads = c.threads;
+  plan->splits = best.splits;
+  plan->k_split = best.k_split;
+  plan->stream_k_steps = best.sk_steps;
+  plan->workspace_bytes = best.workspace;
+  plan->traffic_bytes = best.traffic;
+}
+
 // Ranks the split-K configurations again by split_us where est_ns picked one,
 // and beyond 128 rows the general kernel with them, among the plans whose
 // workspace the caller has. Up to 128 rows a shape that est_ns splits stays
@@ -743,6 +774,41 @@ void refine_split(const iree_mi355x_matmul_desc_t &d, int64_t budget,
     return;
   const double t = general_plan_us(d, *general, cus);
   *use_general = t < 0.92 * t_best;
+}
+
+// W8A16 with weights [N,K]: the macro-tile (kBW8T) modeled fastest for the
+// call within its workspace, or false where the general kernel's plan is.
+// Measured (general / tile, us): 512 x 11008 x 4096 81.5 / 47.8, 777 x 4096 x
+// 4096 53.5 / 42.1, 2048 x 7168 x 1536 73.7 / 44.5; 128 x 4096 x 4096 stays
+// (16.7 / 20.3). Over the 32 of the 84 fitted shapes that take a tile 1.31x.
+bool plan_w8t(const iree_mi355x_matmul_desc_t &d, int64_t budget, int64_t cus,
+              size_t workspace_limit, const GeneralPlan &general,
+              Candidate *best) {
+  int count = 0;
+  const FastConfig *cfgs = fast_configs(&count);
+  double t_best = 0.95 * general_plan_us(d, general, cus);
+  bool found = false;
+  static const int kSplitChoices[] = {1, 2, 3, 4, 6, 8, 12};
+  for (int i = 0; i < count; ++i) {
+    if (cfgs[i].b_mode != kBW8T || cfgs[i].lds_bytes > budget)
+      continue;
+    for (int forced : kSplitChoices) {
+      Candidate c;
+      if ((forced > 1 && !cfgs[i].split_k) ||
+          !evaluate(d, cfgs[i], i, cus, &c, true, forced) ||
+          c.splits != forced ||
+          (c.splits > 1 && c.k_split < kMinStagesPerSplit * cfgs[i].bk) ||
+          (size_t)c.workspace > workspace_limit)
+        continue;
+      const double t = split_us(d, cfgs[i], c.tiles, c.splits, c.k_split, cus);
+      if (t > 0.0 && t < t_best) {
+        *best = c;
+        t_best = t;
+        found = true;
+      }
+    }
+  }
+  return found;
 }
 
 }  // namespace
@@ -902,36 +968,41 @@ int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
         return IREE_MI355X_OK;
       }
     }
-    const FastConfig &c = cfgs[best.index];
-    plan->config_index = best.index;
-    snprintf(plan->config_name, sizeof(plan->config_name), "%s", c.name);
-    plan->tile_m = c.bm;
-    plan->tile_n = c.bn;
-    plan->tile_k = c.bk;
-    plan->lds_bytes = c.lds_bytes;
-    plan->workgroups =
-        best.sk_steps > 0
-            ? best.sk_wgs
-            : best.tiles * best.splits * (d->batch > 0 ? d->batch : 1);
-    plan->threads = c.threads;
-    plan->splits = best.splits;
-    plan->k_split = best.k_split;
-    plan->stream_k_steps = best.sk_steps;
-    plan->workspace_bytes = (size_t)best.workspace > *required
-                                ? best.workspace
-                                : (int64_t)*required;
-    plan->traffic_bytes = best.traffic;
+    describe_fast(*d, best, plan);
+    if ((size_t)plan->workspace_bytes < *required)
+      plan->workspace_bytes = (int64_t)*required;
     return IREE_MI355X_OK;
   }
 
   GeneralPlan g;
   if (!plan_general_desc(*d, false, workspace_limit, &g))
     return IREE_MI355X_UNSUPPORTED;
+  Candidate best;
+  if (wanted_b_mode(*d) == kBW8T &&
+      plan_w8t(*d, budget, cus, workspace_limit, g, &best)) {
+    plan->family = IREE_MI355X_FAMILY_MFMA;
+    describe_fast(*d, best, plan);
+    return IREE_MI355X_OK;
+  }
   describe_general(*d, g, plan);
   return IREE_MI355X_OK;
 }
 
 }  // namespace ihp
+
+namespace {
+
+// Configurations callers may name: all but the W8A16 [N,K] tiles at the
+// table's end, which are the planner's own.
+int listed_configs() {
+  int count = 0;
+  const FastConfig *cfgs = fast_configs(&count);
+  while (count > 0 && cfgs[count - 1].b_mode == kBW8T)
+    --count;
+  return count;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -944,9 +1015,7 @@ int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
 }
 
 int iree_mi355x_mfma_config_count(void) {
-  int count = 0;
-  fast_configs(&count);
-  return count;
+  return listed_configs();
 }
 
 int iree_mi355x_mfma_config_info(int index, const char **name,
@@ -956,7 +1025,7 @@ int iree_mi355x_mfma_config_info(int index, const char **name,
                                  int64_t *lds_bytes, int32_t *threads) {
   int count = 0;
   const FastConfig *cfgs = fast_configs(&count);
-  if (index < 0 || index >= count)
+  if (index < 0 || index >= listed_configs())
     return IREE_MI355X_INVALID_ARGUMENT;
   const FastConfig &c = cfgs[index];
   if (name)
@@ -985,7 +1054,7 @@ int iree_mi355x_mfma_config_info(int index, const char **name,
 int32_t iree_mi355x_mfma_config_layout_flags(int index) {
   int count = 0;
   const FastConfig *cfgs = fast_configs(&count);
-  if (index < 0 || index >= count)
+  if (index < 0 || index >= listed_configs())
     return -1;
   return (int32_t)((cfgs[index].b_mode == kBTN
                         ? IREE_MI355X_MATMUL_B_TRANSPOSED
@@ -1006,20 +1075,20 @@ int config_candidate(int index, int32_t splits, const void *a, const void *b,
                      uint32_t flags, Candidate *out) {
   int count = 0;
   const FastConfig *cfgs = fast_configs(&count);
-  if (index < 0 || index >= count)
+  if (index < 0 || index >= listed_configs())
     return fail(IREE_MI355X_INVALID_ARGUMENT, "mfma_config: bad index %d",
                 index);
   const FastConfig &cfg = cfgs[index];
   const int32_t ae = cfg.elem == kElemI8 ? IREE_MI355X_ELEM_I8
                                          : IREE_MI355X_ELEM_F16;
-  const int32_t be = cfg.b_mode == kBW8 ? IREE_MI355X_ELEM_I8 : ae;
+  const int32_t be = b_mode_w8(cfg.b_mode) ? IREE_MI355X_ELEM_I8 : ae;
   const int32_t ce = cfg.elem == kElemI8
                          ? IREE_MI355X_ELEM_I32
                          : (cfg.out_f32 ? IREE_MI355X_ELEM_F32
                                         : IREE_MI355X_ELEM_F16);
   iree_mi355x_matmul_desc_t d;
   iree_mi355x_matmul_desc_init(&d, ae, be, ce, m, n, k, flags);
-  d.has_scale = cfg.b_mode == kBW8;
+  d.has_scale = b_mode_w8(cfg.b_mode);
   const int64_t aeb = elem_bytes(ae), beb = elem_bytes(be);
   d.a_aligned16 = a && fast_operand(a, lda * aeb);
   d.b_aligned16 = b && fast_operand(b, ldb * beb);

@@ -890,3 +890,23 @@ def test_general_split_fits_the_workspace_it_gets(pkg):
     for shape in ((65, 200, 7), (65, 7, 4100)):
         p = pkg.plan(pkg.make_desc(F16, F16, F16, *shape, 0))
         assert p.config_name == b"general_f16_any"
+
+
+def test_w8a16_row_major_weights_tiles(pkg):
+    """W8A16 with weights [N,K]: the tiles of this layout are planned where
+    they divide the shape, and are not among the configurations a caller
+    names."""
+    p = pkg.plan(pkg.make_desc(F16, I8, F16, 512, 11008, 4096,
+                               pkg.B_TRANSPOSED, has_scale=True))
+    assert p.family == pkg.FAMILY_MFMA
+    assert p.config_name == b"w8a16_tn_128x256x64_w2x4_s4"
+    assert p.workspace_bytes == 0
+    assert not any(c.name.startswith("w8a16_tn_") for c in pkg.mfma_configs())
+    for n, k in ((11008 + 8, 4096), (11008, 4096 + 8)):  # no tile divides
+        p = pkg.plan(pkg.make_desc(F16, I8, F16, 512, n, k, pkg.B_TRANSPOSED,
+                                   has_scale=True))
+        assert p.family == pkg.FAMILY_GENERAL
+    p = pkg.plan(pkg.make_desc(F16, I8, F16, 512, 11008, 4096,
+                               pkg.B_TRANSPOSED, has_scale=True,
+                               aligned=False))
+    assert p.family == pkg.FAMILY_GENERAL
