@@ -91,6 +91,9 @@ int32_t iree_mi355x_classify_matmul(const iree_mi355x_matmul_desc_t *desc);
 
 // Full plan: family, macro-tile, resources. Returns 0 (IREE_MI355X_OK) or
 // IREE_MI355X_UNSUPPORTED.
+// W8A16 of up to 16 rows with weights [N,K] is reported as the row-dot form
+// that such a call runs without a workspace; given one, a call of more rows
+// than one row-dot launch takes (or 5 to 7 on) runs on the general kernel.
 int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *desc,
                             iree_mi355x_matmul_plan_t *plan);
 

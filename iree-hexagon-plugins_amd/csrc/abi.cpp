@@ -314,7 +314,8 @@ size_t iree_mi355x_matmul_workspace_bytes(int64_t m, int64_t n, int64_t k,
       if (f == 1)
         d.flags |= IREE_MI355X_MATMUL_OUT_F32;
       iree_mi355x_matmul_plan_t p;
-      if (iree_mi355x_plan_matmul(&d, &p) == IREE_MI355X_OK &&
+      size_t required = 0;
+      if (plan_matmul(&d, (size_t)-1, &p, &required) == IREE_MI355X_OK &&
           (size_t)p.workspace_bytes > most)
         most = (size_t)p.workspace_bytes;
     }

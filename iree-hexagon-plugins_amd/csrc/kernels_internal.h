@@ -248,9 +248,9 @@ hipError_t launch_gemv(const MatmulArgs &a, int w_bytes, const void *scale,
 // counter) stays under 64 KiB; workgroups per launch (columns dealt in equal
 // runs, taken by the waves one at a time).
 constexpr int64_t kRowdotMaxXBytes = 60 * 1024;
-// W8A16 with W [N,K] and M <= this runs as row-dot launches of at most 8
-// rows of x each (each re-reads W): the MFMA tiles take int8 weights only as
-// [K,N], and the general kernel is several times slower.
+// W8A16 with W [N,K] and M <= this can run as row-dot launches of at most 8
+// rows of x each (each re-reads W); the planner's rowdot_gives_way has where
+// the general kernel is faster.
 constexpr int kRowdotMaxRowsW8A16 = 16;
 // Rows of x per W8A16 row-dot launch: as many as the LDS limit allows (at
 // most 8), dealt evenly over the launches M needs; 0 if one row of x does

@@ -776,6 +776,28 @@ void refine_split(const iree_mi355x_matmul_desc_t &d, int64_t budget,
   *use_general = t < 0.92 * t_best;
 }
 
+// W8A16 rows (M <= 16, weights [N,K]) that the general kernel's K splits
+// compute faster than the row-dot, where the workspace holds the splits it
+// would choose. The row-dot's time grows with every row and each of its
+// launches reads W again; the general kernel's is that of one 64-row tile.
+// Measured (row-dot / general, us) at N x K: M = 16 11008 x 4096 63.2 / 19.6,
+// 4096 x 11008 97.1 / 20.6, 2048 x 512 13.8 / 6.6; two launches at 3 rows
+// 4096 x 11008 22.7 / 20.5; one launch of 8 rows 1024 x 2048 9.0 / 7.8, of 6
+// 6.3 / 7.0 at 1000 x 1008 but 23.1 / 19.5 at 11008 x 4096, of 4 19.0 / 20.0.
+bool rowdot_gives_way(const iree_mi355x_matmul_desc_t &d,
+                      size_t workspace_limit, GeneralPlan *plan) {
+  if (!d.has_scale || !(d.flags & IREE_MI355X_MATMUL_B_TRANSPOSED) ||
+      !types_supported(d) || !gemv_eligible(d))
+    return false;
+  const bool one_launch = rowdot_w8a16_rows(d.m, d.k) >= d.m;
+  if (one_launch && d.m < (d.n * d.k >= (10 << 20) ? 5 : 7))
+    return false;
+  GeneralPlan most;
+  return plan_general_desc(d, false, workspace_limit, plan) &&
+         plan_general_desc(d, false, (size_t)-1, &most) &&
+         plan->splits == most.splits;
+}
+
 // W8A16 with weights [N,K]: the macro-tile (kBW8T) modeled fastest for the
 // call within its workspace, or false where the general kernel's plan is.
 // Measured (general / tile, us): 512 x 11008 x 4096 81.5 / 47.8, 777 x 4096 x
@@ -815,12 +837,30 @@ bool plan_w8t(const iree_mi355x_matmul_desc_t &d, int64_t budget, int64_t cus,
 
 namespace ihp {
 
+int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
+                     size_t workspace_limit, iree_mi355x_matmul_plan_t *plan,
+                     size_t *required);
+
 // The plan of a call with `workspace_limit` bytes of workspace, and the
 // workspace below which the call is refused: what the plan of the first
 // ranking needs, whether or not the refined one needs it (the plan's
 // workspace_bytes is the larger of the two).
 int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
                 iree_mi355x_matmul_plan_t *plan, size_t *required) {
+  GeneralPlan tile;
+  if (rowdot_gives_way(*d, workspace_limit, &tile)) {
+    *required = 0;
+    memset(plan, 0, sizeof(*plan));
+    describe_general(*d, tile, plan);
+    return IREE_MI355X_OK;
+  }
+  return plan_matmul_rows(d, workspace_limit, plan, required);
+}
+
+// plan_matmul with every shape the row-dot takes on the row-dot.
+int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
+                     size_t workspace_limit, iree_mi355x_matmul_plan_t *plan,
+                     size_t *required) {
   *required = 0;
   memset(plan, 0, sizeof(*plan));
   plan->config_index = -1;
@@ -1011,7 +1051,7 @@ int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
   if (!d || !plan)
     return IREE_MI355X_INVALID_ARGUMENT;
   size_t required = 0;
-  return plan_matmul(d, (size_t)-1, plan, &required);
+  return plan_matmul_rows(d, (size_t)-1, plan, &required);
 }
 
 int iree_mi355x_mfma_config_count(void) {

@@ -892,10 +892,13 @@ def test_general_split_fits_the_workspace_it_gets(pkg):
         assert p.config_name == b"general_f16_any"
 
 
-def test_w8a16_row_major_weights_tiles(pkg):
-    """W8A16 with weights [N,K]: the tiles of this layout are planned where
-    they divide the shape, and are not among the configurations a caller
-    names."""
+def test_w8a16_row_major_weights_workspace(pkg):
+    """W8A16 with weights [N,K]: rows past one row-dot launch may split K, so
+    the query covers that, and a call without a workspace is never refused a
+    plan (the row-dot or an unsplit tile); the tiles of this layout are not
+    among the configurations a caller names."""
+    q = pkg.library().iree_mi355x_matmul_workspace_bytes
+    assert q(16, 11008, 4096, pkg.B_TRANSPOSED) > 0
     p = pkg.plan(pkg.make_desc(F16, I8, F16, 512, 11008, 4096,
                                pkg.B_TRANSPOSED, has_scale=True))
     assert p.family == pkg.FAMILY_MFMA

@@ -81,6 +81,8 @@ def run_without_workspace(pkg, x, w, scale, c):
 
 @pytest.mark.parametrize("m,n,k", [
     (600, 4096, 11008),  # split with a workspace
+    (5, 4096, 4096), (7, 1000, 1008), (16, 4096, 4096),  # row-dot or general
+    (3, 300, 11008), (8, 128, 128),
 ])
 def test_with_and_without_workspace(pkg, dev, m, n, k):
     print(m, n, k, flush=True)
