@@ -180,12 +180,13 @@ struct Ready {
 };
 
 // Resolve and validate every command; the largest workspace any dispatch
-// asks for, of the `workspace_limit` bytes it may have, goes to
-// *max_workspace. Enqueues nothing.
+// cannot run without goes to *max_workspace. That alone sizes a slice, at
+// every concurrency: a slice that grew with what a submission has would put
+// one lane's partial tiles over another's counters on a workspace that
+// serves both. Enqueues nothing.
 int prepare(const iree_mi355x_command_buffer_t *cb,
             const iree_mi355x_binding_t *table, uint32_t count,
-            size_t workspace_limit, std::vector<Ready> *out,
-            size_t *max_workspace) {
+            std::vector<Ready> *out, size_t *max_workspace) {
   *max_workspace = 0;
   out->assign(cb->commands.size(), Ready());
   const iree_mi355x_executable_export_table_t &ex = cb->library->exports;
@@ -213,7 +214,6 @@ int prepare(const iree_mi355x_command_buffer_t *cb,
         s.binding_count = (uint32_t)r.ptrs.size();
         s.binding_ptrs = r.ptrs.data();
         s.binding_lengths = r.lengths.data();
-        s.workspace_bytes = workspace_limit;
         s.workspace_query = &need;
         if ((st = ex.ptrs[c.ordinal](nullptr, &s))) {
           const std::string why = iree_mi355x_last_error();
@@ -578,12 +578,10 @@ size_t iree_mi355x_command_buffer_workspace_bytes(
     return 0;
   const uint32_t lanes = lanes_for(
       cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
-  // In order, one buffer serves every dispatch: ask for all that their plans
-  // can use. Lanes take slices, sized by what the plans require only.
   std::vector<Ready> ready;
   size_t need = 0;
-  if (prepare(cb, binding_table, binding_count, lanes == 1 ? SIZE_MAX : 0,
-              &ready, &need) != IREE_MI355X_OK)
+  if (prepare(cb, binding_table, binding_count, &ready, &need) !=
+      IREE_MI355X_OK)
     return 0;
   return need ? slice_bytes(need) * lanes : 0;
 }
@@ -606,9 +604,7 @@ int iree_mi355x_command_buffer_submit(
       cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
   std::vector<Ready> ready;
   size_t need = 0;
-  int st = prepare(cb, binding_table, binding_count,
-                   lanes == 1 && workspace ? workspace_bytes : 0, &ready,
-                   &need);
+  int st = prepare(cb, binding_table, binding_count, &ready, &need);
   if (st)
     return st;
   if (cb->commands.empty())
@@ -634,11 +630,10 @@ int iree_mi355x_command_buffer_submit(
   const uint32_t n = (uint32_t)cb->commands.size();
 
   if (lanes == 1) {
-    // In order on the caller's stream: barriers hold by stream order, and
-    // every dispatch may use the whole workspace.
+    // In order on the caller's stream: barriers hold by stream order. One
+    // slice, as lane 0 has it: what follows holds other lanes' counters.
     for (uint32_t i = 0; i < n && !st; ++i)
-      st = enqueue(cb, i, ready[i], caller, slice ? ws : nullptr,
-                   slice ? workspace_bytes : 0);
+      st = enqueue(cb, i, ready[i], caller, slice ? ws : nullptr, slice);
     roctxRangePop();
     return st;
   }

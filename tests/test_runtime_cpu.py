@@ -134,6 +134,36 @@ def test_workspace_sizing(pkg):
                                (FAKE * 4, 2048 * 4096 * 2)], 4) == 0
 
 
+def dispatches(pkg, *calls):
+    """A command buffer of the matmul_f16 shapes and its fake table."""
+    cb, table = pkg.CommandBuffer(), []
+    for i, (m, n, k) in enumerate(calls):
+        cb.dispatch("matmul_f16", matmul_consts(pkg, m, n, k),
+                    [pkg.slot(3 * i + j) for j in range(3)])
+        base = FAKE * (1 + i) << 14
+        table += [(base, m * k * 2), (base + (1 << 28), k * n * 2),
+                  (base + (2 << 28), m * n * 2)]
+    return cb.end(), table
+
+
+@pytest.mark.parametrize("calls", [
+    [(150, 256, 2048)] * 2,                  # a split re-ranked by its time
+    [(1, 4096, 4096), (777, 3001, 4099)],    # a GEMV beside a general matmul
+    [(16, 4096, 4096), (300, 11008, 4096), (33, 130, 2050)],
+    [(777, 3001, 4099)] * 3,                 # nothing that needs a workspace
+])
+def test_one_slice_size_at_every_concurrency(pkg, calls):
+    """The slice is the query at concurrency 1, whatever the concurrency: a
+    workspace that serves submissions of one slice size has every lane's
+    counters at the same place."""
+    cb, table = dispatches(pkg, *calls)
+    one = cb.workspace_bytes(table, 1)
+    for lanes in range(2, len(calls) + 1):
+        assert cb.workspace_bytes(table, lanes) == lanes * one
+    # a general matmul runs without one
+    assert (one == 0) == all(c == (777, 3001, 4099) for c in calls)
+
+
 def test_workspace_query_through_export(pkg):
     """An export called with a workspace query validates and plans only."""
     st, need = pkg.call_export(

@@ -130,6 +130,40 @@ def test_program_caller_workspace(pkg, oracle, dev):
     assert int(ws[:64 * 1024].count_nonzero()) == 0   # lane 0's counters re-armed
 
 
+@pytest.mark.parametrize("calls", [
+    [(150, 256, 2048)] * 2, [(1, 4096, 4096), (777, 3001, 4099)]])
+def test_lanes_and_in_order_on_one_workspace(pkg, oracle, dev, calls):
+    """One command buffer with lanes, in order, then with lanes again on one
+    caller workspace: an in-order submission stays within lane 0's slice, so
+    the other lanes find their counters zero."""
+    g = torch.Generator().manual_seed(17)
+    cb, table, outs, refs = pkg.CommandBuffer(), [], [], []
+    for i, (m, n, k) in enumerate(calls):
+        a = (torch.randn(m, k, generator=g) * 0.5).half()
+        b = (torch.randn(k, n, generator=g) * 0.05).half()
+        outs.append(torch.empty(m, n, dtype=torch.float16, device=dev))
+        refs.append(oracle.matmul_f16(a.numpy(), b.numpy()))
+        table += [a.to(dev), b.to(dev), outs[-1]]
+        cb.dispatch("matmul_f16", consts(pkg, m, n, k),
+                    [pkg.slot(3 * i + j) for j in range(3)])
+    cb.end()
+    slice_ = cb.workspace_bytes(table, 1)
+    # more than the lanes take: none of it is an in-order submission's
+    ws = torch.zeros(cb.workspace_bytes(table, 2) + (64 << 20),
+                     dtype=torch.uint8, device=dev)
+    for lanes in (2, 1, 2, 1):
+        print(f"lanes {lanes} {calls}", flush=True)
+        for o in outs:
+            o.fill_(9.0)
+        before = ws[slice_:].clone()
+        cb.submit(table, max_concurrent=lanes, workspace=ws)
+        torch.cuda.synchronize()
+        for o, ref in zip(outs, refs):
+            assert oracle.fp16_parity(o.cpu().numpy(), ref) <= FP16_BOUND
+        if lanes == 1:
+            assert torch.equal(ws[slice_:], before)
+
+
 def test_failed_validation_enqueues_nothing(pkg, dev):
     m, n, k = 128, 512, 256
     a = torch.randn(m, k, device=dev).half()
