@@ -1277,19 +1277,21 @@ class CommandBuffer:
         return [(o.kind, o.lane, o.event, o.command) for o in ops[:n]]
 
     def submit(self, table=(), max_concurrent=0, workspace=None, stream=None):
-        """Submit on `stream`; without a `workspace` the lane slices come
-        from the wrapper's workspace of that stream for this slice size
-        (lane l's counters sit at l slices: a buffer serves one slice size)."""
+        """Submit on `stream`; without a `workspace`, in order on the
+        wrapper's flat workspace of that stream, and with lanes on its
+        workspace for this slice size (lane l's counters sit at l slices: a
+        buffer serves one slice size)."""
         arr, n = binding_table(list(table))
         s = _stream_ptr(stream)
         if workspace is None:
-            need = slice_ = \
-                self._lib.iree_mi355x_command_buffer_workspace_bytes(
-                    self._h, arr, n, max_concurrent)
+            need = self._lib.iree_mi355x_command_buffer_workspace_bytes(
+                self._h, arr, n, max_concurrent)
+            slice_ = need
             if need and max_concurrent > 1:
-                slice_ //= 1 + max(
-                    op[1] for op in self.lane_schedule(max_concurrent))
-            ws, wsb = stream_workspace(need, None, s, ("lanes", slice_))
+                slice_ = self._lib.iree_mi355x_command_buffer_workspace_bytes(
+                    self._h, arr, n, 1)
+            ws, wsb = stream_workspace(
+                need, None, s, None if need == slice_ else ("lanes", slice_))
         else:
             ws, wsb = _ptr_len(workspace)
         _check(self._lib.iree_mi355x_command_buffer_submit(

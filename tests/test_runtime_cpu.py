@@ -164,6 +164,29 @@ def test_one_slice_size_at_every_concurrency(pkg, calls):
     assert (one == 0) == all(c == (777, 3001, 4099) for c in calls)
 
 
+def test_in_order_submissions_take_the_flat_workspace(pkg, monkeypatch):
+    """In order the counters open the workspace, as a flat call's do: every
+    such submission of a stream takes the stream's one flat buffer. Lanes
+    have one per slice size."""
+    class Asked(Exception):
+        pass
+
+    def ask(need, device=None, stream=None, layout=None, partial=False):
+        raise Asked(need, layout, partial)
+
+    monkeypatch.setattr(pkg, "stream_workspace", ask)
+    sizes = [(16, 4096, 4096), (16, 4096, 2048), (1, 4096, 4096)]
+    for shape in sizes:
+        cb, table = dispatches(pkg, shape, shape)
+        one = cb.workspace_bytes(table, 1)
+        assert one > 0
+        for lanes in (0, 1, 2):
+            with pytest.raises(Asked) as e:
+                cb.submit(table, max_concurrent=lanes, stream=0)
+            assert e.value.args == ((2 * one, ("lanes", one), False)
+                                    if lanes == 2 else (one, None, False))
+
+
 def test_workspace_query_through_export(pkg):
     """An export called with a workspace query validates and plans only."""
     st, need = pkg.call_export(

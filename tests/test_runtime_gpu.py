@@ -300,6 +300,47 @@ def test_captured_in_order_submission_replays(pkg, oracle, dev):
         p.check(oracle)
 
 
+def test_captured_submission_without_a_workspace(pkg, oracle, dev):
+    """A general matmul and one query against 4000 keys need no workspace in
+    a command buffer: captured on a stream that has none, every replay
+    matches."""
+    import struct
+    g = torch.Generator().manual_seed(33)
+    m, n, k, h, skv, d = 33, 130, 2050, 8, 4000, 128
+    a, b = torch.randn(m, k, generator=g).half(), torch.randn(k, n, generator=g).half()
+    q = torch.randn(1, h, 1, d, generator=g).half()
+    kk, v = (torch.randn(1, h, skv, d, generator=g).half() for _ in range(2))
+    c = torch.zeros(m, n, dtype=torch.float16, device=dev)
+    o = torch.zeros(1, h, 1, d, dtype=torch.float16, device=dev)
+    scale = d ** -0.5
+    cb = pkg.CommandBuffer()
+    cb.dispatch("matmul_f16", consts(pkg, m, n, k),
+                [pkg.slot(0), pkg.slot(1), pkg.slot(2)])
+    cb.dispatch("attention_f16",
+                [1, h, 1, skv, d,
+                 struct.unpack("<I", struct.pack("<f", scale))[0], 0],
+                [pkg.slot(3), pkg.slot(4), pkg.slot(5), pkg.slot(6)])
+    cb.end()
+    table = [t.to(dev) for t in (a, b)] + [c] + [
+        t.to(dev) for t in (q, kk, v)] + [o]
+    assert cb.workspace_bytes(table, 1) == 0
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        cb.submit(table, max_concurrent=1)
+    ref_c = oracle.matmul_f16(a.numpy(), b.numpy())
+    ref_o = oracle.attention_f16(q.numpy(), kk.numpy(), v.numpy(), scale=scale,
+                                 causal=False)
+    for _ in range(3):
+        c.zero_(), o.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert oracle.fp16_parity(c.cpu().numpy(), ref_c) <= FP16_BOUND
+        assert oracle.fp16_parity(o.cpu().numpy(), ref_o) <= FP16_BOUND
+
+
 def test_loaded_executable_dispatches(pkg, oracle, dev):
     """A serialized executable loaded into a private copy of the library:
     its exports run a macro-tile and a split-K matmul through a command
