@@ -309,6 +309,8 @@ def library():
     lib.iree_mi355x_batch_matmul_workspace_bytes.argtypes = [i64, i64, i64,
                                                              i64, u32]
     lib.iree_mi355x_last_error.restype = ctypes.c_char_p
+    # the HIP runtime's, through the library that links it
+    lib.hipStreamIsCapturing.argtypes = [p, p]
     lib.iree_mi355x_version.restype = ctypes.c_char_p
     lib.iree_mi355x_matmul_desc_init.restype = None
     lib.iree_mi355x_matmul_desc_init.argtypes = [
@@ -705,7 +707,8 @@ def stream_workspace(need: int, device=None, stream=None, layout=None,
     have = bufs[-1].numel() if bufs else 0
     if have >= need:
         return bufs[-1].data_ptr(), have
-    if torch.cuda.is_current_stream_capturing():
+    if (torch.cuda.is_current_stream_capturing()
+            or (s.cuda_stream and _capturing(s.cuda_stream))):
         if partial:
             return (bufs[-1].data_ptr(), have) if bufs else (None, 0)
         raise MI355XError(
@@ -722,16 +725,37 @@ def stream_workspace(need: int, device=None, stream=None, layout=None,
     return buf.data_ptr(), size
 
 
+def _capturing(stream) -> bool:
+    """Whether a raw stream, not the null stream, is capturing."""
+    status = ctypes.c_int()
+    library().hipStreamIsCapturing(stream, ctypes.byref(status))
+    return status.value != 0
+
+
 def _call_workspace(need, index, stream):
-    """stream_workspace of a flat call on device `index` and a raw stream."""
-    if need <= 0:
+    """stream_workspace of a flat call on device `index` and a raw stream,
+    (None, 0) under capture: graphs captured on one stream may replay on
+    several at a time, so what runs without a workspace keeps nothing in the
+    stream's. (The null stream cannot be captured.)"""
+    if need <= 0 or (stream and _capturing(stream)):
         return None, 0
     have = _FLAT_WORKSPACES.get((index, stream))
     if have is not None and have[1] >= need:
         return have
     import torch
-    return stream_workspace(need, torch.device("cuda", index), stream,
-                            partial=True)
+    return stream_workspace(need, torch.device("cuda", index), stream)
+
+
+def _call(fn, args, need, index, stream):
+    """One flat call of the library with what it can use of the stream's
+    workspace; a captured one that cannot run without gets what there is."""
+    st = fn(*args, *_call_workspace(need, index, stream), stream)
+    if st == WORKSPACE_TOO_SMALL and need > 0:
+        import torch
+        st = fn(*args, *stream_workspace(
+            need, torch.device("cuda", index), stream, partial=True), stream)
+    if st != OK:
+        _check(st)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -849,18 +873,11 @@ def matmul(a, b, c=None, *, b_transposed=False, accumulate=False,
     s = _stream_ptr(stream)
     if a.dtype != torch.int8 and out_dtype == torch.float32:
         flags |= OUT_F32
-    ws, wsb = _call_workspace(_matmul_workspace_need(m, n, k, flags),
-                              a.get_device(), s)
-    if a.dtype == torch.int8:
-        _check(lib.iree_mi355x_matmul_i8(a.data_ptr(), b.data_ptr(),
-                                         c.data_ptr(), m, n, k, a.stride(0),
-                                         b.stride(0), c.stride(0), flags, ws,
-                                         wsb, s))
-    else:
-        _check(lib.iree_mi355x_matmul_f16(a.data_ptr(), b.data_ptr(),
-                                          c.data_ptr(), m, n, k, a.stride(0),
-                                          b.stride(0), c.stride(0), flags,
-                                          ws, wsb, s))
+    _call(lib.iree_mi355x_matmul_i8 if a.dtype == torch.int8
+          else lib.iree_mi355x_matmul_f16,
+          (a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k, a.stride(0),
+           b.stride(0), c.stride(0), flags),
+          _matmul_workspace_need(m, n, k, flags), a.get_device(), s)
     return c
 
 
@@ -950,12 +967,11 @@ def batch_matmul(a, b, c=None, *, b_transposed=False, accumulate=False,
              (OUT_F32 if out_dtype == torch.float32 else 0) |
              (A_TRANSPOSED if a_transposed else 0))
     st = _stream_ptr(stream)
-    ws, wsb = _call_workspace(_batch_workspace_need(batch, m, n, k, flags),
-                              a.get_device(), st)
-    _check(lib.iree_mi355x_batch_matmul_f16(
-        a3.data_ptr(), b3.data_ptr(), c3.data_ptr(), batch, m, n, k,
-        a3.stride(1), b3.stride(1), c3.stride(1), sa, sb, sc, flags,
-        ctypes.byref(e) if e is not None else None, ws, wsb, st))
+    _call(lib.iree_mi355x_batch_matmul_f16,
+          (a3.data_ptr(), b3.data_ptr(), c3.data_ptr(), batch, m, n, k,
+           a3.stride(1), b3.stride(1), c3.stride(1), sa, sb, sc, flags,
+           ctypes.byref(e) if e is not None else None),
+          _batch_workspace_need(batch, m, n, k, flags), a.get_device(), st)
     return c
 
 
@@ -991,11 +1007,10 @@ def quantized_matmul(x, w, scale, y=None, *, w_transposed=False, stream=None):
         y = torch.empty((m, n), dtype=torch.float16, device=x.device)
     flags = B_TRANSPOSED if w_transposed else 0
     st = _stream_ptr(stream)
-    ws, wsb = _call_workspace(_matmul_workspace_need(m, n, k, flags),
-                              x.get_device(), st)
-    _check(lib.iree_mi355x_w8a16_matmul(
-        x.data_ptr(), w.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k,
-        x.stride(0), w.stride(0), y.stride(0), flags, ws, wsb, st))
+    _call(lib.iree_mi355x_w8a16_matmul,
+          (x.data_ptr(), w.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n,
+           k, x.stride(0), w.stride(0), y.stride(0), flags),
+          _matmul_workspace_need(m, n, k, flags), x.get_device(), st)
     return y
 
 
@@ -1117,8 +1132,8 @@ def attention(q, k, v, o=None, *, causal=True, scale=None, mask=None,
                                                      mask.stride())
     args = _ATTENTION_ARGS.pack(qp, kp, vp, op, mp, b, h, hkv, sq, skv, d, dv,
                                 scale, flags, *st, *ms)
-    ws, wsb = _call_workspace(need, q.get_device(), stp)
-    _check(lib.iree_mi355x_attention_with_workspace(args, ws, wsb, stp))
+    _call(lib.iree_mi355x_attention_with_workspace, (args,), need,
+          q.get_device(), stp)
     return o
 
 

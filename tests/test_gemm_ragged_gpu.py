@@ -219,3 +219,49 @@ def test_general_under_capture(pkg, oracle, dev):
         ref = oracle.matmul_f16(a.numpy(), b.numpy())
         assert oracle.fp16_parity(c.cpu().numpy(), ref) <= 2e-3
     assert oracle.fp16_parity(eager.cpu().numpy(), ref) <= 2e-3
+
+
+@pytest.mark.parametrize("op", ["matmul", "attention"])
+def test_captured_calls_leave_the_stream_workspace_alone(pkg, dev, op):
+    """Captured on a stream whose workspace a warm-up call has filled: the
+    graph runs without it, so it may replay beside other work. Its counters
+    are spoilt before the replays, which a call that counts on them would
+    not survive."""
+    g = torch.Generator().manual_seed(6)
+    if op == "matmul":
+        a, b = (torch.randn(*s, generator=g).half().to(dev)
+                for s in ((33, 2050), (2050, 130)))
+        c = torch.zeros(33, 130, dtype=torch.float16, device=dev)
+
+        def call():
+            pkg.matmul(a, b, c)
+    else:
+        q, k, v = (torch.randn(*s, generator=g).half().to(dev)
+                   for s in ((2, 8, 1, 64), (2, 2, 3000, 64), (2, 2, 3000, 64)))
+        c = torch.zeros(2, 8, 1, 64, dtype=torch.float16, device=dev)
+
+        def call():
+            pkg.attention(q, k, v, c, causal=False)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        call()
+    torch.cuda.synchronize()
+    want = c.float()
+    ws, size = pkg._FLAT_WORKSPACES[dev.index or 0, s.cuda_stream]
+    buf = pkg._STREAM_WORKSPACES[dev.index or 0, s.cuda_stream, None][-1]
+    assert buf.data_ptr() == ws and size == buf.numel()
+    assert int(buf[256 << 10:].count_nonzero()) > 0  # the warm-up split
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        call()
+    buf[:256 << 10].fill_(1)
+    for _ in range(3):
+        c.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((c.float() - want).abs().max() / want.abs().max()) < 2e-3
+    assert bool((buf[:256 << 10] == 1).all())
+    buf[:256 << 10].zero_()
+    torch.cuda.synchronize()

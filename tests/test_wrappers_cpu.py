@@ -133,3 +133,32 @@ def test_mfma_config_operands(pkg):
                                z(128, 256))
     with pytest.raises(TypeError, match="device"):
         pkg.matmul_mfma_config(tn.index, a, bt, z(128, 128))
+
+
+def test_captured_calls_take_a_workspace_only_if_they_must(pkg, monkeypatch):
+    """A call that runs without a workspace keeps no state in its stream's:
+    graphs captured on one stream may replay on several. One that the
+    library refuses without gets it."""
+    monkeypatch.setattr(pkg, "_FLAT_WORKSPACES", {(0, 7): (4096, 1 << 20)})
+    monkeypatch.setattr(pkg, "_capturing", lambda stream: False)
+    assert pkg._call_workspace(512, 0, 7) == (4096, 1 << 20)
+    monkeypatch.setattr(pkg, "_capturing", lambda stream: True)
+    assert pkg._call_workspace(512, 0, 7) == (None, 0)
+    # the null stream cannot be captured
+    monkeypatch.setattr(pkg, "_FLAT_WORKSPACES", {(0, 0): (4096, 1 << 20)})
+    assert pkg._call_workspace(512, 0, 0) == (4096, 1 << 20)
+
+    calls = []
+
+    def fn(a, b, ws, wsb, stream):
+        calls.append((a, b, ws, wsb, stream))
+        return pkg.OK if ws else pkg.WORKSPACE_TOO_SMALL
+
+    monkeypatch.setattr(pkg, "stream_workspace",
+                        lambda need, device, stream, **kw: (4096, 1 << 20))
+    pkg._call(fn, (1, 2), 512, 0, 7)
+    assert calls == [(1, 2, None, 0, 7), (1, 2, 4096, 1 << 20, 7)]
+    with pytest.raises(pkg.MI355XError):
+        pkg._call(lambda *a: pkg.WORKSPACE_TOO_SMALL, (1, 2), 512, 0, 7)
+    with pytest.raises(pkg.MI355XError):
+        pkg._call(lambda *a: pkg.MISALIGNED, (1, 2), 0, 0, 7)
