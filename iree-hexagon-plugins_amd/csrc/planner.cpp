@@ -843,8 +843,8 @@ int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
 
 // The plan of a call with `workspace_limit` bytes of workspace, and the
 // workspace below which the call is refused: what the plan of the first
-// ranking needs, whether or not the refined one needs it (the plan's
-// workspace_bytes is the larger of the two).
+// ranking needs, or less where the refined plan of a call with any workspace
+// uses less. (The workspace_bytes of a refused call's plan are these.)
 int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
                 iree_mi355x_matmul_plan_t *plan, size_t *required) {
   GeneralPlan tile;
@@ -996,20 +996,29 @@ int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
     }
     if (best.index < 0)
       return IREE_MI355X_UNSUPPORTED;
-    *required = best.workspace > 0 ? (size_t)best.workspace : 0;
-    if (!plan->from_tuned_table && cfgs[best.index].split_k) {
-      GeneralPlan g;
-      bool use_general = false;
+    const Candidate first = best;
+    bool use_general = false;
+    GeneralPlan g;
+    *required = (size_t)first.workspace;
+    if (!plan->from_tuned_table && cfgs[first.index].split_k) {
       refine_split(*d, budget, cus, workspace_limit, &best, &g, &use_general);
-      if (use_general) {
-        describe_general(*d, g, plan);
-        if ((size_t)plan->workspace_bytes < *required)
-          plan->workspace_bytes = (int64_t)*required;
-        return IREE_MI355X_OK;
+      if (*required > workspace_limit) {
+        // Refused, unless the plan of a call with any workspace is content
+        // with this one.
+        Candidate c = first;
+        GeneralPlan gc;
+        bool general = false;
+        refine_split(*d, budget, cus, (size_t)-1, &c, &gc, &general);
+        const size_t uses = (size_t)(general ? gc.workspace : c.workspace);
+        if (uses < *required)
+          *required = uses;
       }
     }
-    describe_fast(*d, best, plan);
-    if ((size_t)plan->workspace_bytes < *required)
+    if (use_general)
+      describe_general(*d, g, plan);
+    else
+      describe_fast(*d, best, plan);
+    if (*required > workspace_limit)
       plan->workspace_bytes = (int64_t)*required;
     return IREE_MI355X_OK;
   }

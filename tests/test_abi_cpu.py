@@ -913,3 +913,32 @@ def test_w8a16_row_major_weights_workspace(pkg):
                                pkg.B_TRANSPOSED, has_scale=True,
                                aligned=False))
     assert p.family == pkg.FAMILY_GENERAL
+
+
+def workspace_floor(pkg, m, n, k, flags=0):
+    """What a matmul_f16 call of this shape cannot run without: its export's
+    workspace query with no workspace given."""
+    ldb = k if flags & pkg.B_TRANSPOSED else n
+    st, need = pkg.call_export(
+        "matmul_f16", pkg.matmul_constants(m, n, k, k, ldb, n, flags),
+        [1 << 40, 2 << 40, 3 << 40], [m * k * 2, k * n * 2, m * n * 2],
+        stream=0, query=True)
+    assert st == pkg.OK, pkg.last_error()
+    return need
+
+
+def test_a_plan_asks_for_the_workspace_it_uses(pkg):
+    """A plan that does not split K has no workspace, and no call is refused
+    for more than its plan uses."""
+    split = 0
+    for n, k in ((11008, 4096), (4096, 11008), (4096, 4096), (1024, 2048)):
+        for flags in (0, pkg.B_TRANSPOSED):
+            for m in (130, 150, 192, 257, 300, 384, 500, 777, 1000, 2000):
+                p = pkg.plan(pkg.make_desc(F16, F16, F16, m, n, k, flags))
+                assert (p.workspace_bytes > 0) == (p.splits > 1), (m, n, k)
+                assert workspace_floor(pkg, m, n, k, flags) <= p.workspace_bytes
+                split += p.splits > 1
+    assert split > 10
+    assert workspace_floor(pkg, 300, 11008, 4096, pkg.B_TRANSPOSED) == 0
+    # a few rows split K or are refused
+    assert workspace_floor(pkg, 16, 4096, 4096) > 0
