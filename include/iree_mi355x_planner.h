@@ -39,7 +39,8 @@ typedef enum iree_mi355x_family_e {
   IREE_MI355X_FAMILY_NONE = 0,     // not a dispatch this library takes
   IREE_MI355X_FAMILY_MFMA = 1,     // LDS-DMA MFMA macro-tile kernel
   IREE_MI355X_FAMILY_GENERAL = 2,  // bounds-checked MFMA kernel, any shape
-  IREE_MI355X_FAMILY_GEMV = 3,     // HBM-streaming skinny kernel (M <= 4)
+  IREE_MI355X_FAMILY_GEMV = 3,     // HBM-streaming skinny kernel (M <= 4;
+                                   // W8A16 with weights [N,K]: <= 16)
 } iree_mi355x_family_t;
 
 typedef struct iree_mi355x_matmul_desc_t {
@@ -86,16 +87,22 @@ void iree_mi355x_matmul_desc_init(iree_mi355x_matmul_desc_t *desc,
                                   int64_t k, uint32_t flags);
 
 // Which kernel family takes the dispatch (FAMILY_NONE for element types no
-// kernel computes). Mirrors the HMX eligibility rules, see above.
+// kernel computes): the family of iree_mi355x_plan_matmul's plan. Mirrors the
+// HMX eligibility rules, see above.
 int32_t iree_mi355x_classify_matmul(const iree_mi355x_matmul_desc_t *desc);
 
-// Full plan: family, macro-tile, resources. Returns 0 (IREE_MI355X_OK) or
-// IREE_MI355X_UNSUPPORTED.
-// W8A16 of up to 16 rows with weights [N,K] is reported as the row-dot form
-// that such a call runs without a workspace; given one, a call of more rows
-// than one row-dot launch takes (or 5 to 7 on) runs on the general kernel.
+// Full plan: family, macro-tile, resources, of a call with all the workspace
+// that it can use. Returns 0 (IREE_MI355X_OK) or IREE_MI355X_UNSUPPORTED.
 int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *desc,
                             iree_mi355x_matmul_plan_t *plan);
+
+// The plan of a call with `workspace_bytes` of workspace (0: none), where
+// another one is run in less: K split less, or the row-dot form for W8A16
+// rows with weights [N,K]. A call is refused
+// (IREE_MI355X_WORKSPACE_TOO_SMALL) if its plan's workspace_bytes is more.
+int iree_mi355x_plan_matmul_within(const iree_mi355x_matmul_desc_t *desc,
+                                   size_t workspace_bytes,
+                                   iree_mi355x_matmul_plan_t *plan);
 
 // B operand forms of the MFMA family.
 typedef enum iree_mi355x_b_form_e {

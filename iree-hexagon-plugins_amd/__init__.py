@@ -63,7 +63,8 @@ EXPORTED_SYMBOLS = (
     "iree_mi355x_matmul_workspace_bytes", "iree_mi355x_last_error",
     "iree_mi355x_version", "iree_mi355x_device_count",
     "iree_mi355x_matmul_desc_init", "iree_mi355x_classify_matmul",
-    "iree_mi355x_plan_matmul", "iree_mi355x_mfma_config_count",
+    "iree_mi355x_plan_matmul", "iree_mi355x_plan_matmul_within",
+    "iree_mi355x_mfma_config_count",
     "iree_mi355x_mfma_config_info", "iree_mi355x_matmul_mfma_config",
     "iree_mi355x_executable_library_query", "iree_mi355x_batch_matmul_f16",
     "iree_mi355x_batch_matmul_workspace_bytes",
@@ -317,6 +318,8 @@ def library():
         ctypes.POINTER(MatmulDesc), ctypes.c_int32, ctypes.c_int32,
         ctypes.c_int32, i64, i64, i64, u32]
     lib.iree_mi355x_classify_matmul.argtypes = [ctypes.POINTER(MatmulDesc)]
+    lib.iree_mi355x_plan_matmul_within.argtypes = [
+        ctypes.POINTER(MatmulDesc), sz, ctypes.POINTER(MatmulPlan)]
     lib.iree_mi355x_plan_matmul.argtypes = [ctypes.POINTER(MatmulDesc),
                                             ctypes.POINTER(MatmulPlan)]
     lib.iree_mi355x_mfma_config_info.argtypes = [
@@ -405,10 +408,16 @@ def classify(desc: MatmulDesc) -> int:
     return library().iree_mi355x_classify_matmul(ctypes.byref(desc))
 
 
-def plan(desc: MatmulDesc) -> MatmulPlan:
+def plan(desc: MatmulDesc, workspace_bytes: int | None = None) -> MatmulPlan:
+    """The plan of a call with that much workspace (None: all it can use)."""
     out = MatmulPlan()
-    _check(library().iree_mi355x_plan_matmul(ctypes.byref(desc),
-                                             ctypes.byref(out)))
+    lib = library()
+    if workspace_bytes is None:
+        _check(lib.iree_mi355x_plan_matmul(ctypes.byref(desc),
+                                           ctypes.byref(out)))
+    else:
+        _check(lib.iree_mi355x_plan_matmul_within(
+            ctypes.byref(desc), workspace_bytes, ctypes.byref(out)))
     return out
 
 

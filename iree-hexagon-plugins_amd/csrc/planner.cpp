@@ -664,26 +664,28 @@ void iree_mi355x_matmul_desc_init(iree_mi355x_matmul_desc_t *desc,
   desc->batch = 1;
 }
 
-int32_t iree_mi355x_classify_matmul(const iree_mi355x_matmul_desc_t *d) {
-  if (!d || !types_supported(*d) || d->m < 0 || d->n < 0 || d->k < 0)
+}  // extern "C"
+
+namespace {
+
+// The family that the first ranking plans a dispatch in: by what is eligible,
+// before any times are compared.
+int32_t eligible_family(const iree_mi355x_matmul_desc_t &d) {
+  if (!types_supported(d) || d.m < 0 || d.n < 0 || d.k < 0)
     return IREE_MI355X_FAMILY_NONE;
-  if (gemv_eligible(*d))
+  if (gemv_eligible(d))
     return IREE_MI355X_FAMILY_GEMV;
   int count = 0;
   const FastConfig *cfgs = fast_configs(&count);
-  const int64_t cus = d->num_cus > 0 ? d->num_cus : kDefaultCus;
+  const int64_t cus = d.num_cus > 0 ? d.num_cus : kDefaultCus;
   for (int i = 0; i < count; ++i) {
     Candidate c;
-    if (!cfgs[i].table_only && cfgs[i].lds_bytes <= d->lds_budget_bytes &&
-        evaluate(*d, cfgs[i], i, cus, &c))
+    if (!cfgs[i].table_only && cfgs[i].lds_bytes <= d.lds_budget_bytes &&
+        evaluate(d, cfgs[i], i, cus, &c))
       return IREE_MI355X_FAMILY_MFMA;
   }
   return IREE_MI355X_FAMILY_GENERAL;
 }
-
-}  // extern "C"
-
-namespace {
 
 // The plan fields of a general matmul.
 void describe_general(const iree_mi355x_matmul_desc_t &d,
@@ -837,9 +839,10 @@ bool plan_w8t(const iree_mi355x_matmul_desc_t &d, int64_t budget, int64_t cus,
 
 namespace ihp {
 
-int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
-                     size_t workspace_limit, iree_mi355x_matmul_plan_t *plan,
-                     size_t *required);
+static int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
+                            size_t workspace_limit,
+                            iree_mi355x_matmul_plan_t *plan,
+                            size_t *required);
 
 // The plan of a call with `workspace_limit` bytes of workspace, and the
 // workspace below which the call is refused: what the plan of the first
@@ -858,13 +861,14 @@ int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
 }
 
 // plan_matmul with every shape the row-dot takes on the row-dot.
-int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
-                     size_t workspace_limit, iree_mi355x_matmul_plan_t *plan,
-                     size_t *required) {
+static int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
+                            size_t workspace_limit,
+                            iree_mi355x_matmul_plan_t *plan,
+                            size_t *required) {
   *required = 0;
   memset(plan, 0, sizeof(*plan));
   plan->config_index = -1;
-  const int32_t family = iree_mi355x_classify_matmul(d);
+  const int32_t family = eligible_family(*d);
   plan->family = family;
   if (family == IREE_MI355X_FAMILY_NONE)
     return IREE_MI355X_UNSUPPORTED;
@@ -1055,12 +1059,25 @@ int listed_configs() {
 
 extern "C" {
 
-int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
-                            iree_mi355x_matmul_plan_t *plan) {
+int iree_mi355x_plan_matmul_within(const iree_mi355x_matmul_desc_t *d,
+                                   size_t workspace_bytes,
+                                   iree_mi355x_matmul_plan_t *plan) {
   if (!d || !plan)
     return IREE_MI355X_INVALID_ARGUMENT;
   size_t required = 0;
-  return plan_matmul_rows(d, (size_t)-1, plan, &required);
+  return plan_matmul(d, workspace_bytes, plan, &required);
+}
+
+int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
+                            iree_mi355x_matmul_plan_t *plan) {
+  return iree_mi355x_plan_matmul_within(d, (size_t)-1, plan);
+}
+
+int32_t iree_mi355x_classify_matmul(const iree_mi355x_matmul_desc_t *d) {
+  iree_mi355x_matmul_plan_t plan;
+  if (!d || iree_mi355x_plan_matmul(d, &plan) != IREE_MI355X_OK)
+    return IREE_MI355X_FAMILY_NONE;
+  return plan.family;
 }
 
 int iree_mi355x_mfma_config_count(void) {

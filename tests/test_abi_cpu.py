@@ -163,6 +163,9 @@ def test_planner_w8a16_and_unsupported_types(pkg):
     assert p.family == pkg.FAMILY_MFMA and p.config_name.startswith(b"w8a16_nn_")
     d = pkg.make_desc(F16, I8, F16, 512, 11008, 4096, pkg.B_TRANSPOSED,
                       has_scale=True)
+    assert pkg.classify(d) == pkg.FAMILY_MFMA
+    d = pkg.make_desc(F16, I8, F16, 512, 11008, 4100, pkg.B_TRANSPOSED,
+                      has_scale=True)
     assert pkg.classify(d) == pkg.FAMILY_GENERAL
     for bad in ((F32, F32, F32), (I8, F16, F16), (F16, F16, I32), (I8, I8, F16)):
         d = pkg.make_desc(*bad, 64, 64, 64, 0)
@@ -334,15 +337,15 @@ def test_planner_rowdot_gemv(pkg):
             p = pkg.plan(pkg.make_desc(a, b, c, m, n, k, pkg.B_TRANSPOSED,
                                        **kw))
             assert b"rowdot" not in p.config_name, (m, n, k)
-    # W8A16 up to 16 rows: launches of at most 8 rows each, as many as x's
-    # LDS limit allows (7 at K = 4096), dealt evenly
+    # W8A16 up to 16 rows without a workspace: launches of at most 8 rows
+    # each, as many as x's LDS limit allows (7 at K = 4096), dealt evenly
     p = pkg.plan(pkg.make_desc(F16, I8, F16, 3, 4096, 11008,
-                               pkg.B_TRANSPOSED, has_scale=True))
+                               pkg.B_TRANSPOSED, has_scale=True), 0)
     assert p.config_name == b"gemv_rowdot_w8a16_r3"
     assert p.workgroups == 512 * 2 and p.lds_bytes == 2 * 11008 * 2
     for m, rows in ((5, 5), (7, 7), (8, 4), (12, 6), (16, 6)):
         p = pkg.plan(pkg.make_desc(F16, I8, F16, m, 11008, 4096,
-                                   pkg.B_TRANSPOSED, has_scale=True))
+                                   pkg.B_TRANSPOSED, has_scale=True), 0)
         assert p.config_name == b"gemv_rowdot_w8a16_r%d" % m
         assert p.workgroups == 512 * ((m + rows - 1) // rows)
         assert p.lds_bytes == rows * 4096 * 2
@@ -942,3 +945,39 @@ def test_a_plan_asks_for_the_workspace_it_uses(pkg):
     assert workspace_floor(pkg, 300, 11008, 4096, pkg.B_TRANSPOSED) == 0
     # a few rows split K or are refused
     assert workspace_floor(pkg, 16, 4096, 4096) > 0
+
+
+def test_the_plan_tells_what_runs(pkg):
+    """plan() is the plan of a call with all the workspace it can use, and
+    asks for no other than the workspace query's; classify() is its family.
+    W8A16 rows with weights [N,K] give up the row-dot for K splits only where
+    the workspace holds them."""
+    d = pkg.make_desc(F16, I8, F16, 16, 11008, 4096, pkg.B_TRANSPOSED,
+                      has_scale=True)
+    p = pkg.plan(d)
+    assert p.family == pkg.FAMILY_GENERAL and p.splits > 1
+    assert p.workspace_bytes > 0
+    assert pkg._matmul_workspace_need(16, 11008, 4096,
+                                      pkg.B_TRANSPOSED) >= p.workspace_bytes
+    assert pkg.plan(d, p.workspace_bytes).config_name == p.config_name
+    for less in (0, p.workspace_bytes - 1):
+        q = pkg.plan(d, less)
+        assert q.config_name == b"gemv_rowdot_w8a16_r16"
+        assert q.workspace_bytes == 0
+    # one launch of few rows stays
+    d = pkg.make_desc(F16, I8, F16, 4, 11008, 4096, pkg.B_TRANSPOSED,
+                      has_scale=True)
+    assert pkg.plan(d).config_name == b"gemv_rowdot_w8a16_r4"
+    for types, kw in (((F16, F16, F16), {}), ((F16, F16, F32), {}),
+                      ((I8, I8, I32), {}), ((F16, I8, F16),
+                                            {"has_scale": True})):
+        for flags in (0, pkg.B_TRANSPOSED):
+            for m, n, k in ((1, 4096, 4096), (8, 11008, 4096),
+                            (16, 4096, 4096), (300, 11008, 4096),
+                            (512, 11008, 4096), (777, 3001, 4099),
+                            (4096, 4096, 4096), (150, 256, 2048)):
+                d = pkg.make_desc(*types, m, n, k, flags, **kw)
+                assert pkg.classify(d) == pkg.plan(d).family
+                # a refused call's plan names what it cannot run without
+                q = pkg.plan(d, 0)
+                assert q.workspace_bytes <= pkg.plan(d).workspace_bytes

@@ -79,13 +79,20 @@ def run_without_workspace(pkg, x, w, scale, c):
     assert rc == pkg.OK, pkg.last_error()
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (600, 4096, 11008),  # split with a workspace
-    (5, 4096, 4096), (7, 1000, 1008), (16, 4096, 4096),  # row-dot or general
-    (3, 300, 11008), (8, 128, 128),
+@pytest.mark.parametrize("m,n,k,with_ws,without", [
+    (600, 4096, 11008, "w8a16_tn_128x256x64_w2x4_s4_sk",
+     "w8a16_tn_128x128x64_w2x2_s3_sk"),
+    (5, 4096, 4096, "general_w8a16_tn", "gemv_rowdot_w8a16_r5"),
+    (7, 1000, 1008, "general_w8a16_tn", "gemv_rowdot_w8a16_r7"),
+    (16, 4096, 4096, "general_w8a16_tn", "gemv_rowdot_w8a16_r16"),
+    (3, 300, 11008, "general_w8a16_tn", "gemv_rowdot_w8a16_r3"),
+    (8, 128, 128, "general_w8a16_tn", "general_w8a16_tn"),
 ])
-def test_with_and_without_workspace(pkg, dev, m, n, k):
+def test_with_and_without_workspace(pkg, dev, m, n, k, with_ws, without):
     print(m, n, k, flush=True)
+    desc = pkg.make_desc(0, 1, 0, m, n, k, pkg.B_TRANSPOSED, has_scale=True)
+    assert pkg.plan(desc).config_name.decode() == with_ws
+    assert pkg.plan(desc, 0).config_name.decode() == without
     x, w, scale = operands(m, n, k, 16)
     for run in (lambda c: pkg.quantized_matmul(x, w, scale, c,
                                                w_transposed=True),
