@@ -143,7 +143,8 @@ static int launch_mfma(MatmulArgs &args, const iree_mi355x_matmul_plan_t &plan,
 // The plan of a call with this much workspace, and the workspace without
 // which the call is refused (planner.cpp).
 int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
-                iree_mi355x_matmul_plan_t *plan, size_t *required);
+                iree_mi355x_matmul_plan_t *plan, GeneralPlan *general,
+                size_t *required);
 
 // plan_general for a described matmul (planner.cpp).
 bool plan_general_desc(const iree_mi355x_matmul_desc_t &d, bool wide,
@@ -151,7 +152,7 @@ bool plan_general_desc(const iree_mi355x_matmul_desc_t &d, bool wide,
 
 // plan_matmul through a small per-thread table: a plan depends on nothing but
 // the description and the workspace, and ranking the split configurations
-// takes 3-6 us of host time, as long as the kernel of a small call.
+// takes 1-4 us of host time, as long as the kernel of a small call.
 static int cached_plan(const iree_mi355x_matmul_desc_t &d,
                        size_t workspace_limit, iree_mi355x_matmul_plan_t *plan,
                        GeneralPlan *general, size_t *required) {
@@ -179,10 +180,7 @@ static int cached_plan(const iree_mi355x_matmul_desc_t &d,
     *required = e.required;
     return IREE_MI355X_OK;
   }
-  int st = plan_matmul(&d, workspace_limit, plan, required);
-  if (st == IREE_MI355X_OK && plan->family == IREE_MI355X_FAMILY_GENERAL &&
-      !plan_general_desc(d, false, workspace_limit, general))
-    st = IREE_MI355X_UNSUPPORTED;
+  const int st = plan_matmul(&d, workspace_limit, plan, general, required);
   if (st == IREE_MI355X_OK) {
     memcpy(&e.desc, &d, sizeof(d));
     e.limit = workspace_limit;
@@ -314,8 +312,7 @@ size_t iree_mi355x_matmul_workspace_bytes(int64_t m, int64_t n, int64_t k,
       if (f == 1)
         d.flags |= IREE_MI355X_MATMUL_OUT_F32;
       iree_mi355x_matmul_plan_t p;
-      size_t required = 0;
-      if (plan_matmul(&d, (size_t)-1, &p, &required) == IREE_MI355X_OK &&
+      if (iree_mi355x_plan_matmul(&d, &p) == IREE_MI355X_OK &&
           (size_t)p.workspace_bytes > most)
         most = (size_t)p.workspace_bytes;
     }

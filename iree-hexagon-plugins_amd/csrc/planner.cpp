@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstring>
 #include <tuple>
+#include <vector>
 
 #include "../../include/iree_mi355x_kernels.h"
 #include "../../include/iree_mi355x_planner.h"
@@ -442,6 +443,33 @@ bool evaluate(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
   return true;
 }
 
+// general_us's rates of a tile.
+struct GeneralRates {
+  int bm, bn;
+  double alone, shared, round;
+};
+const GeneralRates &general_rates(const GeneralConfig &c) {
+  static const GeneralRates kRates[] = {{64, 64, 0.403, 0.275, 0.574},
+                                        {64, 128, 0.643, 0.398, 1.16},
+                                        {128, 128, 0.971, 0.541, 1.28}};
+  const GeneralRates *r = kRates;
+  while (r->bm != c.bm || r->bn != c.bn)
+    ++r;
+  return *r;
+}
+
+// What splitting K adds, growing with the splits.
+double general_split_us(const GeneralConfig &c, int64_t m, int64_t workgroups,
+                        int64_t splits) {
+  const int64_t at_once = 8 * 64 * 64 / (c.bm * c.bn);
+  const int64_t rows = m < c.bm ? (m + 15) / 16 * 16 : c.bm;
+  return 1.26 + 0.787 * (double)((splits + at_once - 1) / at_once) +
+         0.342e-6 * (double)(workgroups * rows * c.bn * 4);
+}
+
+constexpr double kGeneralBytesPerUs = 5.2e6;
+constexpr double kGeneralLaunchUs = 3.46;
+
 // Modeled time of a general configuration, in us. A CU holds `wgs` workgroups
 // at a time; a K stage takes a lone workgroup `alone` and a CU's share
 // `shared` for each of several; a round of workgroups adds `round`. Splits
@@ -453,16 +481,7 @@ bool evaluate(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
 double general_us(const GeneralConfig &c, int64_t m, int64_t workgroups,
                   int64_t stages, int64_t splits, double operand_bytes,
                   int64_t cus) {
-  struct Rates {
-    int bm, bn;
-    double alone, shared, round;
-  };
-  static const Rates kRates[] = {{64, 64, 0.403, 0.275, 0.574},
-                                 {64, 128, 0.643, 0.398, 1.16},
-                                 {128, 128, 0.971, 0.541, 1.28}};
-  const Rates *r = kRates;
-  while (r->bm != c.bm || r->bn != c.bn)
-    ++r;
+  const GeneralRates *r = &general_rates(c);
   const int64_t per_cu = (workgroups + cus - 1) / cus;
   const int64_t whole = per_cu / c.wgs, rest = per_cu % c.wgs;
   auto stage = [&](int64_t resident) {
@@ -471,15 +490,84 @@ double general_us(const GeneralConfig &c, int64_t m, int64_t workgroups,
   };
   double t = (double)stages * ((double)whole * stage(c.wgs) + stage(rest)) +
              (double)(whole + (rest > 0)) * r->round;
-  if (t < operand_bytes / 5.2e6)  // 5.2 TB/s
-    t = operand_bytes / 5.2e6;
-  if (splits > 1) {
-    const int64_t at_once = 8 * 64 * 64 / (c.bm * c.bn);
-    const int64_t rows = m < c.bm ? (m + 15) / 16 * 16 : c.bm;
-    t += 1.26 + 0.787 * (double)((splits + at_once - 1) / at_once) +
-         0.342e-6 * (double)(workgroups * rows * c.bn * 4);
-  }
-  return t + 3.46;  // the launch
+  if (t < operand_bytes / kGeneralBytesPerUs)
+    t = operand_bytes / kGeneralBytesPerUs;
+  if (splits > 1)
+    t += general_split_us(c, m, workgroups, splits);
+  return t + kGeneralLaunchUs;
+}
+
+// split_us's rates of a configuration: a K stage of a lone workgroup, a CU's
+// share of one of two, a round.
+struct SplitRates {
+  const char *name;
+  double alone, shared, round;
+};
+const SplitRates kSplitRates[] = {
+    {"f16_nn_32x128x64_w1x4_s4_sk", 0.265, 0.240, 0.785},
+    {"f16_nn_64x128x64_w2x2_s4_sk", 0.306, 0.199, 1.88},
+    {"f16_nn_128x128x64_w2x2_s4_sk", 0.452, 0.167, 2.75},
+    {"f16f32_nn_32x128x64_w1x4_s4_sk", 0.251, 0.220, 0.629},
+    {"f16_tn_32x128x64_w1x4_s4_sk", 0.045, 0.240, 0.831},
+    {"f16_tn_128x128x64_w2x2_s4_sk", 0.205, 0.454, 2.72},
+    {"w8a16_nn_32x256x64_w1x4_s4_sk", 0.218, 0.431, 3.44},
+    {"w8a16_nn_128x256x64_w2x4_s4_sk", 0.178, 0.720, 3.29},
+    {"i8_tn_32x128x128_w1x4_s4_sk", 0.246, 0.309, 1.47},
+    {"i8_tn_128x128x128_w2x2_s4_sk", 0.406, 0.242, 3.04},
+    {"i8_nn_32x256x128_w1x4_s4_sk", 0.483, 0.0932, 1.17},
+    {"i8_nn_128x256x128_w2x4_s3_sk", 0.425, 0.638, 2.48},
+    // W8A16 [N,K], fitted to 1060 timings of 84 shapes (m 20..2048, n
+    // 512..11008, k 512..11008): the pick is 1.2 % slower than the best
+    // of these tiles on average.
+    {"w8a16_tn_256x256x64_w2x4_s3", 1.17, 1.17, 3.55},
+    {"w8a16_tn_128x256x64_w2x4_s4", 0.666, 0.657, 1.88},
+    {"w8a16_tn_128x256x64_w2x4_s4_sk", 0.703, 0.685, 3.21},
+    {"w8a16_tn_128x128x64_w2x2_s3_sk", 0.478, 0.507, 3.73},
+    {"w8a16_tn_64x128x64_w2x2_s4_sk", 0.317, 0.370, 2.50}};
+
+// Those of configuration `index`, or null if it was not fitted; the names are
+// looked up once.
+const SplitRates *split_rates(int index) {
+  static const std::vector<const SplitRates *> by_index = [] {
+    int count = 0;
+    const FastConfig *cfgs = fast_configs(&count);
+    std::vector<const SplitRates *> v(count, nullptr);
+    for (int i = 0; i < count; ++i)
+      for (const SplitRates &r : kSplitRates)
+        if (strcmp(r.name, cfgs[i].name) == 0)
+          v[i] = &r;
+    return v;
+  }();
+  return by_index[index];
+}
+
+// What splitting K adds, growing with the splits.
+double split_cost_us(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
+                     int64_t tiles, int64_t splits) {
+  const int64_t batch = d.batch > 0 ? d.batch : 1;
+  const double rows = (double)(d.m < c.bm ? d.m : c.bm);
+  return 3.1 + 0.588 * (double)splits * rows * c.bn / c.threads / 16.0 +
+         0.31e-6 * (double)(tiles * splits * batch) * rows * c.bn * 4.0;
+}
+
+// The least that any split of a configuration takes, without that cost: the
+// stages dealt evenly over the CUs (a little less, for its rounding), or the
+// operands' bytes.
+constexpr double kSplitBytesPerUs = 13.4e6;
+constexpr double kSplitLaunchUs = 2.75;
+double split_bytes(const iree_mi355x_matmul_desc_t &d) {
+  const int64_t batch = d.batch > 0 ? d.batch : 1;
+  return (double)batch * (double)d.k *
+         ((double)d.m * elem_bytes(d.a_elem) +
+          (double)d.n * elem_bytes(d.b_elem));
+}
+double split_least_us(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
+                      const SplitRates &r, int64_t tiles, int64_t cus) {
+  const int64_t batch = d.batch > 0 ? d.batch : 1;
+  const double even = 0.999 * (double)(tiles * batch) *
+                      (double)(d.k / c.bk) * r.shared / (double)cus;
+  const double bytes = split_bytes(d) / kSplitBytesPerUs;
+  return kSplitLaunchUs + (even > bytes ? even : bytes);
 }
 
 // Modeled time of a split-K configuration at `splits` splits, in us, as
@@ -491,36 +579,8 @@ double general_us(const GeneralConfig &c, int64_t m, int64_t workgroups,
 // best split configuration of those on average, 8 % at most, where est_ns
 // was 12 %. 0 for a configuration that was not fitted.
 double split_us(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
-                int64_t tiles, int64_t splits, int64_t k_split, int64_t cus) {
-  struct Rates {
-    const char *name;
-    double alone, shared, round;
-  };
-  static const Rates kRates[] = {
-      {"f16_nn_32x128x64_w1x4_s4_sk", 0.265, 0.240, 0.785},
-      {"f16_nn_64x128x64_w2x2_s4_sk", 0.306, 0.199, 1.88},
-      {"f16_nn_128x128x64_w2x2_s4_sk", 0.452, 0.167, 2.75},
-      {"f16f32_nn_32x128x64_w1x4_s4_sk", 0.251, 0.220, 0.629},
-      {"f16_tn_32x128x64_w1x4_s4_sk", 0.045, 0.240, 0.831},
-      {"f16_tn_128x128x64_w2x2_s4_sk", 0.205, 0.454, 2.72},
-      {"w8a16_nn_32x256x64_w1x4_s4_sk", 0.218, 0.431, 3.44},
-      {"w8a16_nn_128x256x64_w2x4_s4_sk", 0.178, 0.720, 3.29},
-      {"i8_tn_32x128x128_w1x4_s4_sk", 0.246, 0.309, 1.47},
-      {"i8_tn_128x128x128_w2x2_s4_sk", 0.406, 0.242, 3.04},
-      {"i8_nn_32x256x128_w1x4_s4_sk", 0.483, 0.0932, 1.17},
-      {"i8_nn_128x256x128_w2x4_s3_sk", 0.425, 0.638, 2.48},
-      // W8A16 [N,K], fitted to 1060 timings of 84 shapes (m 20..2048, n
-      // 512..11008, k 512..11008): the pick is 1.2 % slower than the best
-      // of these tiles on average.
-      {"w8a16_tn_256x256x64_w2x4_s3", 1.17, 1.17, 3.55},
-      {"w8a16_tn_128x256x64_w2x4_s4", 0.666, 0.657, 1.88},
-      {"w8a16_tn_128x256x64_w2x4_s4_sk", 0.703, 0.685, 3.21},
-      {"w8a16_tn_128x128x64_w2x2_s3_sk", 0.478, 0.507, 3.73},
-      {"w8a16_tn_64x128x64_w2x2_s4_sk", 0.317, 0.370, 2.50}};
-  const Rates *r = nullptr;
-  for (const Rates &x : kRates)
-    if (strcmp(x.name, c.name) == 0)
-      r = &x;
+                const SplitRates *r, int64_t tiles, int64_t splits,
+                int64_t k_split, int64_t cus) {
   if (!r)
     return 0.0;
   const int64_t batch = d.batch > 0 ? d.batch : 1;
@@ -534,17 +594,12 @@ double split_us(const iree_mi355x_matmul_desc_t &d, const FastConfig &c,
   double t = (double)(k_split / c.bk) *
                  ((double)whole * stage(held) + stage(rest)) +
              (double)(whole + (rest > 0)) * r->round;
-  const double bytes = (double)batch * (double)d.k *
-                       ((double)d.m * elem_bytes(d.a_elem) +
-                        (double)d.n * elem_bytes(d.b_elem));
-  if (t < bytes / 13.4e6)
-    t = bytes / 13.4e6;
-  if (splits > 1) {
-    const double rows = (double)(d.m < c.bm ? d.m : c.bm);
-    t += 3.1 + 0.588 * (double)splits * rows * c.bn / c.threads / 16.0 +
-         0.31e-6 * (double)(tiles * splits * batch) * rows * c.bn * 4.0;
-  }
-  return t + 2.75;  // the launch
+  const double bytes = split_bytes(d) / kSplitBytesPerUs;
+  if (t < bytes)
+    t = bytes;
+  if (splits > 1)
+    t += split_cost_us(d, c, tiles, splits);
+  return t + kSplitLaunchUs;
 }
 
 GeneralKind general_kind(const iree_mi355x_matmul_desc_t &d) {
@@ -602,9 +657,19 @@ bool plan_general(GeneralKind kind, int64_t m, int64_t n, int64_t k,
     const int64_t tiles = ((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
     if (tiles >= ((int64_t)1 << 31))
       continue;
+    // The least that any split of this tile takes: the stages dealt evenly
+    // over the CUs (a little less, for its rounding), or the operands' bytes.
+    const double even = 0.999 * (double)(tiles * batch) * (double)stages *
+                        general_rates(c).shared / (double)cus;
+    const double least =
+        kGeneralLaunchUs + (even > bytes / kGeneralBytesPerUs
+                                ? even
+                                : bytes / kGeneralBytesPerUs);
     for (int64_t want = 1; want <= 32; ++want) {
-      if (want > 1 && (tiles * batch > kMaxWorkspaceCounters ||
-                       want * kMinStagesPerSplit > stages))
+      if (want > 1 &&
+          (tiles * batch > kMaxWorkspaceCounters ||
+           want * kMinStagesPerSplit > stages ||
+           least + general_split_us(c, m, tiles * batch * want, want) > best))
         break;
       const int64_t per = stages > 0 ? (stages + want - 1) / want : 1;
       const int64_t splits = stages > 0 ? (stages + per - 1) / per : 1;
@@ -734,6 +799,54 @@ void describe_fast(const iree_mi355x_matmul_desc_t &d, const Candidate &best,
   plan->traffic_bytes = best.traffic;
 }
 
+// The fitted configuration and the split count of `choices` (ascending, from
+// `from` on) modeled faster than *t_best by split_us, within the workspace.
+// False, and nothing changed, if none is.
+template <int N>
+bool fastest_split(const iree_mi355x_matmul_desc_t &d, int64_t budget,
+                   int64_t cus, size_t workspace_limit,
+                   const int (&choices)[N], int from, double *t_best,
+                   Candidate *best) {
+  int count = 0;
+  const FastConfig *cfgs = fast_configs(&count);
+  const int64_t batch = d.batch > 0 ? d.batch : 1;
+  int index = -1, splits = 0;
+  for (int i = 0; i < count; ++i) {
+    const FastConfig &c = cfgs[i];
+    const SplitRates *rates = split_rates(i);
+    if (!rates || (c.table_only && c.b_mode != kBW8T) ||
+        c.lds_bytes > budget || !fast_fits(d, c))
+      continue;
+    const int64_t tiles = (d.m + c.bm - 1) / c.bm * (d.n / c.bn);
+    if (c.split_k && tiles * batch > kMaxWorkspaceCounters)
+      continue;
+    const int64_t stages = d.k / c.bk;
+    const double least = split_least_us(d, c, *rates, tiles, cus);
+    for (int want : choices) {
+      if (want < from)
+        continue;
+      const int64_t per = (stages + want - 1) / want;
+      if (want > 1 && (!c.split_k || per < kMinStagesPerSplit ||
+                       least + split_cost_us(d, c, tiles, want) > *t_best))
+        break;
+      if ((stages + per - 1) / per != want)
+        continue;
+      if (want > 1 &&
+          (uint64_t)(split_counter_bytes(tiles) +
+                     batch * want * d.m * d.n * 4) > (uint64_t)workspace_limit)
+        break;
+      const double t = split_us(d, c, rates, tiles, want, per * c.bk, cus);
+      if (t < *t_best) {
+        *t_best = t;
+        index = i;
+        splits = want;
+      }
+    }
+  }
+  return index >= 0 &&
+         evaluate(d, cfgs[index], index, cus, best, true, splits);
+}
+
 // Ranks the split-K configurations again by split_us where est_ns picked one,
 // and beyond 128 rows the general kernel with them, among the plans whose
 // workspace the caller has. Up to 128 rows a shape that est_ns splits stays
@@ -743,8 +856,8 @@ void refine_split(const iree_mi355x_matmul_desc_t &d, int64_t budget,
                   GeneralPlan *general, bool *use_general) {
   int count = 0;
   const FastConfig *cfgs = fast_configs(&count);
-  double t_best = split_us(d, cfgs[best->index], best->tiles, best->splits,
-                           best->k_split, cus);
+  double t_best = split_us(d, cfgs[best->index], split_rates(best->index),
+                           best->tiles, best->splits, best->k_split, cus);
   if (t_best <= 0.0)
     return;
   const bool keep_split = d.m <= 128 && best->splits > 1;
@@ -754,24 +867,8 @@ void refine_split(const iree_mi355x_matmul_desc_t &d, int64_t budget,
                ? 1e30
                : (d.m <= 128 ? 0.85 : 0.92) * t_best;
   static const int kSplitChoices[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16};
-  for (int i = 0; i < count; ++i) {
-    if (!cfgs[i].split_k || cfgs[i].table_only || cfgs[i].lds_bytes > budget)
-      continue;
-    for (int forced : kSplitChoices) {
-      Candidate c;
-      if (!evaluate(d, cfgs[i], i, cus, &c, true, forced) ||
-          c.splits != forced || (keep_split && c.splits == 1) ||
-          (c.splits > 1 && c.k_split < kMinStagesPerSplit * cfgs[i].bk) ||
-          (size_t)c.workspace > workspace_limit)
-        continue;
-      const double t =
-          split_us(d, cfgs[i], c.tiles, c.splits, c.k_split, cus);
-      if (t > 0.0 && t < t_best) {
-        *best = c;
-        t_best = t;
-      }
-    }
-  }
+  fastest_split(d, budget, cus, workspace_limit, kSplitChoices,
+                keep_split ? 2 : 1, &t_best, best);
   if (d.m <= 128 || !plan_general_desc(d, false, workspace_limit, general))
     return;
   const double t = general_plan_us(d, *general, cus);
@@ -794,10 +891,13 @@ bool rowdot_gives_way(const iree_mi355x_matmul_desc_t &d,
   const bool one_launch = rowdot_w8a16_rows(d.m, d.k) >= d.m;
   if (one_launch && d.m < (d.n * d.k >= (10 << 20) ? 5 : 7))
     return false;
-  GeneralPlan most;
+  if (!plan_general_desc(d, false, (size_t)-1, plan))
+    return false;
+  if ((size_t)plan->workspace <= workspace_limit)
+    return true;
+  const int most = plan->splits;
   return plan_general_desc(d, false, workspace_limit, plan) &&
-         plan_general_desc(d, false, (size_t)-1, &most) &&
-         plan->splits == most.splits;
+         plan->splits == most;
 }
 
 // W8A16 with weights [N,K]: the macro-tile (kBW8T) modeled fastest for the
@@ -808,31 +908,10 @@ bool rowdot_gives_way(const iree_mi355x_matmul_desc_t &d,
 bool plan_w8t(const iree_mi355x_matmul_desc_t &d, int64_t budget, int64_t cus,
               size_t workspace_limit, const GeneralPlan &general,
               Candidate *best) {
-  int count = 0;
-  const FastConfig *cfgs = fast_configs(&count);
   double t_best = 0.95 * general_plan_us(d, general, cus);
-  bool found = false;
   static const int kSplitChoices[] = {1, 2, 3, 4, 6, 8, 12};
-  for (int i = 0; i < count; ++i) {
-    if (cfgs[i].b_mode != kBW8T || cfgs[i].lds_bytes > budget)
-      continue;
-    for (int forced : kSplitChoices) {
-      Candidate c;
-      if ((forced > 1 && !cfgs[i].split_k) ||
-          !evaluate(d, cfgs[i], i, cus, &c, true, forced) ||
-          c.splits != forced ||
-          (c.splits > 1 && c.k_split < kMinStagesPerSplit * cfgs[i].bk) ||
-          (size_t)c.workspace > workspace_limit)
-        continue;
-      const double t = split_us(d, cfgs[i], c.tiles, c.splits, c.k_split, cus);
-      if (t > 0.0 && t < t_best) {
-        *best = c;
-        t_best = t;
-        found = true;
-      }
-    }
-  }
-  return found;
+  return fastest_split(d, budget, cus, workspace_limit, kSplitChoices, 1,
+                       &t_best, best);
 }
 
 }  // namespace
@@ -842,29 +921,29 @@ namespace ihp {
 static int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
                             size_t workspace_limit,
                             iree_mi355x_matmul_plan_t *plan,
-                            size_t *required);
+                            GeneralPlan *general, size_t *required);
 
 // The plan of a call with `workspace_limit` bytes of workspace, and the
 // workspace below which the call is refused: what the plan of the first
 // ranking needs, or less where the refined plan of a call with any workspace
 // uses less. (The workspace_bytes of a refused call's plan are these.)
+// *general is the configuration of a plan of the general family.
 int plan_matmul(const iree_mi355x_matmul_desc_t *d, size_t workspace_limit,
-                iree_mi355x_matmul_plan_t *plan, size_t *required) {
-  GeneralPlan tile;
-  if (rowdot_gives_way(*d, workspace_limit, &tile)) {
+                iree_mi355x_matmul_plan_t *plan, GeneralPlan *general,
+                size_t *required) {
+  if (rowdot_gives_way(*d, workspace_limit, general)) {
     *required = 0;
-    memset(plan, 0, sizeof(*plan));
-    describe_general(*d, tile, plan);
+    describe_general(*d, *general, plan);
     return IREE_MI355X_OK;
   }
-  return plan_matmul_rows(d, workspace_limit, plan, required);
+  return plan_matmul_rows(d, workspace_limit, plan, general, required);
 }
 
 // plan_matmul with every shape the row-dot takes on the row-dot.
 static int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
                             size_t workspace_limit,
                             iree_mi355x_matmul_plan_t *plan,
-                            size_t *required) {
+                            GeneralPlan *general, size_t *required) {
   *required = 0;
   memset(plan, 0, sizeof(*plan));
   plan->config_index = -1;
@@ -955,7 +1034,7 @@ static int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
       for (int i = 0; i < count; ++i) {
         // Column splits are not ranked: they replace their head below.
         if (cfgs[i].lds_bytes > budget || cfgs[i].table_only ||
-            cfgs[i].head)
+            cfgs[i].head || !fast_fits(*d, cfgs[i]))
           continue;
         for (int forced : kSplitChoices) {
           if (forced && !cfgs[i].split_k)
@@ -1002,24 +1081,24 @@ static int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
       return IREE_MI355X_UNSUPPORTED;
     const Candidate first = best;
     bool use_general = false;
-    GeneralPlan g;
     *required = (size_t)first.workspace;
     if (!plan->from_tuned_table && cfgs[first.index].split_k) {
-      refine_split(*d, budget, cus, workspace_limit, &best, &g, &use_general);
+      refine_split(*d, budget, cus, workspace_limit, &best, general,
+                   &use_general);
       if (*required > workspace_limit) {
         // Refused, unless the plan of a call with any workspace is content
         // with this one.
         Candidate c = first;
         GeneralPlan gc;
-        bool general = false;
-        refine_split(*d, budget, cus, (size_t)-1, &c, &gc, &general);
-        const size_t uses = (size_t)(general ? gc.workspace : c.workspace);
+        bool use_gc = false;
+        refine_split(*d, budget, cus, (size_t)-1, &c, &gc, &use_gc);
+        const size_t uses = (size_t)(use_gc ? gc.workspace : c.workspace);
         if (uses < *required)
           *required = uses;
       }
     }
     if (use_general)
-      describe_general(*d, g, plan);
+      describe_general(*d, *general, plan);
     else
       describe_fast(*d, best, plan);
     if (*required > workspace_limit)
@@ -1027,17 +1106,16 @@ static int plan_matmul_rows(const iree_mi355x_matmul_desc_t *d,
     return IREE_MI355X_OK;
   }
 
-  GeneralPlan g;
-  if (!plan_general_desc(*d, false, workspace_limit, &g))
+  if (!plan_general_desc(*d, false, workspace_limit, general))
     return IREE_MI355X_UNSUPPORTED;
   Candidate best;
   if (wanted_b_mode(*d) == kBW8T &&
-      plan_w8t(*d, budget, cus, workspace_limit, g, &best)) {
+      plan_w8t(*d, budget, cus, workspace_limit, *general, &best)) {
     plan->family = IREE_MI355X_FAMILY_MFMA;
     describe_fast(*d, best, plan);
     return IREE_MI355X_OK;
   }
-  describe_general(*d, g, plan);
+  describe_general(*d, *general, plan);
   return IREE_MI355X_OK;
 }
 
@@ -1064,8 +1142,9 @@ int iree_mi355x_plan_matmul_within(const iree_mi355x_matmul_desc_t *d,
                                    iree_mi355x_matmul_plan_t *plan) {
   if (!d || !plan)
     return IREE_MI355X_INVALID_ARGUMENT;
+  GeneralPlan general;
   size_t required = 0;
-  return plan_matmul(d, workspace_bytes, plan, &required);
+  return plan_matmul(d, workspace_bytes, plan, &general, &required);
 }
 
 int iree_mi355x_plan_matmul(const iree_mi355x_matmul_desc_t *d,
