@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 
 BOUND = {"f16": 2e-3, "f32": 1e-5, "w8a16": 2e-3}
 
-# edges of the 64 / 128 tiles, of a 16-byte load and of a K stage (64 f16,
-# 128 int8), and the smallest of everything
+# edges of the 64x64 tile, of a 16-byte load and of a K stage (64 f16, 128
+# int8), and the smallest of everything
 SHAPES = [(1, 1, 1), (2, 3, 5), (7, 17, 9), (16, 8, 15), (63, 65, 64),
           (64, 64, 128), (65, 63, 129), (127, 129, 63), (128, 128, 200),
           (129, 127, 257), (5, 1030, 777), (300, 72, 130)]
@@ -100,6 +100,112 @@ def test_general_edges(pkg, oracle, dev, kind, at, bt):
         buf, c = output(kind, m, n)
         run(pkg, kind, at, bt, da, db, scale.cuda(), m, n, c)
         check(oracle, kind, at, bt, a, b, scale, buf, m, n)
+
+
+# (tile, M, N, K, split): edges of the larger tiles, whose K loop, fragment
+# counts, swizzles and split sums are their own: one row or column past a tile
+# and one short of it, K tails of one and two elements, one stage and many
+WIDE = [("64x128", 641, 4737, 65, False), ("64x128", 1281, 2305, 130, False),
+        ("128x128", 1025, 4735, 65, False), ("128x128", 1153, 3329, 130, False),
+        ("64x128", 129, 4097, 2689, True), ("64x128", 257, 3329, 1700, True),
+        ("64x128", 131, 4405, 4867, True),
+        ("128x128", 385, 4737, 4099, True), ("128x128", 1281, 1601, 4099, True)]
+TYPES = {"f16": (0, 0, 0), "f32": (0, 0, 3), "i8": (1, 1, 2),
+         "w8a16": (0, 1, 0)}
+
+
+def wide_plan(pkg, kind, at, bt, m, n, k, workspace=None):
+    return pkg.plan(pkg.make_desc(
+        *TYPES[kind], m, n, k,
+        (pkg.B_TRANSPOSED if bt else 0) | (pkg.A_TRANSPOSED if at else 0),
+        has_scale=kind == "w8a16", aligned=False), workspace)
+
+
+def in_64_bits(kind, at, bt, da, db, scale):
+    """The product in float64 (exact for int8)."""
+    a = (da.t() if at else da).double().contiguous()
+    b = (db.t() if bt else db).double().contiguous()
+    c = torch.mm(a, b)
+    return c * scale.double() if kind == "w8a16" else c
+
+
+@pytest.mark.parametrize("kind,at,bt", FORMS)
+def test_general_wide_tiles(pkg, dev, kind, at, bt):
+    ran = set()
+    for i, (tile, m, n, k, split) in enumerate(WIDE):
+        p = wide_plan(pkg, kind, at, bt, m, n, k)
+        if (not p.config_name.endswith(b"_" + tile.encode())
+                or (p.splits > 1) != split):
+            continue
+        ran.add((tile, split))
+        pad, lead = ((1, 1), (5, 3), (8, 8))[i % 3]
+        print(f"{kind} at={at} bt={bt} {m}x{n}x{k} "
+              f"{p.config_name.decode()} x{p.splits}", flush=True)
+        _, _, da, db = operands(kind, at, bt, m, n, k, pad, lead)
+        scale = (torch.rand(n) * 0.019 + 0.001).half().cuda()
+        ref = in_64_bits(kind, at, bt, da, db, scale)
+        for _ in range(2 if split else 1):  # the counters are re-armed
+            buf, c = output(kind, m, n)
+            run(pkg, kind, at, bt, da, db, scale, m, n, c)
+            got = c.double()
+            c.fill_(77)
+            assert bool((buf == 77).all()), "write outside the output view"
+            if kind == "i8":
+                assert torch.equal(got, ref)
+            else:
+                # f32 sums of up to 4099 products: 2e-5
+                err = float((got - ref).abs().max() / ref.abs().max())
+                assert err <= (2e-5 if kind == "f32" else BOUND[kind]), err
+    assert ran == {(t, s) for t in ("64x128", "128x128")
+                   for s in (False, True)}
+
+
+@pytest.mark.parametrize("m,n,k,tile", [(641, 4737, 65, "64x128"),
+                                        (1153, 3329, 130, "128x128"),
+                                        (129, 4097, 2689, "64x128"),
+                                        (385, 4737, 4099, "128x128")])
+@pytest.mark.parametrize("bt", [False, True])
+def test_general_wide_tiles_epilogue(pkg, dev, m, n, k, tile, bt):
+    """C += gate * gelu(x W + bias) from the larger tiles, whole and split, at
+    odd pitches."""
+    p = wide_plan(pkg, "f16", False, bt, m, n, k)
+    assert p.config_name.endswith(b"_" + tile.encode())
+    g = torch.Generator(device=dev).manual_seed(m)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g, device=dev).half()
+
+    x, w = rand(m, k), (rand(*((n, k) if bt else (k, n))) / k ** 0.5)
+    bias, mul, init = rand(n), rand(m, n + 3)[:, :n], rand(m + 2, n + 5)
+    buf = init.clone()
+    c = buf[1:m + 1, :n]
+    pkg.batch_matmul(x[None], w[None], c[None], bias=bias,
+                     activation="gelu_tanh", multiplier=mul[None],
+                     accumulate=True, b_transposed=bt)
+    v = torch.mm(x.double(), (w.t() if bt else w).double().contiguous())
+    v = torch.nn.functional.gelu(v + bias.double(), approximate="tanh")
+    ref = init[1:m + 1, :n].double() + mul.double() * v
+    assert float((c.double() - ref).abs().max() / ref.abs().max()) <= 2e-3
+    buf[1:m + 1, :n] = init[1:m + 1, :n]
+    assert torch.equal(buf, init), "write outside the output view"
+
+
+def test_general_without_the_first_pick_s_workspace(pkg, dev):
+    """An aligned shape whose plan does not split runs with no workspace,
+    where the split tiles that are ranked first would need one."""
+    m, n, k = 300, 11008, 4096
+    g = torch.Generator(device=dev).manual_seed(2)
+    a = torch.randn(m, k, generator=g, device=dev).half()
+    b = torch.randn(n, k, generator=g, device=dev).half()
+    c = torch.empty(m, n, dtype=torch.float16, device=dev)
+    p = pkg.plan(pkg.make_desc(0, 0, 0, m, n, k, pkg.B_TRANSPOSED))
+    assert p.family == pkg.FAMILY_GENERAL and p.workspace_bytes == 0
+    assert pkg.library().iree_mi355x_matmul_f16(
+        a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k, k, k, n,
+        pkg.B_TRANSPOSED, None, 0,
+        torch.cuda.current_stream().cuda_stream) == pkg.OK, pkg.last_error()
+    ref = torch.mm(a.double(), b.double().t().contiguous())
+    assert float((c.double() - ref).abs().max() / ref.abs().max()) <= 2e-3
 
 
 @pytest.mark.parametrize("kind,at,bt", FORMS)
