@@ -79,7 +79,10 @@ def test_no_alloc_repeated_and_rejects_oversized_plans(pkg, oracle, dev):
     for y in ys:
         assert oracle.fp16_parity(y.cpu().numpy(), ref) <= FP16_BOUND
     # a plan needing more than the 32 MiB scratch is refused, nothing written
-    m, n, k = 256, 11008, 11008
+    # (256 rows run unsplit and need none: they are not refused)
+    assert pkg.plan(pkg.make_desc(0, 0, 0, 256, 11008,
+                                  11008)).workspace_bytes == 0
+    m, n, k = 500, 11008, 11008
     assert pkg.plan(pkg.make_desc(0, 0, 0, m, n, k, 0)).workspace_bytes > 32 << 20
     x = torch.zeros(m, k, dtype=torch.float16, device=dev)
     w = torch.zeros(k, n, dtype=torch.float16, device=dev)
@@ -88,3 +91,7 @@ def test_no_alloc_repeated_and_rejects_oversized_plans(pkg, oracle, dev):
     assert "workspace" in pkg.last_error()
     torch.cuda.synchronize()
     assert bool((y == 5.0).all())
+    y = torch.full((256, n), 5.0, dtype=torch.float16, device=dev)
+    assert _call(pkg, "no_alloc", x[:256], w, y, s) == pkg.OK
+    torch.cuda.synchronize()
+    assert bool((y == 0).all())
