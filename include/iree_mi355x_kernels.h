@@ -252,6 +252,20 @@ int iree_mi355x_attention_with_workspace(const iree_mi355x_attention_t *args,
                                          size_t workspace_bytes,
                                          void *stream);
 
+// Which kernel a call with that much workspace runs, NONE if it is refused or
+// has nothing to run: the fused kernel (128 query rows of a head a workgroup),
+// the general one (any head dims, alignment and mask strides), or the
+// row-packed one (the rows of a KV head's query heads packed; where it is
+// modeled faster than the other that would take the call).
+typedef enum iree_mi355x_attention_family_e {
+  IREE_MI355X_ATTENTION_FAMILY_NONE = 0,
+  IREE_MI355X_ATTENTION_FAMILY_FUSED = 1,
+  IREE_MI355X_ATTENTION_FAMILY_GENERAL = 2,
+  IREE_MI355X_ATTENTION_FAMILY_ROWS = 3,
+} iree_mi355x_attention_family_t;
+int32_t iree_mi355x_classify_attention(const iree_mi355x_attention_t *args,
+                                       size_t workspace_bytes);
+
 // The workspace a call of these extents and flags can use (0: none); pointers
 // and strides are not looked at.
 size_t iree_mi355x_attention_workspace_bytes(

@@ -48,6 +48,8 @@ ATTENTION_MASK = 0x4
 ELEM_F16, ELEM_I8, ELEM_I32, ELEM_F32 = 0, 1, 2, 3
 FAMILY_NONE, FAMILY_MFMA, FAMILY_GENERAL, FAMILY_GEMV = 0, 1, 2, 3
 B_FORM_TN, B_FORM_NN, B_FORM_W8A16, B_FORM_NN8 = 0, 1, 2, 3
+(ATTENTION_FAMILY_NONE, ATTENTION_FAMILY_FUSED, ATTENTION_FAMILY_GENERAL,
+ ATTENTION_FAMILY_ROWS) = 0, 1, 2, 3
 FAMILY_NAMES = {FAMILY_NONE: "none", FAMILY_MFMA: "mfma",
                 FAMILY_GENERAL: "general", FAMILY_GEMV: "gemv"}
 
@@ -59,7 +61,7 @@ EXPORTED_SYMBOLS = (
     "iree_mi355x_w8a16_matmul", "iree_mi355x_attention_f16",
     "iree_mi355x_attention_f16_strided", "iree_mi355x_attention",
     "iree_mi355x_attention_with_workspace",
-    "iree_mi355x_attention_workspace_bytes",
+    "iree_mi355x_attention_workspace_bytes", "iree_mi355x_classify_attention",
     "iree_mi355x_matmul_workspace_bytes", "iree_mi355x_last_error",
     "iree_mi355x_version", "iree_mi355x_device_count",
     "iree_mi355x_matmul_desc_init", "iree_mi355x_classify_matmul",
@@ -301,6 +303,7 @@ def library():
     lib.iree_mi355x_attention_with_workspace.argtypes = [p, p, sz, p]
     lib.iree_mi355x_attention_workspace_bytes.restype = sz
     lib.iree_mi355x_attention_workspace_bytes.argtypes = [p]
+    lib.iree_mi355x_classify_attention.argtypes = [p, sz]
     lib.iree_mi355x_matmul_workspace_bytes.restype = sz
     lib.iree_mi355x_matmul_workspace_bytes.argtypes = [i64, i64, i64, u32]
     lib.iree_mi355x_batch_matmul_f16.argtypes = [
@@ -1048,6 +1051,18 @@ def _attention_workspace_need(b, h, hkv, sq, skv, d, dv, flags) -> int:
     a = AttentionArgs(batch=b, heads=h, kv_heads=hkv, seq_q=sq, seq_kv=skv,
                       head_dim=d, head_dim_v=dv, flags=flags)
     return library().iree_mi355x_attention_workspace_bytes(ctypes.byref(a))
+
+
+def classify_attention(args: AttentionArgs,
+                       workspace_bytes: int | None = None) -> int:
+    """ATTENTION_FAMILY_*: the kernel that a call with that much workspace
+    (None: all it can use) runs."""
+    lib = library()
+    if workspace_bytes is None:
+        workspace_bytes = lib.iree_mi355x_attention_workspace_bytes(
+            ctypes.byref(args))
+    return lib.iree_mi355x_classify_attention(ctypes.byref(args),
+                                              workspace_bytes)
 
 
 # iree_mi355x_attention_t and iree_mi355x_attention_strides_t as bytes.

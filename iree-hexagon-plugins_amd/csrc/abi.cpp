@@ -52,6 +52,13 @@ static bool dry_run(int64_t workspace_needed) {
   return true;
 }
 
+// The kernel that a validate-only attention call takes.
+static thread_local int32_t g_attention_family = 0;
+static bool dry_run_attention(int64_t workspace_needed, int32_t family) {
+  g_attention_family = family;
+  return dry_run(workspace_needed);
+}
+
 static bool aligned(const void *p, size_t a) {
   return ((uintptr_t)p % a) == 0;
 }
@@ -685,7 +692,7 @@ static int try_rows(const iree_mi355x_attention_t &a, bool fused,
                    &plan);
   if (!*ran)
     return IREE_MI355X_OK;
-  if (dry_run(plan.workspace))
+  if (dry_run_attention(plan.workspace, IREE_MI355X_ATTENTION_FAMILY_ROWS))
     return ok();
   return launch_status(
       launch_attention_rows(a.q, a.k, a.v, a.o, a.mask, general_layout(a),
@@ -787,7 +794,7 @@ int iree_mi355x_attention_f16_strided(
   const int rows_st = try_rows(a, true, nullptr, 0, stream, &ran);
   if (ran)
     return rows_st;
-  if (dry_run(0))
+  if (dry_run_attention(0, IREE_MI355X_ATTENTION_FAMILY_FUSED))
     return ok();
   AttentionLayout layout;
   for (int i = 0; i < 3; ++i) {
@@ -905,7 +912,8 @@ int iree_mi355x_attention_with_workspace(const iree_mi355x_attention_t *a,
         a->q, a->k, a->v, a->o, a->batch, a->heads, a->kv_heads, a->seq_q,
         a->seq_kv, a->head_dim, a->scale, a->flags & IREE_MI355X_ATTENTION_CAUSAL,
         &a->strides, stream);
-  if (dry_run(0))
+  if (dry_run_attention(0, fast ? IREE_MI355X_ATTENTION_FAMILY_FUSED
+                                : IREE_MI355X_ATTENTION_FAMILY_GENERAL))
     return ok();
   if (fast) {
     AttentionLayout layout;
@@ -934,6 +942,18 @@ int iree_mi355x_attention_with_workspace(const iree_mi355x_attention_t *a,
 
 int iree_mi355x_attention(const iree_mi355x_attention_t *a, void *stream) {
   return iree_mi355x_attention_with_workspace(a, nullptr, 0, stream);
+}
+
+int32_t iree_mi355x_classify_attention(const iree_mi355x_attention_t *a,
+                                       size_t workspace_bytes) {
+  size_t need = 0;
+  g_attention_family = IREE_MI355X_ATTENTION_FAMILY_NONE;
+  set_dry_run(&need);
+  const int st = iree_mi355x_attention_with_workspace(a, nullptr,
+                                                      workspace_bytes, nullptr);
+  set_dry_run(nullptr);
+  return st == IREE_MI355X_OK ? g_attention_family
+                              : IREE_MI355X_ATTENTION_FAMILY_NONE;
 }
 
 size_t iree_mi355x_attention_workspace_bytes(

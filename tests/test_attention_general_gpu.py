@@ -29,6 +29,48 @@ def rand(g, *shape):
     return torch.randn(*shape, generator=g).half()
 
 
+def family(pkg, q, k, v, o, causal=False, mask=None):
+    """The kernel that the wrapper's call of these operands runs."""
+    a = pkg.AttentionArgs(
+        q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), o=o.data_ptr(),
+        batch=q.shape[0], heads=q.shape[1], kv_heads=k.shape[1],
+        seq_q=q.shape[2], seq_kv=k.shape[2], head_dim=q.shape[3],
+        head_dim_v=v.shape[3], scale=0.1,
+        flags=((pkg.CAUSAL if causal else 0) |
+               (pkg.ATTENTION_OUT_F32 if o.dtype == torch.float32 else 0) |
+               (pkg.ATTENTION_MASK if mask is not None else 0)))
+    for f, t in (("q", q), ("k", k), ("v", v), ("o", o)):
+        getattr(a.strides, f)[:] = list(t.stride()[:3])
+    if mask is not None:
+        m = mask.expand(q.shape[0], q.shape[1], q.shape[2], k.shape[2])
+        a.mask = m.data_ptr()
+        a.mask_strides[:] = list(m.stride())
+    return pkg.classify_attention(a)
+
+
+def in_64_bits(q, k, v, scale, causal=False, mask=None):
+    """softmax(q k^T scale + mask) v, rows that see no key 0."""
+    b, h, sq, _ = q.shape
+    group = h // k.shape[1]
+    out = torch.empty(b, h, sq, v.shape[3], dtype=torch.float64,
+                      device=q.device)
+    later = torch.ones(sq, k.shape[2], dtype=torch.bool,
+                       device=q.device).triu(1)
+    if mask is not None:
+        mask = mask.expand(b, h, sq, k.shape[2])
+    for z in range(b):
+        for i in range(h):
+            s = torch.mm(q[z, i].double(), k[z, i // group].double().t()
+                         .contiguous()) * scale
+            if mask is not None:
+                s = s + mask[z, i].double()
+            if causal:
+                s = s.masked_fill(later, -float("inf"))
+            p = torch.softmax(s, -1).nan_to_num_(0.0)
+            out[z, i] = torch.mm(p, v[z, i // group].double())
+    return out
+
+
 def random_mask(g, shape, dead=0.2):
     m = 2 * torch.randn(*shape, generator=g)
     m[torch.rand(*shape, generator=g) < dead] = float("-inf")
@@ -55,6 +97,8 @@ CASES = [
         *c[:7], "x".join(map(str, c[7])) if c[7] else "none", int(c[8]), c[9])
     for c in CASES])
 def test_attention_general_vs_oracle(pkg, oracle, dev, case):
+    # sizes at which most of these run on the row-packed kernel; the general
+    # one has its own cases below
     b, hq, hkv, sq, skv, dqk, dv, mshape, causal, out = case
     print(f"attention general {case}", flush=True)
     g = torch.Generator().manual_seed(sq * 31 + skv * 7 + dqk + dv)
@@ -75,6 +119,67 @@ def test_attention_general_vs_oracle(pkg, oracle, dev, case):
     assert np.isfinite(got).all()
     err = oracle.fp16_parity(got, ref)
     assert err <= (F32_BOUND if out == "f32" else F16_BOUND), err
+
+
+# b, hq, hkv, sq, skv, dqk, dv: both ends of each head-dim bucket (32, 64, 128,
+# 256), head dims apart, ragged query blocks and key blocks, grouped heads
+GENERAL_CASES = [(1, 2, 2, 70, 90, 8, 24), (2, 4, 2, 100, 130, 32, 32),
+                 (1, 3, 1, 65, 129, 40, 64), (1, 2, 2, 130, 63, 24, 40),
+                 (2, 4, 2, 100, 130, 96, 96), (1, 2, 1, 200, 65, 128, 72),
+                 (1, 4, 2, 129, 257, 192, 128), (1, 2, 2, 70, 90, 256, 256),
+                 (1, 3, 1, 1, 500, 160, 200), (1, 2, 2, 300, 40, 136, 8),
+                 (1, 2, 1, 90, 100, 100, 100), (1, 2, 2, 70, 64, 250, 130)]
+
+
+@pytest.mark.parametrize("out", ["f16", "f32"])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("case", GENERAL_CASES, ids=[
+    "b{}h{}/{}q{}k{}d{}x{}".format(*c) for c in GENERAL_CASES])
+def test_attention_general_kernel(pkg, oracle, dev, case, causal, out):
+    """The general kernel at every head-dim bucket: a mask whose keys lie two
+    elements apart goes nowhere else."""
+    b, hq, hkv, sq, skv, dqk, dv = case
+    print(f"attention general kernel {case} {causal} {out}", flush=True)
+    g = torch.Generator().manual_seed(sq * 31 + skv * 7 + dqk + dv)
+    q, k = rand(g, b, hq, sq, dqk), rand(g, b, hkv, skv, dqk)
+    v = rand(g, b, hkv, skv, dv)
+    mask = random_mask(g, (sq, skv), 0.1)
+    wide = torch.zeros(sq, 2 * skv, dtype=torch.float16, device=dev)
+    dmask = wide[:, ::2]
+    dmask.copy_(mask)
+    dt = torch.float32 if out == "f32" else torch.float16
+    buf = torch.full((b, hq, sq, dv + 8), 7.0, dtype=dt, device=dev)
+    o, (dq, dk, dvv) = buf[..., :dv], (t.to(dev) for t in (q, k, v))
+    assert family(pkg, dq, dk, dvv, o, causal,
+                  dmask) == pkg.ATTENTION_FAMILY_GENERAL
+    pkg.attention(dq, dk, dvv, o, causal=causal, mask=dmask)
+    ref = oracle.attention(q.numpy(), k.numpy(), v.numpy(), scale=dqk ** -0.5,
+                           causal=causal, out_f32=out == "f32",
+                           mask=mask.numpy())
+    got = o.cpu().numpy()
+    assert np.isfinite(got).all()
+    assert oracle.fp16_parity(got, ref) <= (F32_BOUND if out == "f32"
+                                            else F16_BOUND)
+    assert bool((buf[..., dv:] == 7).all())
+
+
+@pytest.mark.parametrize("case", [(1, 32, 8, 300, 777, 192, 128, False),
+                                  (1, 16, 16, 777, 777, 256, 256, False),
+                                  (2, 16, 8, 519, 777, 192, 128, True),
+                                  (1, 32, 32, 520, 520, 256, 256, True)])
+def test_attention_general_kernel_prompts(pkg, dev, case):
+    """Prompts with the head dims that only the general kernel takes, without
+    a mask: its vector copies, and causal pairs of query blocks."""
+    b, hq, hkv, sq, skv, dqk, dv, causal = case
+    print(f"attention general prompt {case}", flush=True)
+    g = torch.Generator().manual_seed(sq + dqk)
+    q, k = rand(g, b, hq, sq, dqk).to(dev), rand(g, b, hkv, skv, dqk).to(dev)
+    v = rand(g, b, hkv, skv, dv).to(dev)
+    o = torch.empty(b, hq, sq, dv, dtype=torch.float16, device=dev)
+    assert family(pkg, q, k, v, o, causal) == pkg.ATTENTION_FAMILY_GENERAL
+    pkg.attention(q, k, v, o, causal=causal)
+    ref = in_64_bits(q, k, v, dqk ** -0.5, causal)
+    assert float((o - ref).abs().max() / ref.abs().max()) <= F16_BOUND
 
 
 def test_attention_general_fully_masked_rows(pkg, oracle, dev):
@@ -133,9 +238,9 @@ def test_attention_general_strided_views(pkg, oracle, dev):
 
 
 def test_attention_general_routing(pkg, oracle, dev):
-    # equal head dims of 64 / 128, no mask, f16 out: the MFMA kernel, the
-    # same bits through the descriptor as through attention_f16. A zero mask
-    # with contiguous keys takes the MFMA kernel's mask instance; the same
+    # equal head dims of 64 / 128, no mask, f16 out: the same bits through the
+    # descriptor as through attention_f16. A zero mask with contiguous keys
+    # takes the fused or the row-packed kernel's mask instance; the same
     # zeros read with a key stride of 2 take the general kernel: both within
     # the fp16 bound of the unmasked result, and not the same bits (two
     # kernels ran)
@@ -220,10 +325,11 @@ MFMA_MASK_CASES = [
     "b{}h{}/{}q{}k{}d{}_m{}_c{}".format(*c[:6], "x".join(map(str, c[6])),
                                         int(c[7])) for c in MFMA_MASK_CASES])
 def test_attention_mask_mfma_path(pkg, oracle, dev, case):
-    # head dims 64 / 128 with an additive mask whose keys are contiguous run
-    # the MFMA kernel's mask instance: ragged lengths (tails of query rows and
-    # key blocks), grouped heads, masks broadcast over batch, heads or rows,
-    # -inf entries, with and without the causal mask
+    # head dims 64 / 128 with an additive mask whose keys are contiguous, on
+    # the kernel that is the faster one at these sizes (mostly the row-packed
+    # one): ragged lengths (tails of query rows and key blocks), grouped
+    # heads, masks broadcast over batch, heads or rows, -inf entries, with
+    # and without the causal mask
     b, hq, hkv, sq, skv, d, mshape, causal = case
     print(f"attention mask mfma {case}", flush=True)
     g = torch.Generator().manual_seed(sq + skv + d + hq)
@@ -280,10 +386,10 @@ HEAD_DIM_CASES = [
         *c[:6], "x".join(map(str, c[6])) if c[6] else "none", int(c[7]))
     for c in HEAD_DIM_CASES])
 def test_attention_head_dims_mfma_path(pkg, oracle, dev, case):
-    # head dims that are multiples of 16 up to 128 run the MFMA kernel with
-    # the 64- or 128-wide LDS layout, reading only their own chunks: with
-    # and without masks, grouped heads, ragged lengths, causal or not; the
-    # columns past the head dim of the output's buffer stay untouched
+    # head dims that are multiples of 16 up to 128, on the kernel that is the
+    # faster one at these sizes (mostly the row-packed one): with and without
+    # masks, grouped heads, ragged lengths, causal or not; the columns past
+    # the head dim of the output's buffer stay untouched
     b, hq, hkv, sq, skv, d, mshape, causal = case
     print(f"attention head dim {case}", flush=True)
     g = torch.Generator().manual_seed(sq * 3 + skv + d)
@@ -319,10 +425,9 @@ F32_MFMA_CASES = [
         *c[:6], "x".join(map(str, c[6])) if c[6] else "none", int(c[7]))
     for c in F32_MFMA_CASES])
 def test_attention_f32_mfma_path(pkg, oracle, dev, case):
-    # f32 outputs on the MFMA kernel, stored from registers: several query
-    # blocks per workgroup (the second block's rows must not take the
-    # first's values), ragged lengths, masks, grouped heads, and a canary
-    # past the head dim
+    # f32 outputs, on the kernel that is the faster one at these sizes (the
+    # row-packed one): ragged lengths, masks, grouped heads, and a canary past
+    # the head dim
     b, hq, hkv, sq, skv, d, mshape, causal = case
     print(f"attention f32 mfma {case}", flush=True)
     g = torch.Generator().manual_seed(sq + 2 * skv + d)
@@ -340,3 +445,35 @@ def test_attention_f32_mfma_path(pkg, oracle, dev, case):
     assert np.isfinite(got).all()
     assert oracle.fp16_parity(got, ref) <= F32_BOUND
     assert (wide[..., d:].cpu() == 7.0).all()
+
+
+@pytest.mark.parametrize("out", ["f16", "f32"])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("d", [16, 32, 48, 64, 80, 96, 112, 128])
+def test_attention_fused_kernel(pkg, dev, d, masked, out):
+    """The fused kernel's instances of every head dim, with and without a mask,
+    f16 and f32 out, at sizes where it is the faster one: several pairs of
+    query blocks a head (the second block's rows must not take the first's
+    values), ragged last blocks, grouped heads, causal or not, a canary past
+    the head dim."""
+    for causal in (False, True):
+        b, h, hkv, sq = 2, 32, 8, 600
+        skv = 604 if masked else 599 + causal
+        print(f"attention fused d={d} masked={masked} {out} causal={causal}",
+              flush=True)
+        g = torch.Generator().manual_seed(d + causal)
+        q, k = rand(g, b, h, sq, d).to(dev), rand(g, b, hkv, skv, d).to(dev)
+        v = rand(g, b, hkv, skv, d).to(dev)
+        mask = (random_mask(g, (1, 1, sq, skv), 0.1).to(dev) if masked
+                else None)
+        dt = torch.float32 if out == "f32" else torch.float16
+        buf = torch.full((b, h, sq, d + 16), 7.0, dtype=dt, device=dev)
+        o = buf[..., :d]
+        assert family(pkg, q, k, v, o, causal,
+                      mask) == pkg.ATTENTION_FAMILY_FUSED
+        pkg.attention(q, k, v, o, causal=causal, mask=mask)
+        ref = in_64_bits(q, k, v, d ** -0.5, causal, mask)
+        assert bool(torch.isfinite(o).all())
+        err = float((o - ref).abs().max() / ref.abs().max())
+        assert err <= (F32_BOUND if out == "f32" else F16_BOUND), err
+        assert bool((buf[..., d:] == 7).all())

@@ -18,8 +18,28 @@ def rand(g, *shape):
     return torch.randn(*shape, generator=g).half()
 
 
+def family(pkg, q, k, v, o, causal=False, mask=None):
+    """The kernel that the wrapper's call of these operands runs."""
+    a = pkg.AttentionArgs(
+        q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), o=o.data_ptr(),
+        batch=q.shape[0], heads=q.shape[1], kv_heads=k.shape[1],
+        seq_q=q.shape[2], seq_kv=k.shape[2], head_dim=q.shape[3],
+        head_dim_v=v.shape[3], scale=0.1,
+        flags=((pkg.CAUSAL if causal else 0) |
+               (pkg.ATTENTION_OUT_F32 if o.dtype == torch.float32 else 0) |
+               (pkg.ATTENTION_MASK if mask is not None else 0)))
+    for f, t in (("q", q), ("k", k), ("v", v), ("o", o)):
+        getattr(a.strides, f)[:] = list(t.stride()[:3])
+    if mask is not None:
+        m = mask.expand(q.shape[0], q.shape[1], q.shape[2], k.shape[2])
+        a.mask = m.data_ptr()
+        a.mask_strides[:] = list(m.stride())
+    return pkg.classify_attention(a)
+
+
 def run(pkg, oracle, b, h, hk, sq, skv, d, dv, causal=False, mask=None,
-        out_f32=False, seed=0, cache=0, twice=True, bound=None):
+        out_f32=False, seed=0, cache=0, twice=True, bound=None,
+        rows_only=False):
     g = torch.Generator().manual_seed(seed)
     q = rand(g, b, h, sq, d)
     k = rand(g, b, hk, skv + cache, d)
@@ -30,14 +50,17 @@ def run(pkg, oracle, b, h, hk, sq, skv, d, dv, causal=False, mask=None,
     for _ in range(2 if twice else 1):
         buf = torch.full((b, sq, h, dv + 8), 99.0, dtype=dt, device="cuda")
         o = buf[..., :dv].permute(0, 2, 1, 3)
-        pkg.attention(q.cuda(), kd, vd, o, causal=causal,
-                      mask=None if mask is None else mask.cuda())
+        qd, md = q.cuda(), None if mask is None else mask.cuda()
+        if rows_only:
+            assert family(pkg, qd, kd, vd, o, causal,
+                          md) == pkg.ATTENTION_FAMILY_ROWS
+        pkg.attention(qd, kd, vd, o, causal=causal, mask=md)
         got = o.cpu().numpy()
         assert bool((buf[..., dv:] == 99).all()), "write past the head dim"
         ref = oracle.attention(
             q.numpy(), k[:, :, :skv].contiguous().numpy(),
             v[:, :, :skv].contiguous().numpy(), scale=d ** -0.5,
-            causal=causal,
+            causal=causal, out_f32=out_f32,
             mask=None if mask is None else
             mask.expand(b, h, sq, skv).contiguous().numpy())
         ref = ref.astype(np.float32)
@@ -51,7 +74,8 @@ def need(pkg, b, h, hk, sq, skv, d, dv, flags=0):
     return pkg._attention_workspace_need(b, h, hk, sq, skv, d, dv, flags)
 
 
-# edges: one key, blocks of 32 keys and 16 / 32 rows, a key block for some
+# (most of these are the row-packed kernel's, some of the few-key and causal
+# ones another's) edges: one key, blocks of 32 keys and 16 / 32 rows, a key block for some
 # waves only, head dims short of their bucket, split and unsplit
 @pytest.mark.parametrize("b,h,hk,sq,skv,d,dv", [
     (1, 8, 1, 1, 2048, 128, 128), (2, 8, 2, 1, 3001, 64, 64),
@@ -64,6 +88,27 @@ def test_rows_shapes(pkg, oracle, dev, b, h, hk, sq, skv, d, dv, causal):
     print(f"rows {b} {h} {hk} {sq} {skv} {d} {dv} {causal}", flush=True)
     run(pkg, oracle, b, h, hk, sq, skv, d, dv, causal, cache=5,
         out_f32=sq == 5)
+
+
+@pytest.mark.parametrize("out_f32", [False, True])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("sq,d,dv", [
+    (sq, d, dv) for sq in (3, 37)
+    for d, dv in ((64, 56), (40, 64), (128, 120), (104, 72), (256, 200),
+                  (136, 248))])
+def test_rows_instances(pkg, oracle, dev, sq, d, dv, masked, out_f32):
+    """Every instance: 16- and 32-row tiles of each head-dim bucket, head dims
+    short of it and apart, with and without a mask, f16 and f32 out, keys
+    split over workgroups or (777 keys at 37 queries) not."""
+    skv = 777 if sq == 37 else 1500
+    print(f"rows instance {sq} {skv} {d} {dv} {masked} {out_f32}", flush=True)
+    mask = None
+    if masked:
+        g = torch.Generator().manual_seed(d)
+        mask = torch.randn(sq, skv, generator=g).half()
+        mask[torch.rand(sq, skv, generator=g) < 0.2] = -float("inf")
+    run(pkg, oracle, 1, 4, 1, sq, skv, d, dv, mask=mask, out_f32=out_f32,
+        seed=d + dv, rows_only=True)
 
 
 def test_rows_route_and_split(pkg):
@@ -96,8 +141,9 @@ def test_rows_masks(pkg, oracle, dev, skv, kind):
 
 
 def test_rows_infinities(pkg, dev):
-    """An infinite score takes its row's whole weight; a NaN or infinite
-    value reaches the rows that see it and no others."""
+    """A NaN or infinite value reaches the rows that see it and no others; a
+    +inf score makes its row NaN (inf - inf, as in torch's softmax and the
+    other kernels)."""
     g = torch.Generator().manual_seed(3)
     q, k = rand(g, 1, 4, 3, 64).cuda(), rand(g, 1, 1, 1500, 64).cuda()
     v = rand(g, 1, 1, 1500, 64).cuda()
@@ -105,6 +151,13 @@ def test_rows_infinities(pkg, dev):
     o = pkg.attention(q, k, v, causal=False)
     bad = torch.isnan(o).all(-1)[0]
     assert bool(bad[2, 1]) and int(bad.sum()) == 1
+    # +inf scores: q . k overflows to +inf where q has an infinity and k is
+    # positive, to -inf where k is negative
+    q[0, 2, 1, 5] = float("inf")
+    o = pkg.attention(q, k, v, causal=False)
+    bad = torch.isnan(o).all(-1)[0]
+    assert bool(bad[2, 1]) and int(bad.sum()) == 1
+    assert bool(torch.isfinite(o[0][~bad]).all())
     q[0, 2, 1, 5] = 0
     v[0, 0, 7, 11] = float("inf")
     o = pkg.attention(q, k, v, causal=False)
@@ -116,6 +169,41 @@ def test_rows_infinities(pkg, dev):
     v[0, 0, 1400:] = float("nan")
     o = pkg.attention(q, k[:, :, :1400], v[:, :, :1400], causal=False)
     assert bool(torch.isfinite(o).all())
+
+
+@pytest.mark.parametrize("kernel", ["ROWS", "FUSED"])
+def test_hidden_non_finite_values(pkg, dev, kernel):
+    """Under the causal mask a key's NaN or infinity in K stays out of the
+    rows that do not see it. One in V is multiplied by their weight of 0, so
+    it spreads to rows of its own tile (rows of one 32-row tile on the
+    row-packed kernel, of one 128-row block on the fused one), in its own
+    column and to no earlier tile."""
+    b, h, s, d = (1, 4, 192, 64) if kernel == "ROWS" else (2, 32, 600, 64)
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (rand(g, b, h, s, d).cuda() for _ in range(3))
+    assert family(pkg, q, k, v, torch.empty_like(q), True) == getattr(
+        pkg, "ATTENTION_FAMILY_" + kernel)
+    tile = 32 if kernel == "ROWS" else 128
+    key = s // 2 + 3
+    want = pkg.attention(q, k, v).float()
+
+    def same(got, ref):
+        # a row's maximum may have been moved at another block: rounding
+        return bool(((got.float() - ref).abs() <= 2e-3 * ref.abs().max()).all())
+
+    for bad in (float("nan"), float("inf")):
+        k2, v2 = k.clone(), v.clone()
+        k2[0, 1, key, 7] = bad
+        o = pkg.attention(q, k2, v)
+        assert same(o[0, 1, :key], want[0, 1, :key])
+        assert bool(torch.isnan(o[0, 1, key:]).any())
+        v2[0, 1, key, 11] = bad
+        o = pkg.attention(q, k, v2)
+        first = key // tile * tile
+        assert same(o[0, 1, :first], want[0, 1, :first])
+        assert bool((~torch.isfinite(o[0, 1, key:, 11])).all())
+        o[0, 1, :, 11] = want[0, 1, :, 11].half()
+        assert same(o, want)
 
 
 def test_rows_with_less_workspace(pkg, oracle, dev):

@@ -211,9 +211,9 @@ def test_direct_references_and_attention(pkg, oracle, dev):
 
 def test_general_attention_in_a_command_buffer(pkg, oracle, dev):
     """The 41-word attention_f16 form through a command buffer: a mask in
-    binding 4 taken from the binding table, head dims 96 / 96 with an f32
-    result (the MFMA kernel's f32 mask instance) and 24 / 40 (the general
-    kernel), in one segment on two lanes."""
+    binding 4 taken from the binding table, equal head dims (96 / 96) and
+    head dims apart (24 / 40) with f32 results, in one segment on two
+    lanes."""
     g = torch.Generator().manual_seed(9)
     b, h, s = 1, 2, 192
     cases = []
@@ -244,7 +244,7 @@ def test_general_attention_in_a_command_buffer(pkg, oracle, dev):
     for d, dv, q, k_, v, o in cases:
         ref = oracle.attention(q.numpy(), k_.numpy(), v.numpy(), scale=0.25,
                                causal=True, mask=mask.numpy(), out_f32=True)
-        # both attention kernels round the probabilities to f16: 4e-4
+        # every attention kernel rounds the probabilities to f16: 4e-4
         bound = 4e-4
         assert oracle.fp16_parity(o.cpu().numpy(), ref) <= bound, (d, dv)
 
