@@ -65,6 +65,14 @@ typedef struct iree_mi355x_command_buffer_t iree_mi355x_command_buffer_t;
 #define IREE_MI355X_DEFAULT_CONCURRENCY 1u
 #define IREE_MI355X_MAX_CONCURRENCY 8u
 
+// As max_concurrent, of a query and its submission: in order on the caller's
+// stream, each dispatch with all of a workspace that serves flat calls and
+// in-order submissions only, never lanes. General matmuls and attention that
+// need no workspace then split K or their keys over it, as flat calls do. The
+// query is what the dispatches can use; a submission runs with any workspace
+// down to the query at concurrency 1.
+#define IREE_MI355X_IN_ORDER_WHOLE_WORKSPACE 0x40000000u
+
 // New, empty command buffer recording against `library` (NULL: this
 // library's own table, iree_mi355x_executable_library_query).
 int iree_mi355x_command_buffer_create(
@@ -106,7 +114,8 @@ int iree_mi355x_command_buffer_end(
     iree_mi355x_command_buffer_t *command_buffer);
 
 // Bytes of workspace a submission with this binding table and concurrency
-// needs (one slice per lane, each the largest any dispatch asks for), after
+// needs (one slice per lane, each the largest that any dispatch cannot run
+// without), or with IREE_MI355X_IN_ORDER_WHOLE_WORKSPACE can use, after
 // validating every command; 0 on error (see iree_mi355x_last_error).
 size_t iree_mi355x_command_buffer_workspace_bytes(
     const iree_mi355x_command_buffer_t *command_buffer,
@@ -116,7 +125,8 @@ size_t iree_mi355x_command_buffer_workspace_bytes(
 // Submit on `stream` (hipStream_t; NULL = the null stream): resolves the
 // binding table, validates every command (a failing one enqueues nothing),
 // then enqueues. max_concurrent: 0 = IREE_MI355X_DEFAULT_CONCURRENCY, 1 = in
-// order on `stream` alone, at most IREE_MI355X_MAX_CONCURRENCY. `workspace`
+// order on `stream` alone, at most IREE_MI355X_MAX_CONCURRENCY, or
+// IREE_MI355X_IN_ORDER_WHOLE_WORKSPACE. `workspace`
 // holds the lane slices, sized by iree_mi355x_command_buffer_workspace_bytes
 // (one slice is that query at concurrency 1); a submission that needs one
 // and has none, or a short one, returns IREE_MI355X_WORKSPACE_TOO_SMALL

@@ -749,7 +749,7 @@ def _call_workspace(need, index, stream):
     (None, 0) under capture: graphs captured on one stream may replay on
     several at a time, so what runs without a workspace keeps nothing in the
     stream's. (The null stream cannot be captured.)"""
-    if need <= 0 or (stream and _capturing(stream)):
+    if stream and _capturing(stream):
         return None, 0
     have = _FLAT_WORKSPACES.get((index, stream))
     if have is not None and have[1] >= need:
@@ -761,7 +761,8 @@ def _call_workspace(need, index, stream):
 def _call(fn, args, need, index, stream):
     """One flat call of the library with what it can use of the stream's
     workspace; a captured one that cannot run without gets what there is."""
-    st = fn(*args, *_call_workspace(need, index, stream), stream)
+    ws, wsb = _call_workspace(need, index, stream) if need > 0 else (None, 0)
+    st = fn(*args, ws, wsb, stream)
     if st == WORKSPACE_TOO_SMALL and need > 0:
         import torch
         st = fn(*args, *stream_workspace(
@@ -1230,6 +1231,11 @@ def direct(t, offset: int = 0, length: int | None = None) -> BufferRef:
                      nbytes - offset if length is None else length)
 
 
+# iree_mi355x_command_buffer_submit's max_concurrent
+# (IREE_MI355X_IN_ORDER_WHOLE_WORKSPACE)
+IN_ORDER_WHOLE_WORKSPACE = 0x40000000
+
+
 def _ptr_len(t):
     if isinstance(t, tuple):
         return t
@@ -1317,24 +1323,43 @@ class CommandBuffer:
 
     def submit(self, table=(), max_concurrent=0, workspace=None, stream=None):
         """Submit on `stream`; without a `workspace`, in order on the
-        wrapper's flat workspace of that stream, and with lanes on its
-        workspace for this slice size (lane l's counters sit at l slices: a
-        buffer serves one slice size)."""
+        wrapper's flat workspace of that stream (as much of it as the
+        dispatches can use; under capture what they need), and with lanes on
+        its workspace for this slice size (lane l's counters sit at l slices:
+        a buffer serves one slice size)."""
         arr, n = binding_table(list(table))
         s = _stream_ptr(stream)
-        if workspace is None:
-            need = self._lib.iree_mi355x_command_buffer_workspace_bytes(
-                self._h, arr, n, max_concurrent)
-            slice_ = need
-            if need and max_concurrent > 1:
-                slice_ = self._lib.iree_mi355x_command_buffer_workspace_bytes(
-                    self._h, arr, n, 1)
-            ws, wsb = stream_workspace(
-                need, None, s, None if need == slice_ else ("lanes", slice_))
-        else:
-            ws, wsb = _ptr_len(workspace)
-        _check(self._lib.iree_mi355x_command_buffer_submit(
-            self._h, arr, n, max_concurrent, ws, wsb, s))
+        lib = self._lib
+        args = (self._h, arr, n)
+        if workspace is not None:
+            _check(lib.iree_mi355x_command_buffer_submit(
+                *args, max_concurrent, *_ptr_len(workspace), s))
+            return
+        query = lib.iree_mi355x_command_buffer_workspace_bytes
+        if self._lanes(max_concurrent) == 1:
+            need = query(*args, IN_ORDER_WHOLE_WORKSPACE)
+            ws = (None, 0)
+            if need:
+                import torch
+                ws = _call_workspace(need, torch.cuda.current_device(), s)
+            st = lib.iree_mi355x_command_buffer_submit(
+                *args, IN_ORDER_WHOLE_WORKSPACE, *ws, s)
+            if st != WORKSPACE_TOO_SMALL:
+                _check(st)
+                return
+            max_concurrent = 1  # captured
+        need, slice_ = query(*args, max_concurrent), query(*args, 1)
+        ws = stream_workspace(need, None, s,
+                              ("lanes", slice_) if need > slice_ else None)
+        _check(lib.iree_mi355x_command_buffer_submit(
+            *args, max_concurrent, *ws, s))
+
+    def _lanes(self, max_concurrent) -> int:
+        """Lanes of a submission at this concurrency (0: it is refused)."""
+        if max_concurrent in (0, 1):
+            return 1
+        return 1 + max((op[1] for op in self.lane_schedule(max_concurrent)),
+                       default=-1)
 
 
 def kernel_resources(device: bool = True) -> list[dict]:

@@ -179,14 +179,16 @@ struct Ready {
   uint64_t target_length = 0;
 };
 
-// Resolve and validate every command; the largest workspace any dispatch
-// cannot run without goes to *max_workspace. That alone sizes a slice, at
-// every concurrency: a slice that grew with what a submission has would put
-// one lane's partial tiles over another's counters on a workspace that
-// serves both. Enqueues nothing.
+// Resolve and validate every command; the largest workspace that any dispatch
+// asks for, given `workspace_limit` bytes, goes to *max_workspace (more than
+// the limit: it cannot run with it). Slices are sized at a limit of 0, by what
+// the dispatches cannot run without, at every concurrency: a slice that grew
+// with what a submission has would put one lane's partial tiles over another's
+// counters on a workspace that serves both. Enqueues nothing.
 int prepare(const iree_mi355x_command_buffer_t *cb,
             const iree_mi355x_binding_t *table, uint32_t count,
-            std::vector<Ready> *out, size_t *max_workspace) {
+            size_t workspace_limit, std::vector<Ready> *out,
+            size_t *max_workspace) {
   *max_workspace = 0;
   out->assign(cb->commands.size(), Ready());
   const iree_mi355x_executable_export_table_t &ex = cb->library->exports;
@@ -214,6 +216,7 @@ int prepare(const iree_mi355x_command_buffer_t *cb,
         s.binding_count = (uint32_t)r.ptrs.size();
         s.binding_ptrs = r.ptrs.data();
         s.binding_lengths = r.lengths.data();
+        s.workspace_bytes = workspace_limit;
         s.workspace_query = &need;
         if ((st = ex.ptrs[c.ordinal](nullptr, &s))) {
           const std::string why = iree_mi355x_last_error();
@@ -271,6 +274,20 @@ uint32_t lanes_for(const iree_mi355x_command_buffer_t *cb, uint32_t requested) {
     }
   }
   return std::max(1u, std::min(requested, widest));
+}
+
+// Lanes of a submission's max_concurrent argument.
+uint32_t lanes_of(const iree_mi355x_command_buffer_t *cb,
+                  uint32_t max_concurrent) {
+  if (max_concurrent == IREE_MI355X_IN_ORDER_WHOLE_WORKSPACE)
+    return 1;
+  return lanes_for(
+      cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
+}
+
+bool concurrency_valid(uint32_t max_concurrent) {
+  return max_concurrent <= IREE_MI355X_MAX_CONCURRENCY ||
+         max_concurrent == IREE_MI355X_IN_ORDER_WHOLE_WORKSPACE;
 }
 
 size_t slice_bytes(size_t need) { return (need + 255) & ~(size_t)255; }
@@ -560,10 +577,9 @@ uint32_t iree_mi355x_command_buffer_count(
 uint32_t iree_mi355x_command_buffer_lane_schedule(
     const iree_mi355x_command_buffer_t *cb, uint32_t max_concurrent,
     iree_mi355x_lane_op_t *ops, uint32_t capacity) {
-  if (!cb || max_concurrent > IREE_MI355X_MAX_CONCURRENCY)
+  if (!cb || !concurrency_valid(max_concurrent))
     return 0;
-  const uint32_t lanes = lanes_for(
-      cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
+  const uint32_t lanes = lanes_of(cb, max_concurrent);
   const std::vector<iree_mi355x_lane_op_t> s = lane_schedule(cb, lanes);
   for (uint32_t i = 0; i < capacity && i < s.size(); ++i)
     ops[i] = s[i];
@@ -574,14 +590,14 @@ size_t iree_mi355x_command_buffer_workspace_bytes(
     const iree_mi355x_command_buffer_t *cb,
     const iree_mi355x_binding_t *binding_table, uint32_t binding_count,
     uint32_t max_concurrent) {
-  if (!cb || max_concurrent > IREE_MI355X_MAX_CONCURRENCY)
+  if (!cb || !concurrency_valid(max_concurrent))
     return 0;
-  const uint32_t lanes = lanes_for(
-      cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
+  const bool whole = max_concurrent == IREE_MI355X_IN_ORDER_WHOLE_WORKSPACE;
+  const uint32_t lanes = lanes_of(cb, max_concurrent);
   std::vector<Ready> ready;
   size_t need = 0;
-  if (prepare(cb, binding_table, binding_count, &ready, &need) !=
-      IREE_MI355X_OK)
+  if (prepare(cb, binding_table, binding_count, whole ? SIZE_MAX : 0, &ready,
+              &need) != IREE_MI355X_OK)
     return 0;
   return need ? slice_bytes(need) * lanes : 0;
 }
@@ -596,28 +612,32 @@ int iree_mi355x_command_buffer_submit(
   if (!cb->ended)
     return fail(IREE_MI355X_INVALID_ARGUMENT,
                 "submit: command buffer not ended");
-  if (max_concurrent > IREE_MI355X_MAX_CONCURRENCY)
+  if (!concurrency_valid(max_concurrent))
     return fail(IREE_MI355X_INVALID_ARGUMENT,
                 "submit: concurrency %u > %u", max_concurrent,
                 IREE_MI355X_MAX_CONCURRENCY);
-  const uint32_t lanes = lanes_for(
-      cb, max_concurrent ? max_concurrent : IREE_MI355X_DEFAULT_CONCURRENCY);
+  const bool whole = max_concurrent == IREE_MI355X_IN_ORDER_WHOLE_WORKSPACE;
+  const size_t have = workspace ? workspace_bytes : 0;
+  const uint32_t lanes = lanes_of(cb, max_concurrent);
   std::vector<Ready> ready;
   size_t need = 0;
-  int st = prepare(cb, binding_table, binding_count, &ready, &need);
+  int st = prepare(cb, binding_table, binding_count, whole ? have : 0, &ready,
+                   &need);
   if (st)
     return st;
   if (cb->commands.empty())
     return IREE_MI355X_OK;
-  const size_t slice = need ? slice_bytes(need) : 0;
+  if (whole && need > have)
+    return fail(IREE_MI355X_WORKSPACE_TOO_SMALL,
+                "submit: workspace %zu < %zu", have, need);
+  const size_t slice = whole ? have : need ? slice_bytes(need) : 0;
   // The caller provides the lane slices: the runtime allocates no device
   // memory.
-  if (slice && (!workspace || workspace_bytes < slice * lanes))
+  if (slice && have < slice * lanes)
     return fail(IREE_MI355X_WORKSPACE_TOO_SMALL,
                 "submit: workspace %zu < %zu (%u lanes x %zu; size it with "
                 "iree_mi355x_command_buffer_workspace_bytes)",
-                workspace ? workspace_bytes : (size_t)0, slice * lanes, lanes,
-                slice);
+                have, slice * lanes, lanes, slice);
 
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess)
@@ -631,7 +651,8 @@ int iree_mi355x_command_buffer_submit(
 
   if (lanes == 1) {
     // In order on the caller's stream: barriers hold by stream order. One
-    // slice, as lane 0 has it: what follows holds other lanes' counters.
+    // slice, as lane 0 has it (what follows holds other lanes' counters), or
+    // all of a workspace that no lanes use.
     for (uint32_t i = 0; i < n && !st; ++i)
       st = enqueue(cb, i, ready[i], caller, slice ? ws : nullptr, slice);
     roctxRangePop();

@@ -166,8 +166,10 @@ def test_one_slice_size_at_every_concurrency(pkg, calls):
 
 def test_in_order_submissions_take_the_flat_workspace(pkg, monkeypatch):
     """In order the counters open the workspace, as a flat call's do: every
-    such submission of a stream takes the stream's one flat buffer. Lanes
-    have one per slice size."""
+    such submission of a stream takes the stream's one flat buffer, for all
+    that its dispatches can use. Lanes have one per slice size."""
+    import torch
+
     class Asked(Exception):
         pass
 
@@ -175,16 +177,49 @@ def test_in_order_submissions_take_the_flat_workspace(pkg, monkeypatch):
         raise Asked(need, layout, partial)
 
     monkeypatch.setattr(pkg, "stream_workspace", ask)
-    sizes = [(16, 4096, 4096), (16, 4096, 2048), (1, 4096, 4096)]
-    for shape in sizes:
+    monkeypatch.setattr(pkg, "_FLAT_WORKSPACES", {})
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    for shape in ((16, 4096, 4096), (16, 4096, 2048), (1, 4096, 4096)):
         cb, table = dispatches(pkg, shape, shape)
         one = cb.workspace_bytes(table, 1)
-        assert one > 0
+        all_ = cb.workspace_bytes(table, pkg.IN_ORDER_WHOLE_WORKSPACE)
+        assert 0 < all_ <= one < all_ + 256
         for lanes in (0, 1, 2):
             with pytest.raises(Asked) as e:
                 cb.submit(table, max_concurrent=lanes, stream=0)
             assert e.value.args == ((2 * one, ("lanes", one), False)
-                                    if lanes == 2 else (one, None, False))
+                                    if lanes == 2 else (all_, None, False))
+        # barriers between all commands leave one lane
+        cb = pkg.CommandBuffer()
+        cb.dispatch("matmul_f16", matmul_consts(pkg, *shape),
+                    [pkg.slot(j) for j in range(3)])
+        with pytest.raises(Asked) as e:
+            cb.end().submit(table, max_concurrent=4, stream=0)
+        assert e.value.args == (all_, None, False)
+    # a general matmul and attention need none and can use some
+    cb, table = dispatches(pkg, (777, 3001, 4099))
+    assert cb.workspace_bytes(table, 1) == 0
+    assert cb.workspace_bytes(
+        table, pkg.IN_ORDER_WHOLE_WORKSPACE) == pkg._matmul_workspace_need(
+            777, 3001, 4099, 0)
+
+
+def test_whole_workspace_submissions_are_checked(pkg):
+    """Less than the dispatches cannot run without is refused; other values
+    past the greatest concurrency stay refused."""
+    cb, table = dispatches(pkg, (16, 4096, 4096), (777, 3001, 4099))
+    arr, n = pkg.binding_table(table)
+    one = cb.workspace_bytes(table, 1)
+    lib = pkg.library()
+    for have in (0, one // 2):
+        assert lib.iree_mi355x_command_buffer_submit(
+            cb._h, arr, n, pkg.IN_ORDER_WHOLE_WORKSPACE,
+            FAKE if have else None, have, None) == pkg.WORKSPACE_TOO_SMALL
+    assert cb.lane_schedule(pkg.IN_ORDER_WHOLE_WORKSPACE) == cb.lane_schedule(1)
+    for bad in (9, 0xFFFFFFFF, pkg.IN_ORDER_WHOLE_WORKSPACE + 1):
+        assert cb.workspace_bytes(table, bad) == 0
+        assert lib.iree_mi355x_command_buffer_submit(
+            cb._h, arr, n, bad, FAKE, 1 << 40, None) == pkg.INVALID_ARGUMENT
 
 
 def test_workspace_query_through_export(pkg):

@@ -164,6 +164,62 @@ def test_lanes_and_in_order_on_one_workspace(pkg, oracle, dev, calls):
             assert torch.equal(ws[slice_:], before)
 
 
+def test_in_order_submissions_with_all_of_a_workspace(pkg, oracle, dev):
+    """A general matmul, one query against 4000 keys and a split-K matmul
+    with every amount of workspace from what the last cannot run without to
+    more than all can use, and through the wrapper between flat calls and
+    lanes on one stream."""
+    import struct
+    g = torch.Generator().manual_seed(35)
+    h, skv, d = 8, 4000, 128
+    scale = d ** -0.5
+    shapes = [(33, 130, 2050), (16, 4096, 2048)]
+    cb, table, outs, refs = pkg.CommandBuffer(), [], [], []
+    for i, (m, n, k) in enumerate(shapes):
+        a = (torch.randn(m, k, generator=g) * 0.5).half()
+        b = (torch.randn(k, n, generator=g) * 0.05).half()
+        outs.append(torch.empty(m, n, dtype=torch.float16, device=dev))
+        refs.append(oracle.matmul_f16(a.numpy(), b.numpy()))
+        table += [a.to(dev), b.to(dev), outs[-1]]
+        cb.dispatch("matmul_f16", consts(pkg, m, n, k),
+                    [pkg.slot(3 * i + j) for j in range(3)])
+    q = torch.randn(1, h, 1, d, generator=g).half()
+    kk, v = (torch.randn(1, h, skv, d, generator=g).half() for _ in range(2))
+    outs.append(torch.empty(1, h, 1, d, dtype=torch.float16, device=dev))
+    refs.append(oracle.attention_f16(q.numpy(), kk.numpy(), v.numpy(),
+                                     scale=scale, causal=False))
+    table += [t.to(dev) for t in (q, kk, v)] + [outs[-1]]
+    cb.dispatch("attention_f16",
+                [1, h, 1, skv, d,
+                 struct.unpack("<I", struct.pack("<f", scale))[0], 0],
+                [pkg.slot(6 + j) for j in range(4)])
+    cb.end()
+
+    def check(submit):
+        for o in outs:
+            o.fill_(9.0)
+        submit()
+        torch.cuda.synchronize()
+        for o, ref in zip(outs, refs):
+            assert oracle.fp16_parity(o.cpu().numpy(), ref) <= FP16_BOUND
+
+    whole = pkg.IN_ORDER_WHOLE_WORKSPACE
+    least, most = cb.workspace_bytes(table, 1), cb.workspace_bytes(table, whole)
+    ws = torch.zeros(most + (1 << 20), dtype=torch.uint8, device=dev)
+    for size in (least, (least + most) // 2, most, most + (1 << 20), least):
+        print(f"whole workspace {size}", flush=True)
+        for _ in range(2):
+            check(lambda: cb.submit(table, max_concurrent=whole,
+                                    workspace=(ws.data_ptr(), size)))
+    assert int(ws[:256 << 10].count_nonzero()) == 0
+    for lanes in (1, 3, 0, 2, 1):
+        print(f"wrapper lanes {lanes}", flush=True)
+        check(lambda: cb.submit(table, max_concurrent=lanes))
+        y = pkg.matmul(table[3], table[4])  # flat split-K in between
+        torch.cuda.synchronize()
+        assert oracle.fp16_parity(y.cpu().numpy(), refs[1]) <= FP16_BOUND
+
+
 def test_failed_validation_enqueues_nothing(pkg, dev):
     m, n, k = 128, 512, 256
     a = torch.randn(m, k, device=dev).half()
