@@ -221,13 +221,14 @@ int iree_mi355x_attention_f16_strided(
 // keys are all masked (-inf) writes 0, as the all-masked guard of the
 // decomposed softmax does (examples/attention_layer/attention_layer.mlir:
 // 80-102). head_dim and head_dim_v are 1..256, heads a multiple of
-// kv_heads, heads and batch at most 65535. Shapes the MFMA kernel takes
-// (equal head dims that are multiples of 16 up to 128, f16 or f32 output,
-// the alignment of iree_mi355x_attention_f16_strided, and a mask if any with
-// contiguous keys, its other strides and base 8-byte aligned and seq_kv a
-// multiple of 4) run there; the rest run a general kernel (32-key blocks in
-// LDS, f32 online softmax). _f16 and _f16_strided take head dims 64 and
-// 128 only, on the MFMA kernel.
+// kv_heads, heads and batch at most 65535. The fused kernel takes equal head
+// dims that are multiples of 16 up to 128, f16 or f32 output, the alignment
+// of iree_mi355x_attention_f16_strided, and a mask if any with contiguous
+// keys, its other strides and base 8-byte aligned and seq_kv a multiple of 4;
+// a general kernel takes the rest. A row-packed kernel replaces either where
+// it is modeled faster (few query rows per KV head; see
+// iree_mi355x_classify_attention). _f16 and _f16_strided take head dims 64
+// and 128 only.
 typedef struct iree_mi355x_attention_t {
   const void *q, *k, *v;
   void *o;
@@ -276,9 +277,10 @@ size_t iree_mi355x_attention_workspace_bytes(
 // partials and arrival counters), 0 if none. Mirrors the scratch query of the
 // reference's caller-scratch matmul, hexkl_matmul_f16f16_f32_scratch_bytes
 // (CG/Conversion/HexagonRuntimeLinking.h:35-38). The library allocates no
-// device memory: a call whose plan needs a workspace and gets none, or a
-// smaller one, returns IREE_MI355X_WORKSPACE_TOO_SMALL before anything is
-// launched. A workspace must be zero-filled before its first use and is left
+// device memory: a call that cannot run without a workspace and gets none, or
+// a smaller one, returns IREE_MI355X_WORKSPACE_TOO_SMALL before anything is
+// launched (iree_mi355x_plan_matmul_within tells; a general matmul, or W8A16
+// rows with weights [N,K], runs with any). A workspace must be zero-filled before its first use and is left
 // zero-filled in its counter region (its first 256 KiB) after every call, so
 // one workspace serves any sequence of calls of any shapes; calls that
 // overlap must not share one. The value covers every layout the call may run

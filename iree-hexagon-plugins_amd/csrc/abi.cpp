@@ -124,8 +124,7 @@ static int launch_status(hipError_t e, const char *what) {
   return ok();
 }
 
-// Launch the planned MFMA configuration, with its split-K workspace (the
-// caller's if given and large enough, else the library's).
+// Launch the planned MFMA configuration, with its split-K workspace.
 static int launch_mfma(MatmulArgs &args, const iree_mi355x_matmul_plan_t &plan,
                        void *workspace, size_t workspace_bytes,
                        const char *who) {
